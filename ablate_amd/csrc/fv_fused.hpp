@@ -136,7 +136,7 @@ __device__ __forceinline__ void fused_cell(const MeshView<double>& m, const Phys
         const int s = e & 1;
         const int64_t n = valid[k] ? (int64_t)nb : c;
         double x[2][DIM];
-        load_face_pair<DIM>(m.fdx, f, x);
+        load_face_pair<DIM>(m.fdx, geometry_row(m, f), x);
         double dxn[DIM];
 #pragma unroll
         for (int d = 0; d < DIM; d++) {
@@ -353,8 +353,8 @@ __global__ __launch_bounds__(256) void k_fused(MeshView<double> m, Phys ph, cons
         const int32_t code = fv.fcode[f0 + j];
         const int lc = code & 0xFFFF, rc = (int)((uint32_t)code >> 16);
         double nh[3], area, x[2][DIM];
-        load_face_na(m.fna, f, nh, area);
-        load_face_pair<DIM>(m.fdx, f, x);
+        load_face_na(m.fna, geometry_row(m, f), nh, area);
+        load_face_pair<DIM>(m.fdx, geometry_row(m, f), x);
         SD sl, sr;
         fused_side<DIM, RECON, VISC>(rec, T, hal, nem, lc, x[0], sl);
         if (rc == kFusedGhost) {
@@ -470,8 +470,8 @@ __device__ inline void march_face(const MeshView<double>& m, const Phys& ph, con
     constexpr int NE = DIM + 2;
     const int lc = code & 0xFFFF, rc = (int)((uint32_t)code >> 16);
     double nh[3], area, x[2][DIM];
-    load_face_na(m.fna, f, nh, area);
-    load_face_pair<DIM>(m.fdx, f, x);
+    load_face_na(m.fna, geometry_row(m, f), nh, area);
+    load_face_pair<DIM>(m.fdx, geometry_row(m, f), x);
     SD sl, sr;
     march_side<DIM, RECON, VISC>(ra, rb, T, hal, nem, lc, x[0], sl);
     if (rc == kFusedGhost) {

@@ -1,6 +1,7 @@
 // Host-side device-layout description of a finite-volume mesh for the RHS kernels.
 #pragma once
 #include <cstdint>
+#include <cstring>
 #include <vector>
 
 #include "../../include/ablate_fv.h"
@@ -32,6 +33,53 @@ struct Layout {
 
 // Validates the descriptor and fills the layout; throws std::invalid_argument on bad input.
 void build_layout(const abl_fv_mesh_desc& mesh, const abl_fv_physics_desc& phys, Layout& out);
+
+// The distinct rows (compared bit for bit) among n rows of `width` doubles, row i written by fetch(i, out): index[i]
+// is the number of row i in rows (rows[0 .. width) of row 0 is all zeros, kept whether used or not).  False, with
+// nothing kept, as soon as more than kMaxDistinctRows are found: boxes have a few hundred at most (their offsets
+// differ by rounding only, per direction), other meshes run over the limit within their first few thousand faces.  The
+// limit keeps a table of the widest rows (10 doubles) at 320 KB, a small part of an XCD's 4 MB L2.
+constexpr int kMaxDistinctRows = 4096;
+template <typename Fetch>
+bool distinct_rows(int64_t n, int width, Fetch&& fetch, std::vector<uint16_t>& index, std::vector<double>& rows) {
+    constexpr uint32_t kSlots = 4 * kMaxDistinctRows;
+    std::vector<int32_t> table(kSlots, -1);
+    std::vector<double> row((size_t)width, 0.0);
+    index.assign((size_t)n, 0);
+    rows.clear();
+    const size_t bytes = (size_t)width * sizeof(double);
+    auto find = [&]() -> int32_t {
+        uint64_t hash = 0x9E3779B97F4A7C15ull;
+        for (int j = 0; j < width; j++) {
+            uint64_t v;
+            std::memcpy(&v, &row[(size_t)j], 8);
+            hash = (hash ^ v) * 0xD6E8FEB86659FD93ull;
+            hash ^= hash >> 32;
+        }
+        for (uint32_t s = (uint32_t)hash % kSlots;; s = (s + 1) % kSlots) {
+            if (table[s] < 0) {
+                const int32_t r = (int32_t)(rows.size() / (size_t)width);
+                if (r > kMaxDistinctRows) return -1;
+                table[s] = r;
+                rows.insert(rows.end(), row.begin(), row.end());
+                return r;
+            }
+            if (std::memcmp(&rows[(size_t)table[s] * (size_t)width], row.data(), bytes) == 0) return table[s];
+        }
+    };
+    find();  // row 0: zeros
+    for (int64_t i = 0; i < n; i++) {
+        fetch(i, row.data());
+        const int32_t r = find();
+        if (r < 0) {
+            index = std::vector<uint16_t>();
+            rows = std::vector<double>();
+            return false;
+        }
+        index[(size_t)i] = (uint16_t)r;
+    }
+    return true;
+}
 
 // Cell tiles for the fused face-flux + gather kernel: tile t owns interior cells [t*T, min((t+1)*T, NI)).
 //   start[t] .. start[t+1]   its faces (every face with a cell in the tile), ascending face number

@@ -179,7 +179,8 @@ __device__ inline void load_rec_f(const float* __restrict__ rec, int64_t c, RecF
 // G is the storage/arithmetic type of weights and gradients (double: FP64 form, float: mixed form); state
 // differences are always taken in FP64 before rounding to G.  Each lane writes its cell's record: CellRec (FP64
 // form) or CellRecF (mixed form), word by word into the 64-cell blocks.
-template <typename G, int DIM, bool RECON, bool VISC, int LIM, int KM>
+// TAB: the slot geometry comes from the table of distinct rows (see MeshView).
+template <typename G, int DIM, bool RECON, bool VISC, int LIM, int KM, bool TAB>
 __device__ __forceinline__ void gradients_body(MeshView<G> m, Phys ph, const double* __restrict__ U,
                                                G* __restrict__ gradC, G* __restrict__ gradA, void* __restrict__ rec) {
     constexpr int NE = DIM + 2;
@@ -189,7 +190,12 @@ __device__ __forceinline__ void gradients_body(MeshView<G> m, Phys ph, const dou
     const int64_t c = active ? c_lane : m.NI - 1;  // lanes past the end shadow the last cell and store nothing
     const int64_t N = m.N, NI = m.NI;
     const G* __restrict__ wa_arr = m.swa ? m.swa : m.sw;
-    const bool own_wa = m.swa != nullptr;  // meshes without boundary faces share one weight set
+    // meshes without boundary faces share one weight set
+    const bool own_wa = TAB ? m.saux != 0 : m.swa != nullptr;
+    const G* __restrict__ row[KM];  // table rows of the slots
+    if (TAB)
+#pragma unroll
+        for (int k = 0; k < KM; k++) row[k] = m.stab + (uint32_t)m.srow[k * NI + c] * (uint32_t)m.sstride;
     double uc[NE], ac[NA];
 #pragma unroll
     for (int p = 0; p < NE; p++) uc[p] = U[p * N + c];
@@ -220,13 +226,19 @@ __device__ __forceinline__ void gradients_body(MeshView<G> m, Phys ph, const dou
 #pragma unroll
         for (int p = 0; p < NE; p++) un[p] = U[p * N + n];
         G w[DIM], wa[DIM];
+        if (TAB) {
+            if (RECON) load_row_words<0, DIM>(row[k], w);
+        } else {
 #pragma unroll
-        for (int d = 0; d < DIM; d++)
-            if (RECON) w[d] = m.sw[(k * DIM + d) * NI + c];
+            for (int d = 0; d < DIM; d++)
+                if (RECON) w[d] = m.sw[(k * DIM + d) * NI + c];
+        }
         if (VISC) {
             if (RECON && !own_wa) {  // the aux set is the cell set: reuse the words just loaded
 #pragma unroll
                 for (int d = 0; d < DIM; d++) wa[d] = w[d];
+            } else if (TAB) {
+                load_row_words<0, DIM>(row[k] + m.saux, wa);
             } else {
 #pragma unroll
                 for (int d = 0; d < DIM; d++) wa[d] = wa_arr[(k * DIM + d) * NI + c];
@@ -275,8 +287,11 @@ __device__ __forceinline__ void gradients_body(MeshView<G> m, Phys ph, const dou
             for (int k = 0; k < KM; k++) {
                 const bool valid = m.snbr[k * NI + c] >= 0;
                 G x[DIM];
+                if (TAB)
+                    load_row_words<DIM, DIM>(row[k], x);
+                else
 #pragma unroll
-                for (int d = 0; d < DIM; d++) x[d] = m.slim[(k * DIM + d) * NI + c];
+                    for (int d = 0; d < DIM; d++) x[d] = m.slim[(k * DIM + d) * NI + c];
                 if (!valid) continue;
 #pragma unroll
                 for (int p = 0; p < NE; p++) {
@@ -303,8 +318,11 @@ __device__ __forceinline__ void gradients_body(MeshView<G> m, Phys ph, const dou
                 const int32_t e = m.snbr[k * NI + c];
                 const int64_t n = e >= 0 ? (int64_t)e : c;
                 G v[DIM];  // x_n - x_c
+                if (TAB)
+                    load_row_words<DIM, DIM>(row[k], v);
+                else
 #pragma unroll
-                for (int d = 0; d < DIM; d++) v[d] = m.slim[(k * DIM + d) * NI + c];
+                    for (int d = 0; d < DIM; d++) v[d] = m.slim[(k * DIM + d) * NI + c];
                 if (e < 0) continue;
 #pragma unroll
                 for (int p = 0; p < NE; p++) {
@@ -378,19 +396,19 @@ __device__ __forceinline__ void gradients_body(MeshView<G> m, Phys ph, const dou
     }
 }
 
-template <typename G, int DIM, bool RECON, bool VISC, int LIM, int KM>
+template <typename G, int DIM, bool RECON, bool VISC, int LIM, int KM, bool TAB = false>
 __global__ __launch_bounds__(kBlock) void k_gradients(MeshView<G> m, Phys ph, const double* __restrict__ U,
                                                       G* __restrict__ gradC, G* __restrict__ gradA,
                                                       void* __restrict__ rec) {
-    gradients_body<G, DIM, RECON, VISC, LIM, KM>(m, ph, U, gradC, gradA, rec);
+    gradients_body<G, DIM, RECON, VISC, LIM, KM, TAB>(m, ph, U, gradC, gradA, rec);
 }
 // The same kernel held to 128 VGPRs (four waves per SIMD instead of three: more loads in flight).  Picked for the
 // FP64 3-D forms without the PETSc-family limiter, which fit without spilling (that limiter's would spill).
-template <typename G, int DIM, bool RECON, bool VISC, int LIM, int KM>
+template <typename G, int DIM, bool RECON, bool VISC, int LIM, int KM, bool TAB = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_gradients_w4(
     MeshView<G> m, Phys ph, const double* __restrict__ U, G* __restrict__ gradC, G* __restrict__ gradA,
     void* __restrict__ rec) {
-    gradients_body<G, DIM, RECON, VISC, LIM, KM>(m, ph, U, gradC, gradA, rec);
+    gradients_body<G, DIM, RECON, VISC, LIM, KM, TAB>(m, ph, U, gradC, gradA, rec);
 }
 
 // densityYi gradients (limited, one field) into gS [ns*DIM][N] and Yi aux gradients (unlimited) into gY [ns*DIM][N];
@@ -406,7 +424,6 @@ __device__ __forceinline__ void species_body(MeshView<G> m, Phys ph, const doubl
     const bool recon = ph.recon != 0;
     const bool aux = ph.sdiff != 0;
     const bool bj = ph.limiter == ABL_FV_LIMITER_BARTH_JESPERSEN;
-    const G* __restrict__ wa_arr = m.swa ? m.swa : m.sw;
     const double irho_c = 1.0 / U[kRho * N + c];
     // arithmetic of the gradient sums and the limiter: FP64 in the FP64 form; FP32 in the mixed form (which stores
     // these gradients in FP32), on FP64 state differences rounded once
@@ -423,10 +440,15 @@ __device__ __forceinline__ void species_body(MeshView<G> m, Phys ph, const doubl
         inner[k] = valid[k] && nb[k] < NI;
 #pragma unroll
         for (int d = 0; d < DIM; d++) {
-            w[k][d] = recon ? m.sw[(k * DIM + d) * NI + c] : G(0);
-            wa[k][d] = aux ? wa_arr[(k * DIM + d) * NI + c] : G(0);
-            xl[k][d] = (recon && m.slim) ? m.slim[(k * DIM + d) * NI + c] : G(0);
+            w[k][d] = G(0);
+            wa[k][d] = G(0);
+            xl[k][d] = G(0);
         }
+        if (recon) {
+            load_slot_vec<DIM, KM, kSlotWeight>(m, k, c, w[k]);
+            load_slot_vec<DIM, KM, kSlotLimiter>(m, k, c, xl[k]);
+        }
+        if (aux) load_slot_vec<DIM, KM, kSlotAux>(m, k, c, wa[k]);
         irn[k] = aux ? 1.0 / U[kRho * N + nb[k]] : 0.0;
     }
     bool cancel = false;
@@ -752,11 +774,11 @@ __global__ __launch_bounds__(kBlock) void k_flux(MeshView<double> m, Phys ph, co
         if (e < 0) break;
         const int64_t f = e >> 1;
         const int s = e & 1;
-        const int64_t L = m.fcell[f], Rc = m.fcell[F + f];
+        const int64_t L = m.fcell[f], Rc = m.fcell[F + f], g = geometry_row(m, f);
         const bool ghost = Rc >= NI;  // a ghost is always the right cell
         double nh[3], area, x[2][DIM];
-        load_face_na(m.fna, f, nh, area);
-        load_face_pair<DIM>(m.fdx, f, x);
+        load_face_na(m.fna, g, nh, area);
+        load_face_pair<DIM>(m.fdx, g, x);
         SD sl, sr;
         load_side<DIM, RECON, VISC>(U, rec, N, L, false, x[0], sl);
         load_side<DIM, RECON, VISC>(U, rec, N, Rc, ghost, x[1], sr);
@@ -787,11 +809,11 @@ __global__ __launch_bounds__(kBlock) void k_flux(MeshView<double> m, Phys ph, co
             if (e < 0) break;
             const int64_t f = e >> 1;
             const int s = e & 1;
-            const int64_t L = m.fcell[f], Rc = m.fcell[F + f];
+            const int64_t L = m.fcell[f], Rc = m.fcell[F + f], g = geometry_row(m, f);
             const bool ghost = Rc >= NI;
             double nh[3], area, x[2][DIM], w[2][DIM];
-            load_face_na(m.fna, f, nh, area);
-            load_face_pair<DIM>(m.fdx, f, x);
+            load_face_na(m.fna, g, nh, area);
+            load_face_pair<DIM>(m.fdx, g, x);
             if (VISC && ghost) load_face_pair<DIM>(wa_arr, f, w);
             SD sl, sr;
             load_side<DIM, RECON, VISC>(U, rec, N, L, false, x[0], sl);
@@ -816,15 +838,14 @@ __global__ __launch_bounds__(kBlock) void k_flux(MeshView<double> m, Phys ph, co
 template <int DIM, bool RECON, bool VISC, bool SPECIES, bool PAIRS = false>
 __device__ inline void eval_face(const MeshView<double>& m, const Phys& ph, const double* __restrict__ U,
                                  const double* __restrict__ gradC, const double* __restrict__ gradA,
-                                 const double* __restrict__ rec, int64_t f, double* fe, double* fs,
+                                 const double* __restrict__ rec, const FaceRef& fr, double* fe, double* fs,
                                  int64_t fs_stride) {
     using SD = SideData<DIM, VISC>;
-    const int64_t N = m.N, F = m.F, NI = m.NI;
-    const int64_t L = m.fcell[f], Rc = m.fcell[F + f];
+    const int64_t N = m.N, NI = m.NI, f = fr.f, L = fr.L, Rc = fr.R;
     const bool ghost = Rc >= NI;
     double nh[3], area, x[2][DIM], w[2][DIM];
-    load_face_na(m.fna, f, nh, area);
-    load_face_pair<DIM>(m.fdx, f, x);
+    load_face_na(m.fna, fr.g, nh, area);
+    load_face_pair<DIM>(m.fdx, fr.g, x);
     SD sl, sr;
     load_side<DIM, RECON, VISC>(U, rec, N, L, false, x[0], sl);
     load_side<DIM, RECON, VISC>(U, rec, N, Rc, ghost, x[1], sr);
@@ -868,7 +889,7 @@ __device__ __forceinline__ void face_flux_body(MeshView<double> m, Phys ph, cons
     const int64_t f = xcd_cell_index();
     if (f >= m.F) return;
     double flux[FS];
-    eval_face<DIM, RECON, VISC, SPECIES, true>(m, ph, U, gradC, gradA, rec, f, flux, Fs + 2 * f, 2 * m.F);
+    eval_face<DIM, RECON, VISC, SPECIES, true>(m, ph, U, gradC, gradA, rec, face_ref(m, f), flux, Fs + 2 * f, 2 * m.F);
     if (FS > NE) flux[FS - 1] = 0.0;
     double2* out = reinterpret_cast<double2*>(Fe + FS * f);
 #pragma unroll
@@ -886,14 +907,19 @@ __global__ __launch_bounds__(kBlock) void k_face_flux(MeshView<double> m, Phys p
 // Strategy 3 (tile): one workgroup per tile of T consecutive interior cells.  Its lanes evaluate every face of the
 // tile once into LDS (faces shared with a neighbouring tile are evaluated by both), then each lane gathers its
 // cell's faces from LDS in face-number order.  No face-flux round trip through HBM; the face fluxes and the
-// gather order are those of strategy 2, so the residual is bitwise the same.
+// gather order are those of strategy 2, so the residual is bitwise the same.  A tile's face list holds each face's
+// support cells, number and geometry row (TileFace), so that a face's records are one dependent load away.
+struct TileFace {
+    int32_t L, R, f, g;
+};
+__device__ inline FaceRef tile_face_ref(const int4& t) { return {t.z, t.x, t.y, t.w}; }
 template <int DIM, bool RECON, bool VISC, bool SPECIES, int KM>
 __global__ __launch_bounds__(kTileMax) void k_tile_flux(MeshView<double> m, Phys ph, const double* __restrict__ U,
                                                         const double* __restrict__ gradC,
                                                         const double* __restrict__ gradA,
                                                         const double* __restrict__ rec,
                                                         const int32_t* __restrict__ tstart,
-                                                        const int32_t* __restrict__ tfaces,
+                                                        const int4* __restrict__ tfaces,
                                                         const int32_t* __restrict__ tslot, int nfm,
                                                         double* __restrict__ R, int accumulate) {
     constexpr int NE = DIM + 2;
@@ -902,13 +928,13 @@ __global__ __launch_bounds__(kTileMax) void k_tile_flux(MeshView<double> m, Phys
     double* ls = lds + NE * nfm;   // [ns][nfm]
     const int64_t t = xcd_block_index();
     const int32_t f0 = tstart[t], nf = tstart[t + 1] - f0;
-    // the face number of a lane's next face is loaded one round ahead
-    int32_t fnext = (int)threadIdx.x < nf ? tfaces[f0 + threadIdx.x] : 0;
+    // a lane's next face entry is loaded one round ahead
+    int4 fnext = (int)threadIdx.x < nf ? tfaces[f0 + threadIdx.x] : make_int4(0, 0, 0, 0);
     for (int i = threadIdx.x; i < nf; i += blockDim.x) {
         double flux[NE];
-        const int32_t fcur = fnext;
+        const int4 fcur = fnext;
         if (i + (int)blockDim.x < nf) fnext = tfaces[f0 + i + blockDim.x];
-        eval_face<DIM, RECON, VISC, SPECIES>(m, ph, U, gradC, gradA, rec, (int64_t)fcur, flux, ls + i, nfm);
+        eval_face<DIM, RECON, VISC, SPECIES>(m, ph, U, gradC, gradA, rec, tile_face_ref(fcur), flux, ls + i, nfm);
 #pragma unroll
         for (int p = 0; p < NE; p++) le[p * nfm + i] = flux[p];
     }
@@ -1106,17 +1132,16 @@ __device__ inline void phys_flux_pert(const SidePert<DIM>& sp, const BaselineF<D
 template <int DIM, bool RECON, bool VISC, bool SPECIES, bool RUS>
 __device__ inline void mixed_face(const MeshView<float>& m, const Phys& ph, const double* __restrict__ U,
                                   const float* __restrict__ rec, const float* __restrict__ gS,
-                                  const float* __restrict__ gY, int64_t f, float* dFL, float* dFR, float* sFL,
+                                  const float* __restrict__ gY, const FaceRef& fr, float* dFL, float* dFR, float* sFL,
                                   float* sFR, int64_t s_stride) {
     constexpr int NE = DIM + 2;
     constexpr int NT = ViscTerms<DIM>::NT;
     constexpr bool USE_REC = RECON || VISC;
-    const int64_t N = m.N, F = m.F, NI = m.NI;
-    const int64_t L = m.fcell[f], Rc = m.fcell[F + f];
+    const int64_t N = m.N, NI = m.NI, f = fr.f, L = fr.L, Rc = fr.R;
     const bool ghost = Rc >= NI;
     float nh[3], area, x[2][DIM];
-    load_face_na(m.fna, f, nh, area);
-    load_face_pair<DIM, float>(m.fdx, f, x);
+    load_face_na(m.fna, fr.g, nh, area);
+    load_face_pair<DIM, float>(m.fdx, fr.g, x);
     float nhat[DIM];
 #pragma unroll
     for (int d = 0; d < DIM; d++) nhat[d] = nh[d];
@@ -1437,7 +1462,7 @@ __global__ __launch_bounds__(kBlock) void k_flux_mixed(MeshView<float> m, Phys p
         const int32_t e = m.ell[k * NI + c];
         if (e < 0) break;
         float dFL[NE], dFR[NE];
-        mixed_face<DIM, RECON, VISC, false, RUS>(m, ph, U, rec, nullptr, nullptr, (int64_t)(e >> 1), dFL, dFR, nullptr,
+        mixed_face<DIM, RECON, VISC, false, RUS>(m, ph, U, rec, nullptr, nullptr, face_ref(m, e >> 1), dFL, dFR, nullptr,
                                             nullptr, 0);
         if (e & 1) {
 #pragma unroll
@@ -1464,7 +1489,7 @@ __global__ __launch_bounds__(kTileMax) void k_tile_flux_mixed(MeshView<float> m,
                                                               const float* __restrict__ gS,
                                                               const float* __restrict__ gY,
                                                               const int32_t* __restrict__ tstart,
-                                                              const int32_t* __restrict__ tfaces,
+                                                              const int4* __restrict__ tfaces,
                                                               const int32_t* __restrict__ tslot, int nfm,
                                                               double* __restrict__ R, int accumulate) {
     constexpr int NE = DIM + 2;
@@ -1475,7 +1500,7 @@ __global__ __launch_bounds__(kTileMax) void k_tile_flux_mixed(MeshView<float> m,
     const int32_t f0 = tstart[t], nf = tstart[t + 1] - f0;
     for (int i = threadIdx.x; i < nf; i += blockDim.x) {
         float dFL[NE], dFR[NE];
-        mixed_face<DIM, RECON, VISC, SPECIES, RUS>(m, ph, U, rec, gS, gY, (int64_t)tfaces[f0 + i], dFL, dFR,
+        mixed_face<DIM, RECON, VISC, SPECIES, RUS>(m, ph, U, rec, gS, gY, tile_face_ref(tfaces[f0 + i]), dFL, dFR,
                                               lf + NE * nfm + i, lf + (nrow + NE) * nfm + i, nfm);
 #pragma unroll
         for (int p = 0; p < NE; p++) {
@@ -1519,7 +1544,7 @@ __global__ __launch_bounds__(kBlock) void k_face_flux_mixed(MeshView<float> m, P
     if (f >= m.F) return;
     const int64_t F = m.F;
     float dFL[NE], dFR[NE];
-    mixed_face<DIM, RECON, VISC, SPECIES, RUS>(m, ph, U, rec, gS, gY, f, dFL, dFR, Fm + NE * F + f,
+    mixed_face<DIM, RECON, VISC, SPECIES, RUS>(m, ph, U, rec, gS, gY, face_ref(m, f), dFL, dFR, Fm + NE * F + f,
                                                Fm + (nrow + NE) * F + f, F);
 #pragma unroll
     for (int p = 0; p < NE; p++) {
@@ -1617,7 +1642,7 @@ __global__ __launch_bounds__(kBlock) void k_vjp(MeshView<double> m, Phys ph, con
         const bool ghost = Rc >= NI;
         cghost[k] = 0.0;
         double nh[3], area, uL[NE], uR[NE], fb[NE], QL, QR, QdL;
-        load_face_na(m.fna, f, nh, area);
+        load_face_na(m.fna, geometry_row(m, f), nh, area);
 #pragma unroll
         for (int p = 0; p < NE; p++) {
             uL[p] = U[p * N + L];
@@ -1700,7 +1725,7 @@ __global__ __launch_bounds__(kBlock) void k_vjp_faces(MeshView<double> m, Phys p
     const int64_t L = m.fcell[f], Rc = m.fcell[F + f];
     const bool ghost = Rc >= NI;
     double nh[3], area, uL[NE], uR[NE], fb[NE], QL, QR, QdL;
-    load_face_na(m.fna, f, nh, area);
+    load_face_na(m.fna, geometry_row(m, f), nh, area);
 #pragma unroll
     for (int p = 0; p < NE; p++) {
         uL[p] = U[p * N + L];
@@ -1809,7 +1834,7 @@ __global__ __launch_bounds__(kBlock) void k_vjp_theta(MeshView<double> m, Phys p
         const int64_t N = m.N, F = m.F;
         const int64_t L = m.fcell[f], G = m.fcell[F + f];
         double nh[3], area, uL[NE], uG[NE], fb[NE], QL, QR, QdL;
-        load_face_na(m.fna, f, nh, area);
+        load_face_na(m.fna, geometry_row(m, f), nh, area);
 #pragma unroll
         for (int p = 0; p < NE; p++) {
             uL[p] = U[p * N + L];
@@ -1922,8 +1947,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
     const int64_t L = m.fcell[f], Rc = m.fcell[F + f];
     const bool ghost = Rc >= NI;
     double nh[3], area, x[2][DIM];
-    load_face_na(m.fna, f, nh, area);
-    load_face_pair<DIM>(m.fdx, f, x);
+    const int64_t geo = geometry_row(m, f);
+    load_face_na(m.fna, geo, nh, area);
+    load_face_pair<DIM>(m.fdx, geo, x);
     const double ivL = m.inv_vol[L], ivR = ghost ? 0.0 : m.inv_vol[Rc];
     double g[NE];
 #pragma unroll
@@ -2309,7 +2335,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_cells_e(MeshView<double> m, Phys
         nb[k] = valid[k] ? (int64_t)n : c;
         bnd[k] = nb[k] >= NI;
         double x[2][DIM];
-        load_face_pair<DIM>(m.fdx, f, x);
+        load_face_pair<DIM>(m.fdx, geometry_row(m, f), x);
 #pragma unroll
         for (int d = 0; d < DIM; d++) xs[k][d] = s ? x[1][d] : x[0][d];
         // the record pairs this cell needs: its side's face-state adjoint, the viscous terms and face velocity, the
@@ -2390,9 +2416,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_cells_e(MeshView<double> m, Phys
     if (recon) {
         double wl[KM][DIM];
 #pragma unroll
-        for (int k = 0; k < KM; k++)
-#pragma unroll
-            for (int d = 0; d < DIM; d++) wl[k][d] = m.sw[(k * DIM + d) * NI + c];
+        for (int k = 0; k < KM; k++) load_slot_vec<DIM, KM, kSlotWeight>(m, k, c, wl[k]);
 #pragma unroll
         for (int p = 0; p < NE; p++) {
             double cn[KM], unv[KM];
@@ -2408,7 +2432,6 @@ __global__ __launch_bounds__(kBlock) void k_adj_cells_e(MeshView<double> m, Phys
         }
     }
     if (visc) {
-        const double* __restrict__ wa_arr = m.swa ? m.swa : m.sw;
         double gAb[DIM + 1][DIM], acb[DIM + 1];
 #pragma unroll
         for (int q = 0; q <= DIM; q++) {
@@ -2420,12 +2443,13 @@ __global__ __launch_bounds__(kBlock) void k_adj_cells_e(MeshView<double> m, Phys
 #pragma unroll
         for (int k = 0; k < KM; k++) {
             if (!valid[k]) continue;
-            double anb[DIM + 1], un[NE], unb[NE];
+            double anb[DIM + 1], un[NE], unb[NE], wa[DIM];
+            load_slot_vec<DIM, KM, kSlotAux>(m, k, c, wa);
 #pragma unroll
             for (int q = 0; q <= DIM; q++) {
                 double t = 0.0;
 #pragma unroll
-                for (int d = 0; d < DIM; d++) t += wa_arr[(k * DIM + d) * NI + c] * gAb[q][d];
+                for (int d = 0; d < DIM; d++) t += wa[d] * gAb[q][d];
                 anb[q] = t;
                 acb[q] -= t;
             }
@@ -2469,7 +2493,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     const bool recon = ph.recon != 0, sdiff = ph.sdiff != 0;
     const bool bj = ph.limiter == ABL_FV_LIMITER_BARTH_JESPERSEN;
     const double2* __restrict__ W = reinterpret_cast<const double2*>(b.W);
-    const double* __restrict__ wa_arr = m.swa ? m.swa : m.sw;
     int64_t nb[KM], wb[KM], gi[KM];
     bool valid[KM], bnd[KM];
     double xs[KM][DIM], cnv[KM][DIM], csk[KM], wl[KM][DIM], wa[KM][DIM];
@@ -2485,8 +2508,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
         gi[k] = (valid[k] && bnd[k]) ? nb[k] - NI : -1;
         wb[k] = adjw_pair(f, b.nwp);
         double x[2][DIM], nh[3], area;
-        load_face_pair<DIM>(m.fdx, f, x);
-        load_face_na(m.fna, f, nh, area);
+        const int64_t geo = geometry_row(m, f);
+        load_face_pair<DIM>(m.fdx, geo, x);
+        load_face_na(m.fna, geo, nh, area);
         double cw[4];  // words CL, CR, CD of the record (two pairs from CL's pair on)
         {
             const double2 v0 = W[wb[k] + 64 * (AW::CL / 2)], v1 = W[wb[k] + 64 * (AW::CL / 2 + 1)];
@@ -2502,9 +2526,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
         for (int d = 0; d < DIM; d++) {
             xs[k][d] = s ? x[1][d] : x[0][d];
             cnv[k][d] = cd * nh[d];
-            wl[k][d] = recon ? m.sw[(k * DIM + d) * NI + c] : 0.0;
-            wa[k][d] = sdiff ? wa_arr[(k * DIM + d) * NI + c] : 0.0;
+            wl[k][d] = 0.0;
+            wa[k][d] = 0.0;
         }
+        if (recon) load_slot_vec<DIM, KM, kSlotWeight>(m, k, c, wl[k]);
+        if (sdiff) load_slot_vec<DIM, KM, kSlotAux>(m, k, c, wa[k]);
     }
     const double rho_c = U[c];
     double rbc = 0.0, rbn[KM], rho_n[KM];
@@ -2747,7 +2773,6 @@ __global__ __launch_bounds__(kBlock) void k_face_interpolate(MeshView<double> m,
     const int64_t N = m.N, NI = m.NI, F = m.F;
     const int64_t L = m.fcell[f], R = m.fcell[F + f];
     const bool ghost = R >= NI;
-    const double* __restrict__ wa_arr = m.swa ? m.swa : m.sw;
     const int nq = nc + 1 + DIM + ph.ns;
     for (int q = 0; q < nq; q++) {
         const double vL = face_interp_value<DIM, KM>(U, N, nc, ph, q, L);
@@ -2770,8 +2795,10 @@ __global__ __launch_bounds__(kBlock) void k_face_interpolate(MeshView<double> m,
                 const int32_t e = m.snbr[k * NI + c];
                 if (e < 0) continue;
                 const double dv = face_interp_value<DIM, KM>(U, N, nc, ph, q, e) - vc;
+                double wa[DIM];
+                load_slot_vec<DIM, KM, kSlotAux>(m, k, c, wa);
 #pragma unroll
-                for (int d = 0; d < DIM; d++) gc[d] += wa_arr[(k * DIM + d) * NI + c] * dv;
+                for (int d = 0; d < DIM; d++) gc[d] += wa[d] * dv;
             }
 #pragma unroll
             for (int d = 0; d < DIM; d++) g[d] += 0.5 * gc[d];
@@ -2826,25 +2853,25 @@ using FaceFluxKernel = void (*)(MeshView<double>, Phys, const double*, const dou
                                 double*, double*);
 using GatherKernel = void (*)(MeshView<double>, int, const double*, const double*, double*, int);
 
-template <typename G, int DIM, int KM>
+template <typename G, int DIM, int KM, bool TAB>
 GradKernelT<G> pick_gradients_k(bool recon, bool visc, int lim) {
-    if (!recon) return visc ? k_gradients<G, DIM, false, true, kLimNone, KM> : nullptr;
+    if (!recon) return visc ? k_gradients<G, DIM, false, true, kLimNone, KM, TAB> : nullptr;
     if constexpr (sizeof(G) == 8 && DIM == 3) {
         if (lim != kLimPetsc) {
-            if (visc) return lim == kLimBJ ? k_gradients_w4<G, DIM, true, true, kLimBJ, KM>
-                                           : k_gradients_w4<G, DIM, true, true, kLimNone, KM>;
-            return lim == kLimBJ ? k_gradients_w4<G, DIM, true, false, kLimBJ, KM>
-                                 : k_gradients_w4<G, DIM, true, false, kLimNone, KM>;
+            if (visc) return lim == kLimBJ ? k_gradients_w4<G, DIM, true, true, kLimBJ, KM, TAB>
+                                           : k_gradients_w4<G, DIM, true, true, kLimNone, KM, TAB>;
+            return lim == kLimBJ ? k_gradients_w4<G, DIM, true, false, kLimBJ, KM, TAB>
+                                 : k_gradients_w4<G, DIM, true, false, kLimNone, KM, TAB>;
         }
     }
     if (visc) {
-        if (lim == kLimBJ) return k_gradients<G, DIM, true, true, kLimBJ, KM>;
-        if (lim == kLimPetsc) return k_gradients<G, DIM, true, true, kLimPetsc, KM>;
-        return k_gradients<G, DIM, true, true, kLimNone, KM>;
+        if (lim == kLimBJ) return k_gradients<G, DIM, true, true, kLimBJ, KM, TAB>;
+        if (lim == kLimPetsc) return k_gradients<G, DIM, true, true, kLimPetsc, KM, TAB>;
+        return k_gradients<G, DIM, true, true, kLimNone, KM, TAB>;
     }
-    if (lim == kLimBJ) return k_gradients<G, DIM, true, false, kLimBJ, KM>;
-    if (lim == kLimPetsc) return k_gradients<G, DIM, true, false, kLimPetsc, KM>;
-    return k_gradients<G, DIM, true, false, kLimNone, KM>;
+    if (lim == kLimBJ) return k_gradients<G, DIM, true, false, kLimBJ, KM, TAB>;
+    if (lim == kLimPetsc) return k_gradients<G, DIM, true, false, kLimPetsc, KM, TAB>;
+    return k_gradients<G, DIM, true, false, kLimNone, KM, TAB>;
 }
 // Compile-time slot width of the cell -> face table: 4 (quads, tets), 6 (hexes) or 8.
 inline int slot_width(int K) { return K <= 4 ? 4 : (K <= 6 ? 6 : 8); }
@@ -2858,11 +2885,12 @@ void pick_adj(bool rusanov, int K, AdjFacesKernel& fk, AdjCellsKernel& ce, AdjCe
     }
 }
 template <typename G, int DIM>
-GradKernelT<G> pick_gradients(bool recon, bool visc, int lim, int K) {
+GradKernelT<G> pick_gradients(bool recon, bool visc, int lim, int K, bool tab) {
+    if (tab) return pick_gradients_k<G, DIM, DIM == 2 ? 4 : 6, true>(recon, visc, lim);
     switch (slot_width(K)) {
-        case 4: return pick_gradients_k<G, DIM, 4>(recon, visc, lim);
-        case 6: return pick_gradients_k<G, DIM, 6>(recon, visc, lim);
-        default: return pick_gradients_k<G, DIM, 8>(recon, visc, lim);
+        case 4: return pick_gradients_k<G, DIM, 4, false>(recon, visc, lim);
+        case 6: return pick_gradients_k<G, DIM, 6, false>(recon, visc, lim);
+        default: return pick_gradients_k<G, DIM, 8, false>(recon, visc, lim);
     }
 }
 
@@ -2895,7 +2923,7 @@ MixedFluxKernel pick_flux_mixed(bool recon, bool visc, bool rus) {
     return rus ? pick_flux_mixed2<DIM, true>(recon, visc) : pick_flux_mixed2<DIM, false>(recon, visc);
 }
 using TileMixedKernel = void (*)(MeshView<float>, Phys, const double*, const float*, const float*, const float*,
-                                 const int32_t*, const int32_t*, const int32_t*, int, double*, int);
+                                 const int32_t*, const int4*, const int32_t*, int, double*, int);
 template <int DIM, bool RECON, bool VISC, bool SPECIES, bool RUS>
 TileMixedKernel pick_tile_mixed3(int K) {
     switch (slot_width(K)) {
@@ -2978,7 +3006,7 @@ VjpThetaKernel pick_vjp_theta(bool rusanov) {
     return rusanov ? k_vjp_theta<DIM, true> : k_vjp_theta<DIM, false>;
 }
 using TileKernel = void (*)(MeshView<double>, Phys, const double*, const double*, const double*, const double*,
-                           const int32_t*, const int32_t*, const int32_t*, int, double*, int);
+                           const int32_t*, const int4*, const int32_t*, int, double*, int);
 template <int DIM, bool RECON, bool VISC, int KM>
 TileKernel pick_tile3(bool species) {
     return species ? k_tile_flux<DIM, RECON, VISC, true, KM> : k_tile_flux<DIM, RECON, VISC, false, KM>;
@@ -3288,13 +3316,13 @@ struct SlotGeometry {
     std::vector<G> w, wa, lim;
 };
 template <typename G>
-void build_slot_geometry(const Layout& L, int KM, int lim, SlotGeometry<G>& out) {
+void build_slot_geometry(const Layout& L, int KM, int lim, bool vectors, SlotGeometry<G>& out) {
     const int dim = L.dim;
     const int64_t NI = L.NI, F = L.F;
     out.nbr.assign((size_t)KM * NI, -1);
-    if (!L.fw.empty()) out.w.assign((size_t)KM * dim * NI, G(0));
-    if (!L.fwa.empty()) out.wa.assign((size_t)KM * dim * NI, G(0));
-    if (lim != kLimNone) out.lim.assign((size_t)KM * dim * NI, G(0));
+    if (vectors && !L.fw.empty()) out.w.assign((size_t)KM * dim * NI, G(0));
+    if (vectors && !L.fwa.empty()) out.wa.assign((size_t)KM * dim * NI, G(0));
+    if (vectors && lim != kLimNone) out.lim.assign((size_t)KM * dim * NI, G(0));
     for (int k = 0; k < L.K; k++)
         for (int64_t c = 0; c < NI; c++) {
             const int32_t e = L.ell[(size_t)k * NI + c];
@@ -3302,7 +3330,7 @@ void build_slot_geometry(const Layout& L, int KM, int lim, SlotGeometry<G>& out)
             const int64_t f = e >> 1;
             const int s = e & 1;
             out.nbr[(size_t)k * NI + c] = L.fcell[(size_t)(1 - s) * F + f];
-            for (int d = 0; d < dim; d++) {
+            for (int d = 0; vectors && d < dim; d++) {
                 const size_t o = ((size_t)k * dim + d) * NI + c;
                 const size_t a = (size_t)2 * dim * f + (size_t)s * dim + d;
                 const size_t b = (size_t)2 * dim * f + (size_t)(1 - s) * dim + d;
@@ -3312,6 +3340,40 @@ void build_slot_geometry(const Layout& L, int KM, int lim, SlotGeometry<G>& out)
                 else if (lim == kLimPetsc) out.lim[o] = G(L.fdx[a]) - G(L.fdx[b]);
             }
         }
+}
+
+// The same per-slot geometry as distinct rows (w, limiter geometry, aux weights when they are their own set; an even
+// number of words per row): quads and hexes only.  False when the mesh has too many distinct ones.
+template <typename G>
+struct SlotRows {
+    std::vector<uint16_t> row;
+    std::vector<G> table;
+    int stride = 0, aux = 0;
+};
+template <typename G>
+bool build_slot_rows(const Layout& L, int KM, int lim, SlotRows<G>& out) {
+    const int dim = L.dim;
+    if (L.fw.empty() || !(dim == 2 ? KM == 4 : KM == 6)) return false;
+    const int64_t NI = L.NI;
+    out.aux = L.fwa.empty() ? 0 : 2 * dim;
+    out.stride = (out.aux ? 3 * dim + 1 : 2 * dim) & ~1;
+    std::vector<double> rows;
+    auto fetch = [&](int64_t i, double* r) {
+        for (int j = 0; j < out.stride; j++) r[j] = 0.0;
+        const int32_t e = i < (int64_t)L.K * NI ? L.ell[(size_t)i] : -1;
+        if (e < 0) return;
+        const size_t a = (size_t)2 * dim * (e >> 1) + (size_t)(e & 1) * dim;
+        const size_t b = (size_t)2 * dim * (e >> 1) + (size_t)(1 - (e & 1)) * dim;
+        for (int d = 0; d < dim; d++) {
+            r[d] = G(L.fw[a + d]);
+            if (lim == kLimBJ) r[dim + d] = G(L.fdx[a + d]);
+            else if (lim == kLimPetsc) r[dim + d] = G(L.fdx[a + d]) - G(L.fdx[b + d]);
+            if (out.aux) r[out.aux + d] = G(L.fwa[a + d]);
+        }
+    };
+    if (!distinct_rows((int64_t)KM * NI, out.stride, fetch, out.row, rows)) return false;
+    out.table.assign(rows.begin(), rows.end());
+    return true;
 }
 
 }  // namespace abl
@@ -3325,13 +3387,20 @@ struct abl_fv_solver {
     abl::DevBuf<int32_t> ell, fcell, bface, bslot, slot_kind, snbr;
     abl::DevBuf<double> fna, fdx, fwa, inv_vol, gradC, gradA, slot_state;
     abl::DevBuf<double> sw, swa, slim;  // slot-major gradient geometry (FP64 form)
+    // distinct geometry rows (boxes): row numbers per face and slot; the tables are fna, fdx and stab
+    abl::DevBuf<uint16_t> frow, srow;
+    abl::DevBuf<double> stab;
+    abl::DevBuf<float> stab_f;
+    int slot_stride = 0, slot_aux = 0;
+    bool slot_rows = false;
     abl::DevBuf<double> rec;            // cell records of the FP64 form (rec_pair blocks)
     // face fluxes (allocated when that strategy is selected): FP64 euler records [F][FS] and species pairs
     // [ns/2][F][2];
     // mixed form rows [2 (n_euler + n_species)][F]
     abl::DevBuf<double> face_flux_e, face_flux_s;
     abl::DevBuf<float> face_flux_m;
-    abl::DevBuf<int32_t> tile_start, tile_faces, tile_slot;  // tile strategy (built when selected)
+    abl::DevBuf<int32_t> tile_start, tile_slot;  // tile strategy (built when selected)
+    abl::DevBuf<int4> tile_faces;                // TileFace entries
     int tile_T = 0, tile_nfm = 0;
     int64_t tile_n = 0;
     size_t tile_lds = 0;
@@ -3463,6 +3532,11 @@ struct abl_fv_solver {
         v.sw = sw.ptr;
         v.swa = swa.ptr;
         v.slim = slim.ptr;
+        v.frow = frow.ptr;
+        v.srow = srow.ptr;
+        v.stab = stab.ptr;
+        v.sstride = slot_stride;
+        v.saux = slot_aux;
         return v;
     }
     abl::MeshView<float> view_f() const {
@@ -3482,6 +3556,11 @@ struct abl_fv_solver {
         v.sw = sw_f.ptr;
         v.swa = swa_f.ptr;
         v.slim = slim_f.ptr;
+        v.frow = frow.ptr;
+        v.srow = srow.ptr;
+        v.stab = stab_f.ptr;
+        v.sstride = slot_stride;
+        v.saux = slot_aux;
         return v;
     }
     // Face-flux storage of strategy 2 (see the members).
@@ -3503,7 +3582,8 @@ struct abl_fv_solver {
     // budget.  Needs the host cell -> face table, so it is built at creation.
     // only_T = 0: the largest of 256/128/64 cells within the default LDS budget; otherwise exactly only_T cells
     // within the workgroup LDS limit.  Returns false when no size fits (the strategy then stays unavailable).
-    bool build_tiles(const abl::Layout& lay, int only_T = 0) {
+    // face_rows: geometry row of every face (empty: the face number).
+    bool build_tiles(const abl::Layout& lay, const std::vector<uint16_t>& face_rows, int only_T = 0) {
         const int KM = abl::slot_width(lay.K);
         // LDS per face: FP64 euler + species fluxes, or the mixed form's two FP32 perturbation records
         const int per_face = form == ABL_FV_FORM_FP64 ? (lay.dim + 2 + lay.ns) * (int)sizeof(double)
@@ -3524,7 +3604,13 @@ struct abl_fv_solver {
             HIP_CHECK(hipFuncSetAttribute((const void*)tile_kernel_mixed, hipFuncAttributeMaxDynamicSharedMemorySize,
                                           (int)((size_t)tl.nf_max * per_face)));
         tile_start.upload(tl.start);
-        tile_faces.upload(tl.faces);
+        std::vector<int4> entries(tl.faces.size());
+        for (size_t i = 0; i < entries.size(); i++) {
+            const int32_t f = tl.faces[i];
+            entries[i] = make_int4(lay.fcell[(size_t)f], lay.fcell[(size_t)(host.F + f)], f,
+                                   face_rows.empty() ? f : (int32_t)face_rows[(size_t)f]);
+        }
+        tile_faces.upload(entries);
         tile_slot.upload(tl.slot);
         tile_T = tl.T;
         tile_n = tl.n;
@@ -3675,7 +3761,7 @@ struct abl_fv_solver {
         return ABL_FV_STRATEGY_FACE_FLUX;
     }
     int64_t device_bytes() const {
-        return (int64_t)(ell.bytes() + fcell.bytes() + bface.bytes() + bslot.bytes() + slot_kind.bytes() + fna.bytes() + fdx.bytes() + face_flux_e.bytes() + face_flux_s.bytes() + face_flux_m.bytes() + tile_start.bytes() + tile_faces.bytes() + tile_slot.bytes() + fu_start.bytes() + fu_faces.bytes() + fu_code.bytes() + fu_slot.bytes() + fu_hstart.bytes() + fu_hcell.bytes() + fu_hinfo.bytes() + mr_seq.bytes() + mr_pro.bytes() + mr_stile.bytes() + mr_snext.bytes() + mr_fstart.bytes() + mr_ffaces.bytes() + mr_fcode.bytes() + mr_pfstart.bytes() + mr_pffaces.bytes() + mr_pfcode.bytes() + mr_hstart.bytes() + mr_hcell.bytes() + mr_hinfo.bytes() + mr_gslot.bytes() + snbr.bytes() + vjp_rows.bytes() + sw.bytes() + swa.bytes() + slim.bytes() + sw_f.bytes() + swa_f.bytes() + slim_f.bytes() + fwa.bytes() + inv_vol.bytes() + gradC.bytes() +
+        return (int64_t)(frow.bytes() + srow.bytes() + stab.bytes() + stab_f.bytes() + ell.bytes() + fcell.bytes() + bface.bytes() + bslot.bytes() + slot_kind.bytes() + fna.bytes() + fdx.bytes() + face_flux_e.bytes() + face_flux_s.bytes() + face_flux_m.bytes() + tile_start.bytes() + tile_faces.bytes() + tile_slot.bytes() + fu_start.bytes() + fu_faces.bytes() + fu_code.bytes() + fu_slot.bytes() + fu_hstart.bytes() + fu_hcell.bytes() + fu_hinfo.bytes() + mr_seq.bytes() + mr_pro.bytes() + mr_stile.bytes() + mr_snext.bytes() + mr_fstart.bytes() + mr_ffaces.bytes() + mr_fcode.bytes() + mr_pfstart.bytes() + mr_pffaces.bytes() + mr_pfcode.bytes() + mr_hstart.bytes() + mr_hcell.bytes() + mr_hinfo.bytes() + mr_gslot.bytes() + snbr.bytes() + vjp_rows.bytes() + sw.bytes() + swa.bytes() + slim.bytes() + sw_f.bytes() + swa_f.bytes() + slim_f.bytes() + fwa.bytes() + inv_vol.bytes() + gradC.bytes() +
                          gradA.bytes() + rec.bytes() + adjUghost.bytes() + adjUself.bytes() + adjContrib.bytes() + adjW.bytes() + adjGL.bytes() + mirror.bytes() + recf.bytes() + gS_f.bytes() + gY_f.bytes() + rmin.bytes() + cfl_partial.bytes() + dt_partial.bytes() + cfl_out.bytes() + slot_state.bytes() + counter.bytes() + fna_f.bytes() + fdx_f.bytes() +
                          fwa_f.bytes());
     }
@@ -3776,10 +3862,39 @@ extern "C" int abl_fv_create(const abl_fv_mesh_desc* mesh, const abl_fv_physics_
         const int lim = p.limiter == ABL_FV_LIMITER_NONE ? abl::kLimNone
                         : p.limiter == ABL_FV_LIMITER_BARTH_JESPERSEN ? abl::kLimBJ : abl::kLimPetsc;
         const bool species = p.n_species > 0;
+        // geometry tables of meshes with few distinct face and slot records (else every face and slot keeps its own)
+        std::vector<uint16_t> face_rows;
+        std::vector<double> face_table;  // 4 words of fna, 2 dim of fdx
+        const int face_words = 4 + 2 * L.dim;
+        if (abl::distinct_rows(L.F, face_words,
+                               [&](int64_t f, double* r) {
+                                   for (int j = 0; j < 4; j++) r[j] = L.fna[(size_t)4 * f + j];
+                                   for (int j = 0; j < 2 * L.dim; j++) r[4 + j] = L.fdx[(size_t)2 * L.dim * f + j];
+                               },
+                               face_rows, face_table))
+            s->frow.upload(face_rows);
+        abl::SlotRows<double> slots;
+        abl::SlotRows<float> slots_f;
+        s->slot_rows = form == ABL_FV_FORM_FP64 ? abl::build_slot_rows<double>(L, abl::slot_width(L.K), lim, slots)
+                                                : abl::build_slot_rows<float>(L, abl::slot_width(L.K), lim, slots_f);
+        if (s->slot_rows) {
+            s->srow.upload(form == ABL_FV_FORM_FP64 ? slots.row : slots_f.row);
+            s->slot_stride = form == ABL_FV_FORM_FP64 ? slots.stride : slots_f.stride;
+            s->slot_aux = form == ABL_FV_FORM_FP64 ? slots.aux : slots_f.aux;
+        }
+        // the face geometry arrays as uploaded: all faces, or the distinct rows
+        auto face_array = [&](const std::vector<double>& all, int first, int words) {
+            if (face_rows.empty()) return all;
+            std::vector<double> t;
+            for (size_t r = 0; r * face_words < face_table.size(); r++)
+                t.insert(t.end(), face_table.begin() + (ptrdiff_t)(r * face_words + first),
+                         face_table.begin() + (ptrdiff_t)(r * face_words + first + words));
+            return t;
+        };
         if (mesh->dim == 3) {
             s->species_kernel = abl::pick_species_gradients<double, 3>(L.K);
             s->species_kernel_f = abl::pick_species_gradients<float, 3>(L.K);
-            s->grad_kernel = abl::pick_gradients<double, 3>(s->recon, s->visc, lim, L.K);
+            s->grad_kernel = abl::pick_gradients<double, 3>(s->recon, s->visc, lim, L.K, s->slot_rows);
             s->flux_kernel = abl::pick_flux<3>(s->recon, s->visc, species);
             s->face_flux_kernel = abl::pick_face_flux<3>(s->recon, s->visc, species);
             s->tile_kernel = abl::pick_tile<3>(s->recon, s->visc, species, L.K);
@@ -3789,7 +3904,7 @@ extern "C" int abl_fv_create(const abl_fv_mesh_desc* mesh, const abl_fv_physics_
         } else {
             s->species_kernel = abl::pick_species_gradients<double, 2>(L.K);
             s->species_kernel_f = abl::pick_species_gradients<float, 2>(L.K);
-            s->grad_kernel = abl::pick_gradients<double, 2>(s->recon, s->visc, lim, L.K);
+            s->grad_kernel = abl::pick_gradients<double, 2>(s->recon, s->visc, lim, L.K, s->slot_rows);
             s->flux_kernel = abl::pick_flux<2>(s->recon, s->visc, species);
             s->face_flux_kernel = abl::pick_face_flux<2>(s->recon, s->visc, species);
             s->tile_kernel = abl::pick_tile<2>(s->recon, s->visc, species, L.K);
@@ -3804,10 +3919,11 @@ extern "C" int abl_fv_create(const abl_fv_mesh_desc* mesh, const abl_fv_physics_
         const int64_t N = L.N;
         const int nt = L.dim * (L.dim + 1) / 2 + L.dim;
         if (form == ABL_FV_FORM_FP64) {
-            s->fna.upload(L.fna);
-            s->fdx.upload(L.fdx);
+            s->fna.upload(face_array(L.fna, 0, 4));
+            s->fdx.upload(face_array(L.fdx, 4, 2 * L.dim));
             abl::SlotGeometry<double> sg;
-            abl::build_slot_geometry<double>(L, abl::slot_width(L.K), lim, sg);
+            abl::build_slot_geometry<double>(L, abl::slot_width(L.K), lim, !s->slot_rows, sg);
+            s->stab.upload(slots.table);
             s->snbr.upload(sg.nbr);
             s->sw.upload(sg.w);
             s->swa.upload(sg.wa);
@@ -3823,10 +3939,11 @@ extern "C" int abl_fv_create(const abl_fv_mesh_desc* mesh, const abl_fv_physics_
             }
         } else {
             auto to_f = [](const std::vector<double>& v) { return std::vector<float>(v.begin(), v.end()); };
-            s->fna_f.upload(to_f(L.fna));
-            s->fdx_f.upload(to_f(L.fdx));
+            s->fna_f.upload(to_f(face_array(L.fna, 0, 4)));
+            s->fdx_f.upload(to_f(face_array(L.fdx, 4, 2 * L.dim)));
             abl::SlotGeometry<float> sg;
-            abl::build_slot_geometry<float>(L, abl::slot_width(L.K), lim, sg);
+            abl::build_slot_geometry<float>(L, abl::slot_width(L.K), lim, !s->slot_rows, sg);
+            s->stab_f.upload(slots_f.table);
             s->snbr.upload(sg.nbr);
             s->sw_f.upload(sg.w);
             s->swa_f.upload(sg.wa);
@@ -3842,13 +3959,13 @@ extern "C" int abl_fv_create(const abl_fv_mesh_desc* mesh, const abl_fv_physics_
             }
             const bool rus_m = p.flux_calculator == ABL_FV_FLUX_RUSANOV;
             if (mesh->dim == 3) {
-                s->grad_kernel_f = abl::pick_gradients<float, 3>(s->recon, s->visc, lim, L.K);
+                s->grad_kernel_f = abl::pick_gradients<float, 3>(s->recon, s->visc, lim, L.K, s->slot_rows);
                 s->flux_kernel_mixed = abl::pick_flux_mixed<3>(s->recon, s->visc, rus_m);
                 s->tile_kernel_mixed = abl::pick_tile_mixed<3>(s->recon, s->visc, species, L.K, rus_m);
                 s->face_flux_kernel_mixed = abl::pick_face_flux_mixed<3>(s->recon, s->visc, species, rus_m);
                 s->gather_kernel_mixed = abl::pick_gather_mixed<3>(L.K);
             } else {
-                s->grad_kernel_f = abl::pick_gradients<float, 2>(s->recon, s->visc, lim, L.K);
+                s->grad_kernel_f = abl::pick_gradients<float, 2>(s->recon, s->visc, lim, L.K, s->slot_rows);
                 s->flux_kernel_mixed = abl::pick_flux_mixed<2>(s->recon, s->visc, rus_m);
                 s->tile_kernel_mixed = abl::pick_tile_mixed<2>(s->recon, s->visc, species, L.K, rus_m);
                 s->face_flux_kernel_mixed = abl::pick_face_flux_mixed<2>(s->recon, s->visc, species, rus_m);
@@ -3944,7 +4061,7 @@ extern "C" int abl_fv_create(const abl_fv_mesh_desc* mesh, const abl_fv_physics_
             s->dt_partial.alloc((size_t)2 * std::max<int64_t>(grid_for(L.NI), 1));
             s->cfl_out.alloc(3);
         }
-        s->build_tiles(L);
+        s->build_tiles(L, face_rows);
         s->build_fused(L);
         s->build_march(L);
         s->strategy = s->auto_strategy();
@@ -4191,7 +4308,10 @@ extern "C" int abl_fv_set_tile_size(abl_fv_handle h, int32_t cells) {
         lay.fcell.resize(h->fcell.n);
         HIP_CHECK(hipMemcpy(lay.ell.data(), h->ell.ptr, h->ell.bytes(), hipMemcpyDeviceToHost));
         HIP_CHECK(hipMemcpy(lay.fcell.data(), h->fcell.ptr, h->fcell.bytes(), hipMemcpyDeviceToHost));
-        if (!h->build_tiles(lay, cells))
+        std::vector<uint16_t> face_rows(h->frow.n);
+        if (h->frow.n)
+            HIP_CHECK(hipMemcpy(face_rows.data(), h->frow.ptr, h->frow.bytes(), hipMemcpyDeviceToHost));
+        if (!h->build_tiles(lay, face_rows, cells))
             return fail(h, "abl_fv_set_tile_size: the tile's face fluxes exceed the workgroup LDS");
     } catch (const std::exception& e) {
         return fail(h, std::string("abl_fv_set_tile_size: ") + e.what());
