@@ -6,6 +6,7 @@
 
 #include <cfloat>
 #include <cstdint>
+#include <type_traits>
 
 namespace abl {
 
@@ -36,6 +37,18 @@ constexpr double kSuthMu0 = 1.716e-5, kSuthT0 = 273.0, kSuthS = 111.0, kSuthPr =
 __device__ __host__ inline double sutherland_mu(double T) {
     const double r = T / kSuthT0;
     return kSuthMu0 * sqrt(r) * r * (kSuthT0 + kSuthS) / (T + kSuthS);
+}
+
+// Marks values as used here: the compiler computes them no later than this point (no instruction is emitted).  With
+// __builtin_amdgcn_sched_barrier it bounds how far an unrolled loop's loads and sums may drift apart.
+template <typename T>
+__device__ inline void pin(T& x) {
+    if constexpr (std::is_array_v<T>) {
+#pragma unroll
+        for (auto& y : x) pin(y);
+    } else {
+        asm volatile("" : "+v"(x));
+    }
 }
 
 // Geometry view (G = storage type of the face geometry: double for FP64, float for the mixed form).

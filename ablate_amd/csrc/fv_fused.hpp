@@ -359,7 +359,7 @@ __global__ __launch_bounds__(256) void k_fused(MeshView<double> m, Phys ph, cons
         fused_side<DIM, RECON, VISC>(rec, T, hal, nem, lc, x[0], sl);
         if (rc == kFusedGhost) {
             const int64_t Rc = m.fcell[F + f];
-            load_side<DIM, RECON, VISC>(U, nullptr, N, Rc, true, x[1], sr);
+            ghost_side<DIM, VISC>(U, N, Rc, sr);
             if (VISC) {
                 double w[2][DIM];
                 load_face_pair<DIM>(m.fwa, f, w);
@@ -476,7 +476,7 @@ __device__ inline void march_face(const MeshView<double>& m, const Phys& ph, con
     march_side<DIM, RECON, VISC>(ra, rb, T, hal, nem, lc, x[0], sl);
     if (rc == kFusedGhost) {
         const int64_t Rc = m.fcell[m.F + f];
-        load_side<DIM, RECON, VISC>(U, nullptr, m.N, Rc, true, x[1], sr);
+        ghost_side<DIM, VISC>(U, m.N, Rc, sr);
         if (VISC) {
             double w[2][DIM];
             load_face_pair<DIM>(m.fwa, f, w);

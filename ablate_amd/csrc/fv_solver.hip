@@ -23,6 +23,7 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "fv_adjoint.hpp"
@@ -179,23 +180,29 @@ __device__ inline void load_rec_f(const float* __restrict__ rec, int64_t c, RecF
 // G is the storage/arithmetic type of weights and gradients (double: FP64 form, float: mixed form); state
 // differences are always taken in FP64 before rounding to G.  Each lane writes its cell's record: CellRec (FP64
 // form) or CellRecF (mixed form), word by word into the 64-cell blocks.
-// TAB: the slot geometry comes from the table of distinct rows (see MeshView).
-template <typename G, int DIM, bool RECON, bool VISC, int LIM, int KM, bool TAB>
+// TAB: the slot geometry comes from the table of distinct rows (see MeshView).  GHOSTS: some neighbours may be ghost
+// cells (left out of the cell gradient; the aux set then has its own weights).
+// The body holds no divergent branch: padding slots take the cell itself as neighbour and zero weights, and every
+// condition is a select, so that the loads of several slots are in flight at once.  With a branch per slot the
+// compiler waited for each slot's loads before it issued the next one's, six dependent rounds of memory latency.
+// Measured (branch per slot -> this form): 256^3 hexes, Navier-Stokes FP64, Barth-Jespersen 2.06 -> 1.50 ms (152
+// VGPRs); 96 x 90 x 77 hexes, van Leer 94 -> 71 us (146 VGPRs); 200 x 161 x 150 hexes, mixed 357 -> 316 us.
+template <typename G, int DIM, bool RECON, bool VISC, int LIM, int KM, bool TAB, bool GHOSTS>
 __device__ __forceinline__ void gradients_body(MeshView<G> m, Phys ph, const double* __restrict__ U,
                                                G* __restrict__ gradC, G* __restrict__ gradA, void* __restrict__ rec) {
     constexpr int NE = DIM + 2;
     constexpr int NA = DIM + 1;
-    const int64_t c_lane = xcd_cell_index();
-    const bool active = c_lane < m.NI;
-    const int64_t c = active ? c_lane : m.NI - 1;  // lanes past the end shadow the last cell and store nothing
+    const int64_t c = xcd_cell_index();
+    if (c >= m.NI) return;
     const int64_t N = m.N, NI = m.NI;
     const G* __restrict__ wa_arr = m.swa ? m.swa : m.sw;
-    // meshes without boundary faces share one weight set
-    const bool own_wa = TAB ? m.saux != 0 : m.swa != nullptr;
-    const G* __restrict__ row[KM];  // table rows of the slots
-    if (TAB)
+    int32_t nb[KM];
+    uint32_t row[KM];  // word offsets of the slots' table rows
 #pragma unroll
-        for (int k = 0; k < KM; k++) row[k] = m.stab + (uint32_t)m.srow[k * NI + c] * (uint32_t)m.sstride;
+    for (int k = 0; k < KM; k++) {
+        nb[k] = m.snbr[k * NI + c];
+        row[k] = TAB ? (uint32_t)m.srow[k * NI + c] * (uint32_t)m.sstride : 0u;
+    }
     double uc[NE], ac[NA];
 #pragma unroll
     for (int p = 0; p < NE; p++) uc[p] = U[p * N + c];
@@ -216,68 +223,89 @@ __device__ __forceinline__ void gradients_body(MeshView<G> m, Phys ph, const dou
 #pragma unroll
         for (int d = 0; d < DIM; d++) ga[q][d] = G(0);
 
+    // Two slots in flight: the loads of slot k + 1 are issued before slot k is used.  The pinned sums and scheduling
+    // barriers keep the compiler from loading every slot before it uses the first (290 VGPRs in FP64).
+    double un[2][NE];
+    G w[2][DIM], wa[2][DIM];
+    auto load = [&](int k) {
+        const int64_t n = nb[k] >= 0 ? (int64_t)nb[k] : c;
+        const int b = k & 1;
 #pragma unroll
-    for (int k = 0; k < KM; k++) {
-        const int32_t e = m.snbr[k * NI + c];
-        const bool valid = e >= 0;
-        const int64_t n = valid ? (int64_t)e : c;
-        const bool bnd = n >= NI;
-        double un[NE];
-#pragma unroll
-        for (int p = 0; p < NE; p++) un[p] = U[p * N + n];
-        G w[DIM], wa[DIM];
+        for (int p = 0; p < NE; p++) un[b][p] = U[p * N + n];
         if (TAB) {
-            if (RECON) load_row_words<0, DIM>(row[k], w);
+            if (RECON || !GHOSTS) load_row_words<0, DIM>(m.stab + row[k], w[b]);
+            if (VISC && GHOSTS) load_row_words<0, DIM>(m.stab + row[k] + m.saux, wa[b]);
         } else {
 #pragma unroll
-            for (int d = 0; d < DIM; d++)
-                if (RECON) w[d] = m.sw[(k * DIM + d) * NI + c];
-        }
-        if (VISC) {
-            if (RECON && !own_wa) {  // the aux set is the cell set: reuse the words just loaded
-#pragma unroll
-                for (int d = 0; d < DIM; d++) wa[d] = w[d];
-            } else if (TAB) {
-                load_row_words<0, DIM>(row[k] + m.saux, wa);
-            } else {
-#pragma unroll
-                for (int d = 0; d < DIM; d++) wa[d] = wa_arr[(k * DIM + d) * NI + c];
+            for (int d = 0; d < DIM; d++) {
+                if (RECON || !GHOSTS) w[b][d] = m.sw[(k * DIM + d) * NI + c];
+                if (VISC && GHOSTS) wa[b][d] = wa_arr[(k * DIM + d) * NI + c];
             }
         }
-        if (!valid) continue;
+    };
+    load(0);
+#pragma unroll
+    for (int k = 0; k < KM; k++) {
+        const int b = k & 1;
+        if (k + 1 < KM) load(k + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        const bool valid = nb[k] >= 0;
+        const bool inner = !GHOSTS || nb[k] < NI;
         if (RECON) {
 #pragma unroll
             for (int p = 0; p < NE; p++) {
-                const G delta = G(un[p] - uc[p]);
+                const G delta = valid ? G(un[b][p] - uc[p]) : G(0);
                 if (LIM == kLimBJ) {
                     dmin[p] = fmin(dmin[p], delta);
                     dmax[p] = fmax(dmax[p], delta);
                 }
                 // cellInterpolant.cpp:405-411 with delta = u_R - u_L: the left cell adds w0.delta and the right cell
                 // subtracts w1.delta, i.e. both add w.(u_n - u_c) with their own side's weight (bitwise the same)
-                if (!bnd)
+                const G dg = inner ? delta : G(0);
 #pragma unroll
-                    for (int d = 0; d < DIM; d++) g[p][d] += w[d] * delta;
+                for (int d = 0; d < DIM; d++) g[p][d] += w[b][d] * dg;
             }
         }
         if (VISC) {
             double an[NA];
-            aux_of<DIM>(un, ph, an);
+            aux_of<DIM>(un[b], ph, an);
 #pragma unroll
             for (int q = 0; q < NA; q++) {
-                const G delta = G(an[q] - ac[q]);
+                const G delta = valid ? G(an[q] - ac[q]) : G(0);
+                // without boundary faces the aux set is the cell set
 #pragma unroll
-                for (int d = 0; d < DIM; d++) ga[q][d] += wa[d] * delta;
+                for (int d = 0; d < DIM; d++) ga[q][d] += (GHOSTS ? wa[b][d] : w[b][d]) * delta;
             }
         }
+        if (RECON) pin(g);
+        if (RECON && LIM == kLimBJ) {
+            pin(dmin);
+            pin(dmax);
+        }
+        if (VISC) pin(ga);
+        __builtin_amdgcn_sched_barrier(0);
     }
 
+    G tq[ViscTerms<DIM>::NT];
+    if (VISC) {
+        stress_heat<G, DIM>(G(ph.mu), G(ph.k), ga, tq);
+        pin(tq);
+    }
     if (RECON && LIM != kLimNone) {
         G phi[NE];
+        // limiter geometry of slot k (zero in padding slots)
+        auto limiter_vec = [&](int k, G* x) {
+            if (TAB)
+                load_row_words<DIM, DIM>(m.stab + row[k], x);
+            else
+#pragma unroll
+                for (int d = 0; d < DIM; d++) x[d] = m.slim[(k * DIM + d) * NI + c];
+        };
         if (LIM == kLimBJ) {
             // phi = min(1, (u_max - u_c)/max_f D_f+, (u_min - u_c)/min_f D_f-), D_f = grad.(x_f - x_c): the per-face
             // minimum collapsed onto the extreme projections (division is monotone).
-            G dpos[NE], dneg[NE];
+            G dpos[NE], dneg[NE], x[2][DIM];
+            limiter_vec(0, x[0]);
 #pragma unroll
             for (int p = 0; p < NE; p++) {
                 dpos[p] = G(0);
@@ -285,72 +313,90 @@ __device__ __forceinline__ void gradients_body(MeshView<G> m, Phys ph, const dou
             }
 #pragma unroll
             for (int k = 0; k < KM; k++) {
-                const bool valid = m.snbr[k * NI + c] >= 0;
-                G x[DIM];
-                if (TAB)
-                    load_row_words<DIM, DIM>(row[k], x);
-                else
-#pragma unroll
-                    for (int d = 0; d < DIM; d++) x[d] = m.slim[(k * DIM + d) * NI + c];
-                if (!valid) continue;
+                if (k + 1 < KM) limiter_vec(k + 1, x[(k + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int p = 0; p < NE; p++) {
                     G D = G(0);
 #pragma unroll
-                    for (int d = 0; d < DIM; d++) D += g[p][d] * x[d];
+                    for (int d = 0; d < DIM; d++) D += g[p][d] * x[k & 1][d];
                     dpos[p] = fmax(dpos[p], D);
                     dneg[p] = fmin(dneg[p], D);
                 }
+                pin(dpos);
+                pin(dneg);
+                __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
             for (int p = 0; p < NE; p++) {
+                const G up = dmax[p] / dpos[p], dn = dmin[p] / dneg[p];
                 G v = G(1);
-                if (dpos[p] > G(0)) v = fmin(v, dmax[p] / dpos[p]);
-                if (dneg[p] < G(0)) v = fmin(v, dmin[p] / dneg[p]);
+                v = dpos[p] > G(0) ? fmin(v, up) : v;
+                v = dneg[p] < G(0) ? fmin(v, dn) : v;
                 phi[p] = v;
+                pin(phi[p]);
+                __builtin_amdgcn_sched_barrier(0);
             }
         } else {
             // DMPlexApplyLimiter_Internal (cellInterpolant.cpp:282-328): f = 1/2 (u_n - u_c) / (grad.(x_n - x_c))
 #pragma unroll
             for (int p = 0; p < NE; p++) phi[p] = sizeof(G) == 8 ? G(DBL_MAX) : G(FLT_MAX);
+            auto load_lim = [&](int k) {  // neighbour state and x_n - x_c
+                pin(nb[k]);               // (addresses formed again, not kept from the first loop)
+                const int64_t n = nb[k] >= 0 ? (int64_t)nb[k] : c;
 #pragma unroll
-            for (int k = 0; k < KM; k++) {
-                const int32_t e = m.snbr[k * NI + c];
-                const int64_t n = e >= 0 ? (int64_t)e : c;
-                G v[DIM];  // x_n - x_c
-                if (TAB)
-                    load_row_words<DIM, DIM>(row[k], v);
-                else
+                for (int p = 0; p < NE; p++) un[k & 1][p] = U[p * N + n];
+                limiter_vec(k, w[k & 1]);
+            };
+            auto limit = [&](auto type) {  // the limiter function is fixed outside the slot loop
+                load_lim(0);
 #pragma unroll
-                    for (int d = 0; d < DIM; d++) v[d] = m.slim[(k * DIM + d) * NI + c];
-                if (e < 0) continue;
+                for (int k = 0; k < KM; k++) {
+                    if (k + 1 < KM) load_lim(k + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    const int b = k & 1;
 #pragma unroll
-                for (int p = 0; p < NE; p++) {
-                    G denom = G(0);
+                    for (int p = 0; p < NE; p++) {
+                        G denom = G(0);
 #pragma unroll
-                    for (int d = 0; d < DIM; d++) denom += g[p][d] * v[d];
-                    const G flim = G(0.5) * G(U[p * N + n] - uc[p]) / denom;
-                    phi[p] = pmin(phi[p], limiter_phi<G>(ph.limiter, flim));
+                        for (int d = 0; d < DIM; d++) denom += g[p][d] * w[b][d];
+                        const G flim = G(0.5) * G(un[b][p] - uc[p]) / denom;
+                        const G l = pmin(phi[p], limiter_phi<G>(decltype(type)::value, flim));
+                        phi[p] = nb[k] >= 0 ? l : phi[p];
+                        pin(phi[p]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
                 }
+            };
+            switch (ph.limiter) {
+                case ABL_FV_LIMITER_ZERO: limit(std::integral_constant<int, 1>()); break;
+                case ABL_FV_LIMITER_MINMOD: limit(std::integral_constant<int, 2>()); break;
+                case ABL_FV_LIMITER_VANLEER: limit(std::integral_constant<int, 3>()); break;
+                case ABL_FV_LIMITER_VANALBADA: limit(std::integral_constant<int, 4>()); break;
+                case ABL_FV_LIMITER_SUPERBEE: limit(std::integral_constant<int, 5>()); break;
+                case ABL_FV_LIMITER_MC: limit(std::integral_constant<int, 6>()); break;
+                default: limit(std::integral_constant<int, 7>()); break;
             }
         }
         bool cancel = false;
 #pragma unroll
-        for (int p = 0; p < NE; p++)
-            if (phi[p] == G(0))
+        for (int p = 0; p < NE; p++) {
+            bool large = false;
 #pragma unroll
-                for (int d = 0; d < DIM; d++)
-                    if (double(fabs(g[p][d])) > ph.max_lim_grad) cancel = true;
+            for (int d = 0; d < DIM; d++) large |= double(fabs(g[p][d])) > ph.max_lim_grad;
+            cancel |= (phi[p] == G(0)) & large;
+        }
 #pragma unroll
-        for (int p = 0; p < NE; p++)
+        for (int p = 0; p < NE; p++) {
+            const G f = cancel ? G(0) : phi[p];
 #pragma unroll
-            for (int d = 0; d < DIM; d++) g[p][d] *= cancel ? G(0) : phi[p];
+            for (int d = 0; d < DIM; d++) g[p][d] *= f;
+        }
     }
-    G tq[ViscTerms<DIM>::NT];
-    if (VISC) stress_heat<G, DIM>(G(ph.mu), G(ph.k), ga, tq);
     if (sizeof(G) == 8) {
         using CR = CellRec<DIM>;
-        if (active) {
+        {
             double w[CR::RS];
 #pragma unroll
             for (int p = 0; p < NE; p++) {
@@ -362,7 +408,7 @@ __device__ __forceinline__ void gradients_body(MeshView<G> m, Phys ph, const dou
             for (int q = 0; q < ViscTerms<DIM>::NT; q++) w[CR::T0 + q] = VISC ? double(tq[q]) : 0.0;
 #pragma unroll
             for (int i = CR::END; i < CR::RS; i++) w[i] = 0.0;
-            double2* __restrict__ r = reinterpret_cast<double2*>(rec) + rec_pair<DIM>(c_lane);
+            double2* __restrict__ r = reinterpret_cast<double2*>(rec) + rec_pair<DIM>(c);
 #pragma unroll
             for (int q = 0; q < CR::NP; q++) r[CR::BLOCK * q] = make_double2(w[2 * q], w[2 * q + 1]);
         }
@@ -380,7 +426,7 @@ __device__ __forceinline__ void gradients_body(MeshView<G> m, Phys ph, const dou
 #pragma unroll
         for (int q = 0; q < ViscTerms<DIM>::NT; q++)
             if (VISC) t[CR::TF + q] = float(tq[q]);
-        if (active) {
+        {
             uint64_t wd[2 * CR::NP];
 #pragma unroll
             for (int i = 0; i < CR::U0 / 2; i++)
@@ -389,26 +435,25 @@ __device__ __forceinline__ void gradients_body(MeshView<G> m, Phys ph, const dou
             for (int p = 0; p < NE; p++) wd[CR::U0 / 2 + p] = (uint64_t)__double_as_longlong(uc[p]);
 #pragma unroll
             for (int i = CR::RSW; i < 2 * CR::NP; i++) wd[i] = 0;
-            ulonglong2* __restrict__ w = reinterpret_cast<ulonglong2*>(rec) + recf_pair<DIM>(c_lane);
+            ulonglong2* __restrict__ w = reinterpret_cast<ulonglong2*>(rec) + recf_pair<DIM>(c);
 #pragma unroll
             for (int q = 0; q < CR::NP; q++) w[64 * q] = make_ulonglong2(wd[2 * q], wd[2 * q + 1]);
         }
     }
 }
 
-template <typename G, int DIM, bool RECON, bool VISC, int LIM, int KM, bool TAB = false>
+template <typename G, int DIM, bool RECON, bool VISC, int LIM, int KM, bool TAB, bool GHOSTS>
 __global__ __launch_bounds__(kBlock) void k_gradients(MeshView<G> m, Phys ph, const double* __restrict__ U,
                                                       G* __restrict__ gradC, G* __restrict__ gradA,
                                                       void* __restrict__ rec) {
-    gradients_body<G, DIM, RECON, VISC, LIM, KM, TAB>(m, ph, U, gradC, gradA, rec);
+    gradients_body<G, DIM, RECON, VISC, LIM, KM, TAB, GHOSTS>(m, ph, U, gradC, gradA, rec);
 }
-// The same kernel held to 128 VGPRs (four waves per SIMD instead of three: more loads in flight).  Picked for the
-// FP64 3-D forms without the PETSc-family limiter, which fit without spilling (that limiter's would spill).
-template <typename G, int DIM, bool RECON, bool VISC, int LIM, int KM, bool TAB = false>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_gradients_w4(
+// The same kernel held to three waves per SIMD (168 VGPRs), for the FP64 3-D forms.
+template <typename G, int DIM, bool RECON, bool VISC, int LIM, int KM, bool TAB, bool GHOSTS>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_gradients_w3(
     MeshView<G> m, Phys ph, const double* __restrict__ U, G* __restrict__ gradC, G* __restrict__ gradA,
     void* __restrict__ rec) {
-    gradients_body<G, DIM, RECON, VISC, LIM, KM, TAB>(m, ph, U, gradC, gradA, rec);
+    gradients_body<G, DIM, RECON, VISC, LIM, KM, TAB, GHOSTS>(m, ph, U, gradC, gradA, rec);
 }
 
 // densityYi gradients (limited, one field) into gS [ns*DIM][N] and Yi aux gradients (unlimited) into gY [ns*DIM][N];
@@ -588,17 +633,18 @@ __device__ inline void side_cell_values(const double* u, SideData<DIM, VISC>& sd
 }
 
 // Loads side data of cell c for a face whose centroid is at x_c + dx: from the cell record when the gradient pass
-// ran (reconstruction or diffusion), else from the state.  Ghost cells have zero gradients and read the state;
-// their viscous terms are filled by ghost_visc.  (Each branch keeps its own arrays so that they stay in
-// registers.)
+// ran (reconstruction or diffusion), else from the state.  A ghost cell has no record: its face takes `c` = the
+// interior cell here (a valid address) and ghost_side afterwards.  Both sides' loads thereby stand in one
+// straight line and are in flight together; with the choice between record and state around the loads, the right
+// side's were issued only when the left side's had arrived.
 template <int DIM, bool RECON, bool VISC>
 __device__ inline void load_side(const double* __restrict__ U, const double* __restrict__ rec, int64_t N, int64_t c,
-                                 bool ghost, const double* dx, SideData<DIM, VISC>& sd) {
+                                 const double* dx, SideData<DIM, VISC>& sd) {
     using CR = CellRec<DIM>;
     constexpr int NE = DIM + 2;
-    if ((RECON || VISC) && !ghost) {
-        constexpr int NL = VISC ? CR::END : CR::T0;
-        double r[2 * ((NL + 1) / 2)];
+    constexpr int NL = VISC ? CR::END : (RECON ? CR::T0 : NE);
+    double r[2 * ((NL + 1) / 2)];
+    if constexpr (RECON || VISC) {
         const double2* __restrict__ rb = reinterpret_cast<const double2*>(rec) + rec_pair<DIM>(c);
 #pragma unroll
         for (int q = 0; q < (NL + 1) / 2; q++) {
@@ -608,30 +654,37 @@ __device__ inline void load_side(const double* __restrict__ U, const double* __r
             r[2 * q] = v.x;
             r[2 * q + 1] = v.y;
         }
-#pragma unroll
-        for (int p2 = 0; p2 < NE; p2++) {
-            double a = 0.0;
-            if (RECON)
-#pragma unroll
-                for (int d = 0; d < DIM; d++) a += r[CR::G0 + p2 * DIM + d] * dx[d];
-            sd.uf[p2] = r[p2] + a;
-        }
-        if (VISC)
-#pragma unroll
-            for (int q = 0; q < ViscTerms<DIM>::NT; q++) sd.tq[q] = r[CR::T0 + q];
-        side_cell_values<DIM, VISC>(r, sd);
     } else {
-        double u[NE];
 #pragma unroll
-        for (int p2 = 0; p2 < NE; p2++) {
-            u[p2] = U[p2 * N + c];
-            sd.uf[p2] = u[p2];
-        }
-        if (VISC)
-#pragma unroll
-            for (int q = 0; q < ViscTerms<DIM>::NT; q++) sd.tq[q] = 0.0;
-        side_cell_values<DIM, VISC>(u, sd);
+        for (int p2 = 0; p2 < NE; p2++) r[p2] = U[p2 * N + c];
     }
+#pragma unroll
+    for (int p2 = 0; p2 < NE; p2++) {
+        double a = 0.0;
+        if (RECON)
+#pragma unroll
+            for (int d = 0; d < DIM; d++) a += r[CR::G0 + p2 * DIM + d] * dx[d];
+        sd.uf[p2] = RECON ? r[p2] + a : r[p2];
+    }
+    if (VISC)
+#pragma unroll
+        for (int q = 0; q < ViscTerms<DIM>::NT; q++) sd.tq[q] = r[CR::T0 + q];
+    side_cell_values<DIM, VISC>(r, sd);
+}
+// Side data of ghost cell c: zero gradients, the state from U; its viscous terms are filled by ghost_visc.
+template <int DIM, bool VISC>
+__device__ inline void ghost_side(const double* __restrict__ U, int64_t N, int64_t c, SideData<DIM, VISC>& sd) {
+    constexpr int NE = DIM + 2;
+    double u[NE];
+#pragma unroll
+    for (int p2 = 0; p2 < NE; p2++) {
+        u[p2] = U[p2 * N + c];
+        sd.uf[p2] = u[p2];
+    }
+    if (VISC)
+#pragma unroll
+        for (int q = 0; q < ViscTerms<DIM>::NT; q++) sd.tq[q] = 0.0;
+    side_cell_values<DIM, VISC>(u, sd);
 }
 
 // Viscous terms of a ghost cell: its one-neighbour least-squares gradient w (a_interior - a_ghost)
@@ -647,6 +700,25 @@ __device__ inline void ghost_visc(const Phys& ph, const double* w, const SideDat
         for (int q = 0; q < DIM; q++) gA[1 + q][d] = w[d] * (in.vel[q] - gh.vel[q]);
     }
     stress_heat<double, DIM>(ph.mu, ph.k, gA, gh.tq);
+}
+
+// Both sides of face f (left cell L, right cell Rc, which may be a ghost); w receives the boundary face's aux weights.
+template <int DIM, bool RECON, bool VISC>
+__device__ inline void load_sides(const MeshView<double>& m, const Phys& ph, const double* __restrict__ U,
+                                  const double* __restrict__ rec, int64_t f, int64_t L, int64_t Rc,
+                                  const double (*x)[DIM], double (*w)[DIM], SideData<DIM, VISC>& sl,
+                                  SideData<DIM, VISC>& sr) {
+    constexpr bool USE_REC = RECON || VISC;  // (a first-order inviscid face reads the ghost's state row itself)
+    const bool ghost = Rc >= m.NI;
+    load_side<DIM, RECON, VISC>(U, rec, m.N, L, x[0], sl);
+    load_side<DIM, RECON, VISC>(U, rec, m.N, USE_REC && ghost ? L : Rc, x[1], sr);
+    if (USE_REC && ghost) {
+        ghost_side<DIM, VISC>(U, m.N, Rc, sr);
+        if (VISC) {
+            load_face_pair<DIM>(m.fwa, f, w);
+            ghost_visc<DIM, VISC>(ph, w[1], sl, sr);
+        }
+    }
 }
 
 // The flux through one face oriented left -> right (ComputeFluxSourceTerms + the continuous face loop,
@@ -765,7 +837,6 @@ __global__ __launch_bounds__(kBlock) void k_flux(MeshView<double> m, Phys ph, co
     const int64_t c = xcd_cell_index();
     if (c >= m.NI) return;
     const int64_t N = m.N, F = m.F, NI = m.NI;
-    const double* __restrict__ wa_arr = m.fwa;  // present whenever ghosts meet diffusion
     double acc[NE];
 #pragma unroll
     for (int p = 0; p < NE; p++) acc[p] = 0.0;
@@ -775,18 +846,12 @@ __global__ __launch_bounds__(kBlock) void k_flux(MeshView<double> m, Phys ph, co
         const int64_t f = e >> 1;
         const int s = e & 1;
         const int64_t L = m.fcell[f], Rc = m.fcell[F + f], g = geometry_row(m, f);
-        const bool ghost = Rc >= NI;  // a ghost is always the right cell
         double nh[3], area, x[2][DIM];
         load_face_na(m.fna, g, nh, area);
         load_face_pair<DIM>(m.fdx, g, x);
         SD sl, sr;
-        load_side<DIM, RECON, VISC>(U, rec, N, L, false, x[0], sl);
-        load_side<DIM, RECON, VISC>(U, rec, N, Rc, ghost, x[1], sr);
-        if (VISC && ghost) {
-            double w[2][DIM];
-            load_face_pair<DIM>(wa_arr, f, w);
-            ghost_visc<DIM, VISC>(ph, w[1], sl, sr);
-        }
+        double w[2][DIM];
+        load_sides<DIM, RECON, VISC>(m, ph, U, rec, f, L, Rc, x, w, sl, sr);
         double flux[NE], cl, cr, cd;
         face_flux<DIM, VISC>(ph, nh, area, sl, sr, flux, cl, cr, cd);
         const double sign = s == 0 ? -1.0 : 1.0;
@@ -814,11 +879,8 @@ __global__ __launch_bounds__(kBlock) void k_flux(MeshView<double> m, Phys ph, co
             double nh[3], area, x[2][DIM], w[2][DIM];
             load_face_na(m.fna, g, nh, area);
             load_face_pair<DIM>(m.fdx, g, x);
-            if (VISC && ghost) load_face_pair<DIM>(wa_arr, f, w);
             SD sl, sr;
-            load_side<DIM, RECON, VISC>(U, rec, N, L, false, x[0], sl);
-            load_side<DIM, RECON, VISC>(U, rec, N, Rc, ghost, x[1], sr);
-            if (VISC && ghost) ghost_visc<DIM, VISC>(ph, w[1], sl, sr);
+            load_sides<DIM, RECON, VISC>(m, ph, U, rec, f, L, Rc, x, w, sl, sr);
             double flux[NE], cl, cr, cd;
             face_flux<DIM, VISC>(ph, nh, area, sl, sr, flux, cl, cr, cd);
             const double fs = species_face_flux<DIM, RECON, VISC>(m, U, gradC, gradA, comp, sp, f, L, Rc, ghost, x, nh,
@@ -841,18 +903,13 @@ __device__ inline void eval_face(const MeshView<double>& m, const Phys& ph, cons
                                  const double* __restrict__ rec, const FaceRef& fr, double* fe, double* fs,
                                  int64_t fs_stride) {
     using SD = SideData<DIM, VISC>;
-    const int64_t N = m.N, NI = m.NI, f = fr.f, L = fr.L, Rc = fr.R;
-    const bool ghost = Rc >= NI;
+    const int64_t f = fr.f, L = fr.L, Rc = fr.R;
+    const bool ghost = Rc >= m.NI;
     double nh[3], area, x[2][DIM], w[2][DIM];
     load_face_na(m.fna, fr.g, nh, area);
     load_face_pair<DIM>(m.fdx, fr.g, x);
     SD sl, sr;
-    load_side<DIM, RECON, VISC>(U, rec, N, L, false, x[0], sl);
-    load_side<DIM, RECON, VISC>(U, rec, N, Rc, ghost, x[1], sr);
-    if (VISC && ghost) {
-        load_face_pair<DIM>(m.fwa, f, w);
-        ghost_visc<DIM, VISC>(ph, w[1], sl, sr);
-    }
+    load_sides<DIM, RECON, VISC>(m, ph, U, rec, f, L, Rc, x, w, sl, sr);
     double cl, cr, cd;
     face_flux<DIM, VISC>(ph, nh, area, sl, sr, fe, cl, cr, cd);
     if (!SPECIES) return;
@@ -956,7 +1013,7 @@ __global__ __launch_bounds__(kTileMax) void k_tile_flux(MeshView<double> m, Phys
         double acc = 0.0;
 #pragma unroll
         for (int k = 0; k < KM; k++)
-            if (sg[k] != 0.0) acc += sg[k] * le[p * nfm + li[k]];
+            acc += sg[k] * (sg[k] != 0.0 ? le[p * nfm + li[k]] : 0.0);
         const double r = acc * iv;
         R[p * N + c] = accumulate ? R[p * N + c] + r : r;
     }
@@ -965,7 +1022,7 @@ __global__ __launch_bounds__(kTileMax) void k_tile_flux(MeshView<double> m, Phys
         double a = 0.0;
 #pragma unroll
         for (int k = 0; k < KM; k++)
-            if (sg[k] != 0.0) a += sg[k] * ls[sp * nfm + li[k]];
+            a += sg[k] * (sg[k] != 0.0 ? ls[sp * nfm + li[k]] : 0.0);
         const int64_t comp = NE + sp;
         const double r = a * iv;
         R[comp * N + c] = accumulate ? R[comp * N + c] + r : r;
@@ -1006,7 +1063,7 @@ __global__ __launch_bounds__(kBlock) void k_gather(MeshView<double> m, int ns, c
         acc[p] = 0.0;
 #pragma unroll
         for (int k = 0; k < KM; k++)
-            if (sg[k] != 0.0) acc[p] += sg[k] * v[k][p];
+            acc[p] += sg[k] * (sg[k] != 0.0 ? v[k][p] : 0.0);
     }
     const double iv = m.inv_vol[c];
 #pragma unroll
@@ -1022,10 +1079,8 @@ __global__ __launch_bounds__(kBlock) void k_gather(MeshView<double> m, int ns, c
 #pragma unroll
         for (int k = 0; k < KM; k++) {
             const double2 fv = Fs2[(int64_t)q * F + fk[k]];
-            if (sg[k] != 0.0) {
-                a0 += sg[k] * fv.x;
-                a1 += sg[k] * fv.y;
-            }
+            a0 += sg[k] * (sg[k] != 0.0 ? fv.x : 0.0);
+            a1 += sg[k] * (sg[k] != 0.0 ? fv.y : 0.0);
         }
         for (int h = 0; h < 2 && 2 * q + h < ns; h++) {
             const int sp = 2 * q + h;
@@ -1152,8 +1207,11 @@ __device__ inline void mixed_face(const MeshView<float>& m, const Phys& ph, cons
 #pragma unroll
         for (int p = 0; p < NE; p++) rl.u[p] = U[p * N + L];
     }
-    if (USE_REC && !ghost) {
-        load_rec_f<DIM, RECON, VISC>(rec, Rc, rr);
+    if (USE_REC) {  // a ghost has no record: the left cell's stands in, so that both loads are in flight together
+        load_rec_f<DIM, RECON, VISC>(rec, ghost ? L : Rc, rr);
+        if (ghost)
+#pragma unroll
+            for (int p = 0; p < NE; p++) rr.u[p] = U[p * N + Rc];
     } else {
 #pragma unroll
         for (int p = 0; p < NE; p++) rr.u[p] = U[p * N + Rc];
@@ -1525,7 +1583,7 @@ __global__ __launch_bounds__(kTileMax) void k_tile_flux_mixed(MeshView<float> m,
         double acc = 0.0;
 #pragma unroll
         for (int k = 0; k < KM; k++)
-            if (sg[k] != 0.0) acc += sg[k] * double(lf[p * nfm + off[k]]);
+            acc += sg[k] * (sg[k] != 0.0 ? double(lf[p * nfm + off[k]]) : 0.0);
         const double r = acc * iv;
         R[p * N + c] = accumulate ? R[p * N + c] + r : r;
     }
@@ -1574,7 +1632,7 @@ __global__ __launch_bounds__(kBlock) void k_gather_mixed(MeshView<float> m, int 
         double acc = 0.0;
 #pragma unroll
         for (int k = 0; k < KM; k++)
-            if (sg[k] != 0.0) acc += sg[k] * double(Fm[p * m.F + off[k]]);
+            acc += sg[k] * (sg[k] != 0.0 ? double(Fm[p * m.F + off[k]]) : 0.0);
         const double r = acc * iv;
         R[p * N + c] = accumulate ? R[p * N + c] + r : r;
     }
@@ -2853,25 +2911,21 @@ using FaceFluxKernel = void (*)(MeshView<double>, Phys, const double*, const dou
                                 double*, double*);
 using GatherKernel = void (*)(MeshView<double>, int, const double*, const double*, double*, int);
 
-template <typename G, int DIM, int KM, bool TAB>
+template <typename G, int DIM, int KM, bool TAB, bool GHOSTS>
 GradKernelT<G> pick_gradients_k(bool recon, bool visc, int lim) {
-    if (!recon) return visc ? k_gradients<G, DIM, false, true, kLimNone, KM, TAB> : nullptr;
-    if constexpr (sizeof(G) == 8 && DIM == 3) {
-        if (lim != kLimPetsc) {
-            if (visc) return lim == kLimBJ ? k_gradients_w4<G, DIM, true, true, kLimBJ, KM, TAB>
-                                           : k_gradients_w4<G, DIM, true, true, kLimNone, KM, TAB>;
-            return lim == kLimBJ ? k_gradients_w4<G, DIM, true, false, kLimBJ, KM, TAB>
-                                 : k_gradients_w4<G, DIM, true, false, kLimNone, KM, TAB>;
-        }
-    }
-    if (visc) {
-        if (lim == kLimBJ) return k_gradients<G, DIM, true, true, kLimBJ, KM, TAB>;
-        if (lim == kLimPetsc) return k_gradients<G, DIM, true, true, kLimPetsc, KM, TAB>;
-        return k_gradients<G, DIM, true, true, kLimNone, KM, TAB>;
-    }
-    if (lim == kLimBJ) return k_gradients<G, DIM, true, false, kLimBJ, KM, TAB>;
-    if (lim == kLimPetsc) return k_gradients<G, DIM, true, false, kLimPetsc, KM, TAB>;
-    return k_gradients<G, DIM, true, false, kLimNone, KM, TAB>;
+    if (!recon) return visc ? k_gradients<G, DIM, false, true, kLimNone, KM, TAB, GHOSTS> : nullptr;
+    auto pick = [&](auto limiter) -> GradKernelT<G> {
+        constexpr int LIM = decltype(limiter)::value;
+        if constexpr (sizeof(G) == 8 && DIM == 3)
+            return visc ? k_gradients_w3<G, DIM, true, true, LIM, KM, TAB, GHOSTS>
+                        : k_gradients_w3<G, DIM, true, false, LIM, KM, TAB, GHOSTS>;
+        else
+            return visc ? k_gradients<G, DIM, true, true, LIM, KM, TAB, GHOSTS>
+                        : k_gradients<G, DIM, true, false, LIM, KM, TAB, GHOSTS>;
+    };
+    if (lim == kLimBJ) return pick(std::integral_constant<int, kLimBJ>());
+    if (lim == kLimPetsc) return pick(std::integral_constant<int, kLimPetsc>());
+    return pick(std::integral_constant<int, kLimNone>());
 }
 // Compile-time slot width of the cell -> face table: 4 (quads, tets), 6 (hexes) or 8.
 inline int slot_width(int K) { return K <= 4 ? 4 : (K <= 6 ? 6 : 8); }
@@ -2885,12 +2939,15 @@ void pick_adj(bool rusanov, int K, AdjFacesKernel& fk, AdjCellsKernel& ce, AdjCe
     }
 }
 template <typename G, int DIM>
-GradKernelT<G> pick_gradients(bool recon, bool visc, int lim, int K, bool tab) {
-    if (tab) return pick_gradients_k<G, DIM, DIM == 2 ? 4 : 6, true>(recon, visc, lim);
-    switch (slot_width(K)) {
-        case 4: return pick_gradients_k<G, DIM, 4, false>(recon, visc, lim);
-        case 6: return pick_gradients_k<G, DIM, 6, false>(recon, visc, lim);
-        default: return pick_gradients_k<G, DIM, 8, false>(recon, visc, lim);
+GradKernelT<G> pick_gradients(bool recon, bool visc, int lim, int K, bool tab, bool ghosts) {
+    constexpr int KT = DIM == 2 ? 4 : 6;  // slot width of the shapes with slot tables (kSlotRows)
+    if (tab) return ghosts ? pick_gradients_k<G, DIM, KT, true, true>(recon, visc, lim)
+                           : pick_gradients_k<G, DIM, KT, true, false>(recon, visc, lim);
+    if (slot_width(K) == KT && !ghosts) return pick_gradients_k<G, DIM, KT, false, false>(recon, visc, lim);
+    switch (slot_width(K)) {  // without ghosts these read the one weight set for both gradients
+        case 4: return pick_gradients_k<G, DIM, 4, false, true>(recon, visc, lim);
+        case 6: return pick_gradients_k<G, DIM, 6, false, true>(recon, visc, lim);
+        default: return pick_gradients_k<G, DIM, 8, false, true>(recon, visc, lim);
     }
 }
 
@@ -3894,7 +3951,7 @@ extern "C" int abl_fv_create(const abl_fv_mesh_desc* mesh, const abl_fv_physics_
         if (mesh->dim == 3) {
             s->species_kernel = abl::pick_species_gradients<double, 3>(L.K);
             s->species_kernel_f = abl::pick_species_gradients<float, 3>(L.K);
-            s->grad_kernel = abl::pick_gradients<double, 3>(s->recon, s->visc, lim, L.K, s->slot_rows);
+            s->grad_kernel = abl::pick_gradients<double, 3>(s->recon, s->visc, lim, L.K, s->slot_rows, L.has_boundary);
             s->flux_kernel = abl::pick_flux<3>(s->recon, s->visc, species);
             s->face_flux_kernel = abl::pick_face_flux<3>(s->recon, s->visc, species);
             s->tile_kernel = abl::pick_tile<3>(s->recon, s->visc, species, L.K);
@@ -3904,7 +3961,7 @@ extern "C" int abl_fv_create(const abl_fv_mesh_desc* mesh, const abl_fv_physics_
         } else {
             s->species_kernel = abl::pick_species_gradients<double, 2>(L.K);
             s->species_kernel_f = abl::pick_species_gradients<float, 2>(L.K);
-            s->grad_kernel = abl::pick_gradients<double, 2>(s->recon, s->visc, lim, L.K, s->slot_rows);
+            s->grad_kernel = abl::pick_gradients<double, 2>(s->recon, s->visc, lim, L.K, s->slot_rows, L.has_boundary);
             s->flux_kernel = abl::pick_flux<2>(s->recon, s->visc, species);
             s->face_flux_kernel = abl::pick_face_flux<2>(s->recon, s->visc, species);
             s->tile_kernel = abl::pick_tile<2>(s->recon, s->visc, species, L.K);
@@ -3959,13 +4016,13 @@ extern "C" int abl_fv_create(const abl_fv_mesh_desc* mesh, const abl_fv_physics_
             }
             const bool rus_m = p.flux_calculator == ABL_FV_FLUX_RUSANOV;
             if (mesh->dim == 3) {
-                s->grad_kernel_f = abl::pick_gradients<float, 3>(s->recon, s->visc, lim, L.K, s->slot_rows);
+                s->grad_kernel_f = abl::pick_gradients<float, 3>(s->recon, s->visc, lim, L.K, s->slot_rows, L.has_boundary);
                 s->flux_kernel_mixed = abl::pick_flux_mixed<3>(s->recon, s->visc, rus_m);
                 s->tile_kernel_mixed = abl::pick_tile_mixed<3>(s->recon, s->visc, species, L.K, rus_m);
                 s->face_flux_kernel_mixed = abl::pick_face_flux_mixed<3>(s->recon, s->visc, species, rus_m);
                 s->gather_kernel_mixed = abl::pick_gather_mixed<3>(L.K);
             } else {
-                s->grad_kernel_f = abl::pick_gradients<float, 2>(s->recon, s->visc, lim, L.K, s->slot_rows);
+                s->grad_kernel_f = abl::pick_gradients<float, 2>(s->recon, s->visc, lim, L.K, s->slot_rows, L.has_boundary);
                 s->flux_kernel_mixed = abl::pick_flux_mixed<2>(s->recon, s->visc, rus_m);
                 s->tile_kernel_mixed = abl::pick_tile_mixed<2>(s->recon, s->visc, species, L.K, rus_m);
                 s->face_flux_kernel_mixed = abl::pick_face_flux_mixed<2>(s->recon, s->visc, species, rus_m);

@@ -96,8 +96,8 @@ def stream_probe(gib, reps=10):
     return out
 
 
-KERNELS = {"face_flux": ["k_gradients_w4", "k_face_flux", "k_gather"], "recompute": ["k_gradients_w4", "k_flux"],
-           "tile": ["k_gradients_w4", "k_tile_flux"], "fused": ["k_fused"], "march": ["k_march"]}
+KERNELS = {"face_flux": ["k_gradients_w3", "k_face_flux", "k_gather"], "recompute": ["k_gradients_w3", "k_flux"],
+           "tile": ["k_gradients_w3", "k_tile_flux"], "fused": ["k_fused"], "march": ["k_march"]}
 
 
 def recorded_traffic(workload, n, strategy):
