@@ -49,23 +49,29 @@ constexpr int kCuLdsBytes = 160 * 1024;  // LDS of one gfx950 compute unit
 
 // ============================================================================================ kernels
 
-__global__ __launch_bounds__(kBlock) void k_ghost_fill(int64_t nb, const int32_t* __restrict__ bface,
-                                                       const int32_t* __restrict__ bslot, const int32_t* __restrict__ fcell,
-                                                       int64_t F, int64_t N, int nc, const int32_t* __restrict__ slot_kind,
-                                                       const double* __restrict__ slot_state, double* __restrict__ U) {
+// Ghost rows of the state, and (Z not null) zeros in the ghost rows of the result, which every ghost cell's one
+// boundary face covers.  One lane per boundary face and component (blockIdx.y), the cells straight from bcell: two
+// dependent loads deep.  A lane per face that walked the components took 22 us for 62208 faces of 15 components (each
+// store to U may alias the next component's load), and the zeros were a launch of their own.
+__global__ __launch_bounds__(kBlock) void k_ghost_fill(int64_t nb, const int2* __restrict__ bcell,
+                                                       const int32_t* __restrict__ bslot, int64_t N, int nc,
+                                                       const int32_t* __restrict__ slot_kind,
+                                                       const double* __restrict__ slot_state, double* __restrict__ U,
+                                                       double* __restrict__ Z) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nb) return;
-    const int32_t f = bface[i], s = bslot[i];
-    const int32_t interior = fcell[f], ghost = fcell[F + f];
+    const int p = blockIdx.y;
+    const int2 cells = bcell[i];  // interior, ghost
+    const int32_t s = bslot[i];
     const int kind = slot_kind[s];
+    const double ui = U[(int64_t)p * N + cells.x], state = slot_state[s * nc + p];
+    const int64_t g = (int64_t)p * N + cells.y;
+    if (Z) Z[g] = 0.0;
     if (kind == ABL_FV_BC_GHOST) return;  // caller-filled: the ghost rows are inputs
-    for (int p = 0; p < nc; p++) {
-        const double ui = U[(int64_t)p * N + interior];
-        double v = ui;  // OUTFLOW: zero-gradient extrapolation
-        if (kind == ABL_FV_BC_INFLOW) v = slot_state[s * nc + p];
-        if (kind == kBcInflowAtFace) v = 2.0 * slot_state[s * nc + p] - ui;  // essentialGhost.cpp:17-20
-        U[(int64_t)p * N + ghost] = v;
-    }
+    double v = ui;  // OUTFLOW: zero-gradient extrapolation
+    if (kind == ABL_FV_BC_INFLOW) v = state;
+    if (kind == kBcInflowAtFace) v = 2.0 * state - ui;  // essentialGhost.cpp:17-20
+    U[g] = v;
 }
 
 // Aux values of a cell: temperature (PerfectGas TemperatureFunction, perfectGas.cpp:76-86) and velocity.
@@ -977,7 +983,7 @@ __global__ __launch_bounds__(kTileMax) void k_tile_flux(MeshView<double> m, Phys
                                                         const double* __restrict__ rec,
                                                         const int32_t* __restrict__ tstart,
                                                         const int4* __restrict__ tfaces,
-                                                        const int32_t* __restrict__ tslot, int nfm,
+                                                        const int32_t* __restrict__ tslot, int T, int nfm,
                                                         double* __restrict__ R, int accumulate) {
     constexpr int NE = DIM + 2;
     extern __shared__ double lds[];
@@ -985,7 +991,14 @@ __global__ __launch_bounds__(kTileMax) void k_tile_flux(MeshView<double> m, Phys
     double* ls = lds + NE * nfm;   // [ns][nfm]
     const int64_t t = xcd_block_index();
     const int32_t f0 = tstart[t], nf = tstart[t + 1] - f0;
-    // a lane's next face entry is loaded one round ahead
+    // the gather's tables are loaded before the faces, a lane's next face entry one round ahead
+    const int64_t c = t * T + threadIdx.x;
+    const int64_t N = m.N, NI = m.NI;
+    const int64_t ca = (int)threadIdx.x < T && c < NI ? c : t * T;
+    int32_t es[KM];
+#pragma unroll
+    for (int k = 0; k < KM; k++) es[k] = tslot[k * NI + ca];
+    const double iv = m.inv_vol[ca];
     int4 fnext = (int)threadIdx.x < nf ? tfaces[f0 + threadIdx.x] : make_int4(0, 0, 0, 0);
     for (int i = threadIdx.x; i < nf; i += blockDim.x) {
         double flux[NE];
@@ -996,36 +1009,36 @@ __global__ __launch_bounds__(kTileMax) void k_tile_flux(MeshView<double> m, Phys
         for (int p = 0; p < NE; p++) le[p * nfm + i] = flux[p];
     }
     __syncthreads();
-    const int64_t c = t * blockDim.x + threadIdx.x;
-    if (c >= m.NI) return;
-    const int64_t N = m.N, NI = m.NI;
+    if ((int)threadIdx.x >= T || c >= NI) return;
     int li[KM];
     double sg[KM];
 #pragma unroll
     for (int k = 0; k < KM; k++) {
-        const int32_t e = tslot[k * NI + c];
-        li[k] = e >= 0 ? (e >> 1) : 0;
-        sg[k] = e < 0 ? 0.0 : ((e & 1) ? 1.0 : -1.0);
+        li[k] = es[k] >= 0 ? (es[k] >> 1) : 0;
+        sg[k] = es[k] < 0 ? 0.0 : ((es[k] & 1) ? 1.0 : -1.0);
     }
-    const double iv = m.inv_vol[c];
+    // sum over the slots of one row of face fluxes; every slot is read, padding slots are dropped by select
+    auto gather = [&](const double* row) {
+        double v[KM], acc = 0.0;
 #pragma unroll
-    for (int p = 0; p < NE; p++) {
-        double acc = 0.0;
+        for (int k = 0; k < KM; k++) v[k] = row[li[k]];
 #pragma unroll
-        for (int k = 0; k < KM; k++)
-            acc += sg[k] * (sg[k] != 0.0 ? le[p * nfm + li[k]] : 0.0);
-        const double r = acc * iv;
-        R[p * N + c] = accumulate ? R[p * N + c] + r : r;
-    }
+        for (int k = 0; k < KM; k++) acc += sg[k] * (sg[k] != 0.0 ? v[k] : 0.0);
+        return acc * iv;
+    };
+    double r[NE];
+#pragma unroll
+    for (int p = 0; p < NE; p++) r[p] = gather(le + p * nfm);
+    if (accumulate)
+#pragma unroll
+        for (int p = 0; p < NE; p++) r[p] = R[p * N + c] + r[p];
+#pragma unroll
+    for (int p = 0; p < NE; p++) R[p * N + c] = r[p];
     if (!SPECIES) return;
     for (int sp = 0; sp < ph.ns; sp++) {
-        double a = 0.0;
-#pragma unroll
-        for (int k = 0; k < KM; k++)
-            a += sg[k] * (sg[k] != 0.0 ? ls[sp * nfm + li[k]] : 0.0);
+        const double a = gather(ls + sp * nfm);
         const int64_t comp = NE + sp;
-        const double r = a * iv;
-        R[comp * N + c] = accumulate ? R[comp * N + c] + r : r;
+        R[comp * N + c] = accumulate ? R[comp * N + c] + a : a;
     }
 }
 
@@ -1548,7 +1561,7 @@ __global__ __launch_bounds__(kTileMax) void k_tile_flux_mixed(MeshView<float> m,
                                                               const float* __restrict__ gY,
                                                               const int32_t* __restrict__ tstart,
                                                               const int4* __restrict__ tfaces,
-                                                              const int32_t* __restrict__ tslot, int nfm,
+                                                              const int32_t* __restrict__ tslot, int T, int nfm,
                                                               double* __restrict__ R, int accumulate) {
     constexpr int NE = DIM + 2;
     extern __shared__ double lds_d[];
@@ -1556,6 +1569,14 @@ __global__ __launch_bounds__(kTileMax) void k_tile_flux_mixed(MeshView<float> m,
     const int nrow = NE + (SPECIES ? ph.ns : 0);
     const int64_t t = xcd_block_index();
     const int32_t f0 = tstart[t], nf = tstart[t + 1] - f0;
+    // the gather's tables are loaded before the faces
+    const int64_t c = t * T + threadIdx.x;
+    const int64_t N = m.N, NI = m.NI;
+    const int64_t ca = (int)threadIdx.x < T && c < NI ? c : t * T;
+    int32_t es[KM];
+#pragma unroll
+    for (int k = 0; k < KM; k++) es[k] = tslot[k * NI + ca];
+    const double iv = m.inv_vol[ca];
     for (int i = threadIdx.x; i < nf; i += blockDim.x) {
         float dFL[NE], dFR[NE];
         mixed_face<DIM, RECON, VISC, SPECIES, RUS>(m, ph, U, rec, gS, gY, tile_face_ref(tfaces[f0 + i]), dFL, dFR,
@@ -1567,23 +1588,21 @@ __global__ __launch_bounds__(kTileMax) void k_tile_flux_mixed(MeshView<float> m,
         }
     }
     __syncthreads();
-    const int64_t c = t * blockDim.x + threadIdx.x;
-    if (c >= m.NI) return;
-    const int64_t N = m.N, NI = m.NI;
+    if ((int)threadIdx.x >= T || c >= NI) return;
     int off[KM];
     double sg[KM];
 #pragma unroll
     for (int k = 0; k < KM; k++) {
-        const int32_t e = tslot[k * NI + c];
-        off[k] = e >= 0 ? ((e & 1) ? nrow * nfm : 0) + (e >> 1) : 0;
-        sg[k] = e < 0 ? 0.0 : ((e & 1) ? 1.0 : -1.0);
+        off[k] = es[k] >= 0 ? ((es[k] & 1) ? nrow * nfm : 0) + (es[k] >> 1) : 0;
+        sg[k] = es[k] < 0 ? 0.0 : ((es[k] & 1) ? 1.0 : -1.0);
     }
-    const double iv = m.inv_vol[c];
     for (int p = 0; p < nrow; p++) {
+        float v[KM];
         double acc = 0.0;
 #pragma unroll
-        for (int k = 0; k < KM; k++)
-            acc += sg[k] * (sg[k] != 0.0 ? double(lf[p * nfm + off[k]]) : 0.0);
+        for (int k = 0; k < KM; k++) v[k] = lf[p * nfm + off[k]];
+#pragma unroll
+        for (int k = 0; k < KM; k++) acc += sg[k] * (sg[k] != 0.0 ? double(v[k]) : 0.0);
         const double r = acc * iv;
         R[p * N + c] = accumulate ? R[p * N + c] + r : r;
     }
@@ -2980,7 +2999,7 @@ MixedFluxKernel pick_flux_mixed(bool recon, bool visc, bool rus) {
     return rus ? pick_flux_mixed2<DIM, true>(recon, visc) : pick_flux_mixed2<DIM, false>(recon, visc);
 }
 using TileMixedKernel = void (*)(MeshView<float>, Phys, const double*, const float*, const float*, const float*,
-                                 const int32_t*, const int4*, const int32_t*, int, double*, int);
+                                 const int32_t*, const int4*, const int32_t*, int, int, double*, int);
 template <int DIM, bool RECON, bool VISC, bool SPECIES, bool RUS>
 TileMixedKernel pick_tile_mixed3(int K) {
     switch (slot_width(K)) {
@@ -3063,7 +3082,7 @@ VjpThetaKernel pick_vjp_theta(bool rusanov) {
     return rusanov ? k_vjp_theta<DIM, true> : k_vjp_theta<DIM, false>;
 }
 using TileKernel = void (*)(MeshView<double>, Phys, const double*, const double*, const double*, const double*,
-                           const int32_t*, const int4*, const int32_t*, int, double*, int);
+                           const int32_t*, const int4*, const int32_t*, int, int, double*, int);
 template <int DIM, bool RECON, bool VISC, int KM>
 TileKernel pick_tile3(bool species) {
     return species ? k_tile_flux<DIM, RECON, VISC, true, KM> : k_tile_flux<DIM, RECON, VISC, false, KM>;
@@ -3442,6 +3461,7 @@ struct abl_fv_solver {
     abl::Layout host;  // metadata only after upload (arrays released)
     abl::Phys ph{};
     abl::DevBuf<int32_t> ell, fcell, bface, bslot, slot_kind, snbr;
+    abl::DevBuf<int2> bcell;  // interior and ghost cell of every boundary face
     abl::DevBuf<double> fna, fdx, fwa, inv_vol, gradC, gradA, slot_state;
     abl::DevBuf<double> sw, swa, slim;  // slot-major gradient geometry (FP64 form)
     // distinct geometry rows (boxes): row numbers per face and slot; the tables are fna, fdx and stab
@@ -3458,7 +3478,7 @@ struct abl_fv_solver {
     abl::DevBuf<float> face_flux_m;
     abl::DevBuf<int32_t> tile_start, tile_slot;  // tile strategy (built when selected)
     abl::DevBuf<int4> tile_faces;                // TileFace entries
-    int tile_T = 0, tile_nfm = 0;
+    int tile_T = 0, tile_threads = 0, tile_nfm = 0;
     int64_t tile_n = 0;
     size_t tile_lds = 0;
     double tile_redundancy = 0.0;  // face evaluations of the tile kernel per face
@@ -3647,7 +3667,15 @@ struct abl_fv_solver {
                                                       : 2 * (lay.dim + 2 + lay.ns) * (int)sizeof(float);
         abl::Tiles tl;
         const size_t budget = only_T ? (size_t)abl::kTileLdsMax : (size_t)abl::kTileLdsDefault;
-        for (int T = only_T ? only_T : abl::kTileDefault; T >= 64; T /= 2) {
+        // Fewer than two default tiles per CU leave the chip part empty and one tile's rounds of faces a serial chain:
+        // small meshes take 64-cell tiles, and tiles of any size 256 lanes while there are at most four workgroups per
+        // CU (41 x 36 x 29 hexes, Navier-Stokes FP64: 16.3 us with 256-cell tiles, 13.3 us so; 96 x 90 x 77: 104.8 us
+        // with 256-cell tiles, 113.9 us with 64-cell tiles of 256 lanes).
+        int dev = 0, cus = 256;
+        HIP_CHECK(hipGetDevice(&dev));
+        HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        const int T0 = (lay.NI + abl::kTileDefault - 1) / abl::kTileDefault < 2 * cus ? 64 : abl::kTileDefault;
+        for (int T = only_T ? only_T : T0; T >= 64; T /= 2) {
             abl::build_tiles(lay, KM, T, tl);
             if ((size_t)tl.nf_max * per_face <= budget) break;
             tl.n = 0;
@@ -3670,6 +3698,7 @@ struct abl_fv_solver {
         tile_faces.upload(entries);
         tile_slot.upload(tl.slot);
         tile_T = tl.T;
+        tile_threads = tl.n <= 4 * (int64_t)cus ? std::max(tl.T, abl::kBlock) : tl.T;
         tile_n = tl.n;
         tile_nfm = tl.nf_max;
         tile_lds = (size_t)tl.nf_max * per_face;
@@ -3818,7 +3847,7 @@ struct abl_fv_solver {
         return ABL_FV_STRATEGY_FACE_FLUX;
     }
     int64_t device_bytes() const {
-        return (int64_t)(frow.bytes() + srow.bytes() + stab.bytes() + stab_f.bytes() + ell.bytes() + fcell.bytes() + bface.bytes() + bslot.bytes() + slot_kind.bytes() + fna.bytes() + fdx.bytes() + face_flux_e.bytes() + face_flux_s.bytes() + face_flux_m.bytes() + tile_start.bytes() + tile_faces.bytes() + tile_slot.bytes() + fu_start.bytes() + fu_faces.bytes() + fu_code.bytes() + fu_slot.bytes() + fu_hstart.bytes() + fu_hcell.bytes() + fu_hinfo.bytes() + mr_seq.bytes() + mr_pro.bytes() + mr_stile.bytes() + mr_snext.bytes() + mr_fstart.bytes() + mr_ffaces.bytes() + mr_fcode.bytes() + mr_pfstart.bytes() + mr_pffaces.bytes() + mr_pfcode.bytes() + mr_hstart.bytes() + mr_hcell.bytes() + mr_hinfo.bytes() + mr_gslot.bytes() + snbr.bytes() + vjp_rows.bytes() + sw.bytes() + swa.bytes() + slim.bytes() + sw_f.bytes() + swa_f.bytes() + slim_f.bytes() + fwa.bytes() + inv_vol.bytes() + gradC.bytes() +
+        return (int64_t)(frow.bytes() + srow.bytes() + stab.bytes() + stab_f.bytes() + bcell.bytes() + ell.bytes() + fcell.bytes() + bface.bytes() + bslot.bytes() + slot_kind.bytes() + fna.bytes() + fdx.bytes() + face_flux_e.bytes() + face_flux_s.bytes() + face_flux_m.bytes() + tile_start.bytes() + tile_faces.bytes() + tile_slot.bytes() + fu_start.bytes() + fu_faces.bytes() + fu_code.bytes() + fu_slot.bytes() + fu_hstart.bytes() + fu_hcell.bytes() + fu_hinfo.bytes() + mr_seq.bytes() + mr_pro.bytes() + mr_stile.bytes() + mr_snext.bytes() + mr_fstart.bytes() + mr_ffaces.bytes() + mr_fcode.bytes() + mr_pfstart.bytes() + mr_pffaces.bytes() + mr_pfcode.bytes() + mr_hstart.bytes() + mr_hcell.bytes() + mr_hinfo.bytes() + mr_gslot.bytes() + snbr.bytes() + vjp_rows.bytes() + sw.bytes() + swa.bytes() + slim.bytes() + sw_f.bytes() + swa_f.bytes() + slim_f.bytes() + fwa.bytes() + inv_vol.bytes() + gradC.bytes() +
                          gradA.bytes() + rec.bytes() + adjUghost.bytes() + adjUself.bytes() + adjContrib.bytes() + adjW.bytes() + adjGL.bytes() + mirror.bytes() + recf.bytes() + gS_f.bytes() + gY_f.bytes() + rmin.bytes() + cfl_partial.bytes() + dt_partial.bytes() + cfl_out.bytes() + slot_state.bytes() + counter.bytes() + fna_f.bytes() + fdx_f.bytes() +
                          fwa_f.bytes());
     }
@@ -3846,6 +3875,13 @@ std::string unset_boundary(abl_fv_handle h) {
 
 // theta_bar is the adjoint of the inflow states: with no inflow slot every contribution is zero and the theta_bar
 // passes (and their copy back to the host) are skipped.
+// Ghost rows of U from the boundary conditions; zeros in the ghost rows of Z (null: none).
+void fill_ghosts(abl_fv_handle h, hipStream_t st, double* U, double* Z) {
+    const abl::Layout& L = h->host;
+    hipLaunchKernelGGL(abl::k_ghost_fill, dim3(grid_for(h->n_bfaces), (unsigned)L.nc), dim3(abl::kBlock), 0, st,
+                       h->n_bfaces, h->bcell.ptr, h->bslot.ptr, L.N, L.nc, h->slot_kind.ptr, h->slot_state.ptr, U, Z);
+}
+
 bool has_inflow(abl_fv_handle h) {
     for (int v : h->bc_slots)
         if (h->h_slot_kind[v] == ABL_FV_BC_INFLOW) return true;
@@ -4085,6 +4121,10 @@ extern "C" int abl_fv_create(const abl_fv_mesh_desc* mesh, const abl_fv_physics_
             }
         }
         s->bface.upload(bf);
+        std::vector<int2> bc(bf.size());
+        for (size_t i = 0; i < bf.size(); i++)
+            bc[i] = make_int2(L.fcell[(size_t)bf[i]], L.fcell[(size_t)(L.F + bf[i])]);
+        s->bcell.upload(bc);
         s->bslot.upload(bs);
         s->h_slot_kind.assign(abl::kMaxBcSlots, ABL_FV_BC_NONE);
         s->h_slot_at_face.assign(abl::kMaxBcSlots, 0);
@@ -4227,11 +4267,7 @@ extern "C" int abl_fv_rhs(abl_fv_handle h, double time, double* U, double* R, in
         hipStream_t st = (hipStream_t)stream;
         const abl::Layout& L = h->host;
         if (h->n_bfaces) {
-            h->timed(ABL_FV_PHASE_GHOST, st, [&] {
-                hipLaunchKernelGGL(abl::k_ghost_fill, dim3(grid_for(h->n_bfaces)), dim3(abl::kBlock), 0, st, h->n_bfaces,
-                                   h->bface.ptr, h->bslot.ptr, h->fcell.ptr, L.F, L.N, L.nc, h->slot_kind.ptr,
-                                   h->slot_state.ptr, U);
-            });
+            h->timed(ABL_FV_PHASE_GHOST, st, [&] { fill_ghosts(h, st, U, accumulate ? nullptr : R); });
         }
         const dim3 grid(grid_for(L.NI)), block(abl::kBlock);
         if (h->form == ABL_FV_FORM_MIXED) {
@@ -4258,9 +4294,9 @@ extern "C" int abl_fv_rhs(abl_fv_handle h, double time, double* U, double* R, in
                 });
             } else if (h->strategy == ABL_FV_STRATEGY_TILE) {
                 h->timed(ABL_FV_PHASE_FLUX, st, [&] {
-                    hipLaunchKernelGGL(h->tile_kernel_mixed, dim3((unsigned)h->tile_n), dim3(h->tile_T), h->tile_lds, st,
+                    hipLaunchKernelGGL(h->tile_kernel_mixed, dim3((unsigned)h->tile_n), dim3(h->tile_threads), h->tile_lds, st,
                                        vf, h->ph, U, h->recf.ptr, h->gS_f.ptr, h->gY_f.ptr, h->tile_start.ptr,
-                                       h->tile_faces.ptr, h->tile_slot.ptr, h->tile_nfm, R, accumulate);
+                                       h->tile_faces.ptr, h->tile_slot.ptr, h->tile_T, h->tile_nfm, R, accumulate);
                 });
             } else {
                 h->timed(ABL_FV_PHASE_FLUX, st, [&] {
@@ -4292,10 +4328,10 @@ extern "C" int abl_fv_rhs(abl_fv_handle h, double time, double* U, double* R, in
         }
         if (h->strategy == ABL_FV_STRATEGY_TILE) {
             h->timed(ABL_FV_PHASE_FLUX, st, [&] {
-                hipLaunchKernelGGL(h->tile_kernel, dim3((unsigned)h->tile_n), dim3(h->tile_T), h->tile_lds, st, v, h->ph,
+                hipLaunchKernelGGL(h->tile_kernel, dim3((unsigned)h->tile_n), dim3(h->tile_threads), h->tile_lds, st, v, h->ph,
                                    U, h->gradC.ptr, h->gradA.ptr, h->rec.ptr, h->tile_start.ptr,
                                    h->tile_faces.ptr,
-                                   h->tile_slot.ptr, h->tile_nfm, R, accumulate);
+                                   h->tile_slot.ptr, h->tile_T, h->tile_nfm, R, accumulate);
             });
         } else if (h->strategy == ABL_FV_STRATEGY_FACE_FLUX) {
             h->timed(ABL_FV_PHASE_FLUX, st, [&] {
@@ -4313,8 +4349,6 @@ extern "C" int abl_fv_rhs(abl_fv_handle h, double time, double* U, double* R, in
             });
         }
         }
-        if (!accumulate && L.N > L.NI)
-            hipLaunchKernelGGL(abl::k_zero_rows, dim3(grid_for((L.N - L.NI) * L.nc)), block, 0, st, R, L.N, L.NI, L.nc);
         HIP_CHECK(hipGetLastError());
     } catch (const std::exception& e) {
         return fail(h, std::string("abl_fv_rhs: ") + e.what());
@@ -4440,11 +4474,7 @@ int vjp_second_order(abl_fv_handle h, double* U, const double* Rbar, double* Uba
         }
         const dim3 grid(grid_for(L.NI)), block(abl::kBlock);
         if (h->n_bfaces)
-            h->timed(ABL_FV_PHASE_GHOST, st, [&] {
-                hipLaunchKernelGGL(abl::k_ghost_fill, dim3(grid_for(h->n_bfaces)), block, 0, st, h->n_bfaces,
-                                   h->bface.ptr, h->bslot.ptr, h->fcell.ptr, L.F, L.N, L.nc, h->slot_kind.ptr,
-                                   h->slot_state.ptr, U);
-            });
+            h->timed(ABL_FV_PHASE_GHOST, st, [&] { fill_ghosts(h, st, U, Ubar); });
         const auto v = h->view();
         h->timed(ABL_FV_PHASE_GRADIENTS, st, [&] {
             hipLaunchKernelGGL(h->grad_kernel, grid, block, 0, st, v, h->ph, U, h->gradC.ptr, h->gradA.ptr,
@@ -4465,7 +4495,6 @@ int vjp_second_order(abl_fv_handle h, double* U, const double* Rbar, double* Uba
                                Ubar);
         });
         if (NG > 0) {
-            hipLaunchKernelGGL(abl::k_zero_rows, dim3(grid_for(NG * L.nc)), block, 0, st, Ubar, L.N, L.NI, L.nc);
             hipLaunchKernelGGL(abl::k_ghost_adjoint_out, dim3(grid_for(NG)), block, 0, st, NG, L.N, L.NI, L.nc,
                                h->ghost_slot.ptr, h->slot_kind.ptr, h->adjUghost.ptr, Ubar);
         }
@@ -4531,11 +4560,8 @@ int vjp_first_order(abl_fv_handle h, double* U, const double* Rbar, double* Ubar
     const int fl = h->phys.flux_calculator;
     try {
         if (h->n_bfaces) {
-            h->timed(ABL_FV_PHASE_GHOST, st, [&] {
-                hipLaunchKernelGGL(abl::k_ghost_fill, dim3(grid_for(h->n_bfaces)), dim3(abl::kBlock), 0, st, h->n_bfaces,
-                                   h->bface.ptr, h->bslot.ptr, h->fcell.ptr, L.F, L.N, L.nc, h->slot_kind.ptr,
-                                   h->slot_state.ptr, U);
-            });
+            // the ghost rows of Ubar are zeroed first: the VJP kernel then writes those of caller-filled ghosts
+            h->timed(ABL_FV_PHASE_GHOST, st, [&] { fill_ghosts(h, st, U, Ubar); });
         }
         const dim3 grid(grid_for(L.NI)), block(abl::kBlock);
         const bool noflux = fl == ABL_FV_FLUX_OFF || fl == ABL_FV_FLUX_NONE;
@@ -4543,10 +4569,6 @@ int vjp_first_order(abl_fv_handle h, double* U, const double* Rbar, double* Ubar
             hipLaunchKernelGGL(abl::k_zero_rows, dim3(grid_for(L.N * L.nc)), block, 0, st, Ubar, L.N, (int64_t)0, L.nc);
         } else {
             const auto v = h->view();
-            // ghost rows first: the VJP kernel then writes those of caller-filled ghosts
-            if (L.N > L.NI)
-                hipLaunchKernelGGL(abl::k_zero_rows, dim3(grid_for((L.N - L.NI) * L.nc)), block, 0, st, Ubar, L.N, L.NI,
-                                   L.nc);
             h->timed(ABL_FV_PHASE_VJP, st, [&] {
                 if (rows) {
                     hipLaunchKernelGGL(h->vjp_faces, dim3(grid_for(L.F)), block, 0, st, v, h->ph, U, Rbar, rows);
