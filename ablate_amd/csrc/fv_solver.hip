@@ -118,6 +118,13 @@ __device__ inline double rec_word(const double* __restrict__ rec, int64_t c, int
     return rec[2 * (rec_pair<DIM>(c) + (int64_t)CellRec<DIM>::BLOCK * (i >> 1)) + (i & 1)];
 }
 
+// Face records (fluxes, adjoints) of np word pairs, in blocks of 64 consecutive faces: pair q of face f is the double2 at
+// face_pair(f, np) + 64 q.  A wave of consecutive faces stores each pair with one coalesced 1 KB access, and the gather
+// of a wave of consecutive cells, whose faces cluster, reads it from a few lines.  With one contiguous record per face
+// every load of the gather touched 64 lines and used 16 bytes of each (k_gather_coef at 128^3: 334 against 272 us).
+__device__ inline int64_t face_pair(int64_t f, int np) { return (f >> 6) * 64 * (int64_t)np + (f & 63); }
+inline int64_t face_pairs_total(int64_t F, int np) { return (F + 63) / 64 * 64 * np; }
+
 // FP64 species gradients: per species and cell 2 DIM words, [0, DIM) the limited densityYi gradient and
 // [DIM, 2 DIM) the Yi aux gradient, stored as DIM word pairs; pair j of species sp of cell c is the double2 at
 // (sp DIM + j) N + c.  Lanes of consecutive cells move each pair with one coalesced 16-byte access, and a face's
@@ -780,6 +787,12 @@ __device__ inline void face_flux(const Phys& ph, const double* nhat, double area
     }
 }
 
+// The advection flux of one species from both sides' face values, in one fixed order of operations: the strategies that
+// evaluate it per face and per cell agree bit for bit.
+__device__ inline double species_advection(double cl, double yL, double cr, double yR) {
+    return __builtin_fma(cl, yL, cr * yR);
+}
+
 // Species fluxes of one face (SpeciesTransport AdvectionFlux / DiffusionSpeciesFlux, speciesTransport.cpp:196-341)
 // from the coefficients of face_flux: sum over species of a per-species scalar expression.
 template <int DIM, bool RECON, bool VISC>
@@ -812,9 +825,9 @@ __device__ inline double species_face_flux(const MeshView<double>& m, const doub
             pl += vL[d] * x[0][d];
             if (!ghost) pr += vR[d] * x[1][d];
         }
-        flux = cl * (yL + pl) + cr * (yR + pr);
+        flux = species_advection(cl, yL + pl, cr, yR + pr);
     } else {
-        flux = cl * yL + cr * yR;
+        flux = species_advection(cl, yL, cr, yR);
     }
     if (VISC) {
         double dot = 0.0;
@@ -903,6 +916,10 @@ __global__ __launch_bounds__(kBlock) void k_flux(MeshView<double> m, Phys ph, co
 // Species flux sp goes to fs[sp * fs_stride], or with PAIRS to fs[(sp / 2) * fs_stride + sp % 2] (species pairs
 // interleaved: the face-flux strategy's rows, written and read by the gather two species per 16-byte access; fs
 // 16-byte aligned).
+// First-order inviscid species fluxes are cl rhoY_L + cr rhoY_R: with PAIRS their two coefficients (fe[NE], fe[NE + 1])
+// stand for all of them and the gather forms them from the cells (kCoefGather).
+template <bool RECON, bool VISC, bool SPECIES>
+constexpr bool kCoefGather = SPECIES && !RECON && !VISC;
 template <int DIM, bool RECON, bool VISC, bool SPECIES, bool PAIRS = false>
 __device__ inline void eval_face(const MeshView<double>& m, const Phys& ph, const double* __restrict__ U,
                                  const double* __restrict__ gradC, const double* __restrict__ gradA,
@@ -919,7 +936,10 @@ __device__ inline void eval_face(const MeshView<double>& m, const Phys& ph, cons
     double cl, cr, cd;
     face_flux<DIM, VISC>(ph, nh, area, sl, sr, fe, cl, cr, cd);
     if (!SPECIES) return;
-    if constexpr (PAIRS) {
+    if constexpr (PAIRS && kCoefGather<RECON, VISC, SPECIES>) {
+        fe[DIM + 2] = cl;
+        fe[DIM + 3] = cr;
+    } else if constexpr (PAIRS) {
         // two species per 16-byte store
         for (int q = 0; 2 * q < ph.ns; q++) {
             const int sp = 2 * q;
@@ -939,24 +959,23 @@ __device__ inline void eval_face(const MeshView<double>& m, const Phys& ph, cons
 }
 
 // Strategy 2 (face flux + gather), pass 1: one lane per face, flux evaluated once and stored: euler components as a
-// padded record [F][FS] (one contiguous read per face in the gather), species as interleaved pairs [ns/2][F][2]
-// (coalesced 16-byte stores; species inside the record would make every store of a wave touch 64 cache lines,
-// measured 2.5x slower).
+// records of FS words (face_pair blocks), species as interleaved pairs [ns/2][F][2].
 template <int DIM, bool RECON, bool VISC, bool SPECIES>
 __device__ __forceinline__ void face_flux_body(MeshView<double> m, Phys ph, const double* __restrict__ U,
                                                const double* __restrict__ gradC, const double* __restrict__ gradA,
                                                const double* __restrict__ rec, double* __restrict__ Fe,
                                                double* __restrict__ Fs) {
     constexpr int NE = DIM + 2;
-    constexpr int FS = (NE + 1) & ~1;
+    constexpr int NW = NE + (kCoefGather<RECON, VISC, SPECIES> ? 2 : 0);
+    constexpr int FS = (NW + 1) & ~1;
     const int64_t f = xcd_cell_index();
     if (f >= m.F) return;
     double flux[FS];
     eval_face<DIM, RECON, VISC, SPECIES, true>(m, ph, U, gradC, gradA, rec, face_ref(m, f), flux, Fs + 2 * f, 2 * m.F);
-    if (FS > NE) flux[FS - 1] = 0.0;
-    double2* out = reinterpret_cast<double2*>(Fe + FS * f);
+    if (FS > NW) flux[FS - 1] = 0.0;
+    double2* out = reinterpret_cast<double2*>(Fe) + face_pair(f, FS / 2);
 #pragma unroll
-    for (int i = 0; i < FS / 2; i++) out[i] = make_double2(flux[2 * i], flux[2 * i + 1]);
+    for (int i = 0; i < FS / 2; i++) out[64 * i] = make_double2(flux[2 * i], flux[2 * i + 1]);
 }
 template <int DIM, bool RECON, bool VISC, bool SPECIES>
 __global__ __launch_bounds__(kBlock) void k_face_flux(MeshView<double> m, Phys ph, const double* __restrict__ U,
@@ -1062,10 +1081,10 @@ __global__ __launch_bounds__(kBlock) void k_gather(MeshView<double> m, int ns, c
     double v[KM][FS];
 #pragma unroll
     for (int k = 0; k < KM; k++) {
-        const double2* rec = reinterpret_cast<const double2*>(Fe + FS * fk[k]);
+        const double2* rec = reinterpret_cast<const double2*>(Fe) + face_pair(fk[k], FS / 2);
 #pragma unroll
         for (int i = 0; i < FS / 2; i++) {
-            const double2 t = rec[i];
+            const double2 t = rec[64 * i];
             v[k][2 * i] = t.x;
             v[k][2 * i + 1] = t.y;
         }
@@ -1102,6 +1121,79 @@ __global__ __launch_bounds__(kBlock) void k_gather(MeshView<double> m, int ns, c
             const double r = a * iv;
             R[comp * N + c] = accumulate ? R[comp * N + c] + r : r;
         }
+    }
+}
+
+// The same for first-order inviscid species: the face records hold the two species coefficients after the euler fluxes,
+// and each cell forms its faces' species fluxes from its own and its neighbours' densities (k_gather's order and
+// values).  A face then moves 8 words instead of 6 + ns, written once and read twice: 128^3 hexes with ten species,
+// k_face_flux 333 -> 132 us, gather 295 -> 272 us.
+template <int DIM, int KM>
+__global__ __launch_bounds__(kBlock) void k_gather_coef(MeshView<double> m, int ns, const double* __restrict__ U,
+                                                        const double* __restrict__ Fe, double* __restrict__ R,
+                                                        int accumulate) {
+    constexpr int NE = DIM + 2;
+    constexpr int FS = (NE + 3) & ~1;
+    const int64_t c = xcd_cell_index();
+    if (c >= m.NI) return;
+    const int64_t N = m.N, NI = m.NI;
+    int32_t e[KM], nb[KM];
+#pragma unroll
+    for (int k = 0; k < KM; k++) {
+        e[k] = k < m.K ? m.ell[k * NI + c] : -1;
+        nb[k] = m.snbr[k * NI + c];
+    }
+    const double iv = m.inv_vol[c];
+    double acc[NE], al[KM], ar[KM];  // species coefficients of the left and the right density, signed for this cell
+#pragma unroll
+    for (int p = 0; p < NE; p++) acc[p] = 0.0;
+#pragma unroll
+    for (int k = 0; k < KM; k++) {
+        const bool valid = e[k] >= 0;
+        const double2* rec = reinterpret_cast<const double2*>(Fe) + face_pair(valid ? (int64_t)(e[k] >> 1) : 0, FS / 2);
+        double v[FS];
+#pragma unroll
+        for (int i = 0; i < FS / 2; i++) {
+            const double2 t = rec[64 * i];
+            v[2 * i] = t.x;
+            v[2 * i + 1] = t.y;
+        }
+        const double sg = !valid ? 0.0 : ((e[k] & 1) ? 1.0 : -1.0);
+#pragma unroll
+        for (int p = 0; p < NE; p++) acc[p] += sg * (valid ? v[p] : 0.0);
+        al[k] = sg * v[NE];
+        ar[k] = sg * v[NE + 1];
+    }
+#pragma unroll
+    for (int p = 0; p < NE; p++) acc[p] *= iv;
+    if (accumulate)
+#pragma unroll
+        for (int p = 0; p < NE; p++) acc[p] = R[p * N + c] + acc[p];
+#pragma unroll
+    for (int p = 0; p < NE; p++) R[p * N + c] = acc[p];
+    // species, the next one's densities in flight while one is summed
+    double yc, yn[KM];
+    auto load = [&](int sp) {
+        const int64_t row = (int64_t)(NE + sp) * N;
+        yc = U[row + c];
+#pragma unroll
+        for (int k = 0; k < KM; k++) yn[k] = U[row + (e[k] >= 0 ? (int64_t)nb[k] : c)];
+    };
+    load(0);
+    for (int sp = 0; sp < ns; sp++) {
+        const int64_t row = (int64_t)(NE + sp) * N;
+        double y0 = yc, y[KM], a = 0.0;
+#pragma unroll
+        for (int k = 0; k < KM; k++) y[k] = yn[k];
+        if (sp + 1 < ns) load(sp + 1);
+#pragma unroll
+        for (int k = 0; k < KM; k++) {
+            const bool right = e[k] & 1;  // the cell is the right one
+            const double f = species_advection(al[k], right ? y[k] : y0, ar[k], right ? y0 : y[k]);
+            a += e[k] >= 0 ? f : 0.0;
+        }
+        const double r = a * iv;
+        R[row + c] = accumulate ? R[row + c] + r : r;
     }
 }
 
@@ -1664,25 +1756,30 @@ __global__ __launch_bounds__(kBlock) void k_gather_mixed(MeshView<float> m, int 
 // every face contributes dF/dU_side^T g_f with g_f = Rbar_R / V_R - Rbar_L / V_L.  One lane per interior cell
 // recomputes the forward flux of each of its faces and keeps its own side's adjoint (deterministic gather).
 
+// Seed of one component of a face, Rbar_R / V_R - Rbar_L / V_L (a ghost right side: rbR = ivR = 0), in one fixed order of
+// operations: the kernels that form it per face and per cell agree bit for bit.
+__device__ inline double face_seed_of(double rbR, double ivR, double rbL, double ivL) {
+    return __builtin_fma(rbR, ivR, -(rbL * ivL));
+}
+
 // Adjoint seeds of face f: g[p] for euler components and the species sums QL = sum g_sp rhoY_L,
 // QR = sum g_sp rhoY_R, QdL = sum g_sp (rhoY_R - rhoY_L).
 template <int DIM, int UNR = 2>
 __device__ inline void face_seed(const MeshView<double>& m, const Phys& ph, const double* __restrict__ U,
                                  const double* __restrict__ Rb, int64_t L, int64_t Rc, bool ghost, double* fb,
-                                 double& QL, double& QR, double& QdL, double* gout = nullptr, int64_t gstride = 0) {
+                                 double& QL, double& QR, double& QdL) {
     constexpr int NE = DIM + 2;
     const int64_t N = m.N;
     const double ivL = m.inv_vol[L], ivR = ghost ? 0.0 : m.inv_vol[Rc];
 #pragma unroll
-    for (int p = 0; p < NE; p++) fb[p] = (ghost ? 0.0 : Rb[p * N + Rc] * ivR) - Rb[p * N + L] * ivL;
+    for (int p = 0; p < NE; p++) fb[p] = face_seed_of(ghost ? 0.0 : Rb[p * N + Rc], ivR, Rb[p * N + L], ivL);
     QL = 0.0;
     QR = 0.0;
     QdL = 0.0;
 #pragma unroll UNR
     for (int sp = 0; sp < ph.ns; sp++) {  // UNR species' loads in flight
         const int64_t comp = NE + sp;
-        const double g = (ghost ? 0.0 : Rb[comp * N + Rc] * ivR) - Rb[comp * N + L] * ivL;
-        if (gout) gout[sp * gstride] = g;
+        const double g = face_seed_of(ghost ? 0.0 : Rb[comp * N + Rc], ivR, Rb[comp * N + L], ivL);
         const double yl = U[comp * N + L], yr = U[comp * N + Rc];
         QL += g * yl;
         QR += g * yr;
@@ -1708,9 +1805,14 @@ __global__ __launch_bounds__(kBlock) void k_vjp(MeshView<double> m, Phys ph, con
     const int64_t c = xcd_cell_index();
     if (c >= m.NI) return;
     const int64_t N = m.N, F = m.F, NI = m.NI;
-    double ub[NE], coef[KM], cghost[KM];  // cghost: species multiplier of a caller-filled ghost across slot k
+    // cghost: species multiplier of a caller-filled ghost across slot k; ug: the ghost sides folded back into the cell,
+    // summed apart (k_vjp_gather's order)
+    double ub[NE], ug[NE], coef[KM], cghost[KM];
 #pragma unroll
-    for (int p = 0; p < NE; p++) ub[p] = 0.0;
+    for (int p = 0; p < NE; p++) {
+        ub[p] = 0.0;
+        ug[p] = 0.0;
+    }
 #pragma unroll
     for (int k = 0; k < KM; k++) {
         const Slot sl = face_slot(m, k, c);
@@ -1742,11 +1844,11 @@ __global__ __launch_bounds__(kBlock) void k_vjp(MeshView<double> m, Phys ph, con
             const int gk = slot_kind[ghost_slot[Rc - NI]];
             if (gk == ABL_FV_BC_OUTFLOW) {  // the ghost copies this cell's state: its adjoint flows back here
 #pragma unroll
-                for (int p = 0; p < NE; p++) ub[p] += ubR[p];
+                for (int p = 0; p < NE; p++) ug[p] += ubR[p];
                 cf += cR;
             } else if (gk == kBcInflowAtFace) {  // ghost = 2 state - this cell
 #pragma unroll
-                for (int p = 0; p < NE; p++) ub[p] -= ubR[p];
+                for (int p = 0; p < NE; p++) ug[p] -= ubR[p];
                 cf -= cR;
             } else if (gk == ABL_FV_BC_GHOST) {  // caller-filled ghost: its own adjoint row (one face per ghost)
 #pragma unroll
@@ -1757,7 +1859,7 @@ __global__ __launch_bounds__(kBlock) void k_vjp(MeshView<double> m, Phys ph, con
         coef[k] = cf;
     }
 #pragma unroll
-    for (int p = 0; p < NE; p++) Ub[p * N + c] = ub[p];
+    for (int p = 0; p < NE; p++) Ub[p * N + c] = ub[p] + ug[p];
     if (ph.ns == 0) return;
     // species: the faces' cells and inverse volumes are loaded once for all species
     int64_t sL[KM], sR[KM];
@@ -1778,7 +1880,7 @@ __global__ __launch_bounds__(kBlock) void k_vjp(MeshView<double> m, Phys ph, con
 #pragma unroll
         for (int k = 0; k < KM; k++) {
             const bool ghost = sR[k] >= NI;
-            const double g = (ghost ? 0.0 : Rb[comp * N + sR[k]] * ivR[k]) - Rb[comp * N + sL[k]] * ivL[k];
+            const double g = face_seed_of(ghost ? 0.0 : Rb[comp * N + sR[k]], ivR[k], Rb[comp * N + sL[k]], ivL[k]);
             a += coef[k] * g;
             if (cghost[k] != 0.0) Ub[comp * N + sR[k]] = cghost[k] * g;
         }
@@ -1787,15 +1889,20 @@ __global__ __launch_bounds__(kBlock) void k_vjp(MeshView<double> m, Phys ph, con
 }
 
 // First-order VJP, face-centric (abl_fv_rhs_vjp; k_vjp above stays the allocation-free form): one lane per face
-// reverses the face's flux once for both sides and stores the side adjoints, the species multipliers and the
-// species seeds as rows [2 NE + 2 + ns][F] (ubL, ubR, cL, cR, g per species): coalesced stores.  k_vjp_gather then
-// sums them per cell in slot order exactly as k_vjp sums its own evaluations, so both forms give the same Ubar bit
-// for bit; each face is reversed once instead of once per side, and the gather reads each face's species seeds
-// instead of both cells' Rbar rows.
+// reverses the face's flux once for both sides and stores a record of two halves, one per side: the side's euler adjoint
+// and its species multiplier (VjpRec).  k_vjp_gather sums each cell's halves in slot order and forms the species
+// seeds from its own and its neighbours' Rbar, exactly as k_vjp does, so both forms give the same Ubar bit for bit.
+// With the seeds stored as ns more words per face the two kernels took 624 + 387 us at 128^3 hexes with ten species,
+// so 449 + 290 us.
+template <int DIM>
+struct VjpRec {
+    static constexpr int SW = (DIM + 4) & ~1;  // words per side: NE adjoints, the multiplier, padding to a pair
+};
 template <int DIM, bool RUS>
-__global__ __launch_bounds__(kBlock) void k_vjp_faces(MeshView<double> m, Phys ph, const double* __restrict__ U,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_vjp_faces(MeshView<double> m, Phys ph, const double* __restrict__ U,
                                                       const double* __restrict__ Rb, double* __restrict__ fr) {
     constexpr int NE = DIM + 2;
+    constexpr int SW = VjpRec<DIM>::SW;
     const int64_t f = xcd_cell_index();
     if (f >= m.F) return;
     const int64_t N = m.N, F = m.F, NI = m.NI;
@@ -1808,86 +1915,131 @@ __global__ __launch_bounds__(kBlock) void k_vjp_faces(MeshView<double> m, Phys p
         uL[p] = U[p * N + L];
         uR[p] = U[p * N + Rc];
     }
-    face_seed<DIM, 5>(m, ph, U, Rb, L, Rc, ghost, fb, QL, QR, QdL, fr + (2 * NE + 2) * F + f, F);
-    double ubL[NE], ubR[NE], cL, cR;
+    face_seed<DIM, 5>(m, ph, U, Rb, L, Rc, ghost, fb, QL, QR, QdL);
+    double w[2][SW], cL, cR;
 #pragma unroll
-    for (int p = 0; p < NE; p++) {
-        ubL[p] = 0.0;
-        ubR[p] = 0.0;
+    for (int i = 0; i < SW; i++) {
+        w[0][i] = 0.0;
+        w[1][i] = 0.0;
     }
-    face_vjp<DIM, RUS>(uL, uR, QL, QR, QdL, nh, area, ph, fb, ubL, ubR, cL, cR);
+    face_vjp<DIM, RUS>(uL, uR, QL, QR, QdL, nh, area, ph, fb, w[0], w[1], cL, cR);
+    w[0][NE] = cL;
+    w[1][NE] = cR;
+    double2* __restrict__ out = reinterpret_cast<double2*>(fr) + face_pair(f, SW);
 #pragma unroll
-    for (int p = 0; p < NE; p++) {
-        fr[p * F + f] = ubL[p];
-        fr[(NE + p) * F + f] = ubR[p];
-    }
-    fr[2 * NE * F + f] = cL;
-    fr[(2 * NE + 1) * F + f] = cR;
+    for (int sd = 0; sd < 2; sd++)
+#pragma unroll
+        for (int i = 0; i < SW / 2; i++) out[64 * (sd * (SW / 2) + i)] = make_double2(w[sd][2 * i], w[sd][2 * i + 1]);
 }
 
-// Per-cell sums of the face rows of k_vjp_faces: its own side of each face in slot order, the ghost side folded back
-// for outflow (copy) and enforce-at-face inflow (2 state - cell) ghosts, a caller-filled ghost's own adjoint row;
-// then each species from the faces' multipliers and seeds (the species flux is the multiplier times the species
-// value).  Padding slots add 0 x (face 0's seed), as k_vjp does.
+// Per-cell sums of the face records of k_vjp_faces: its own half of each face in slot order, then the ghost halves
+// folded back for outflow (copy) and enforce-at-face inflow (2 state - cell) ghosts, a caller-filled ghost's own adjoint
+// row; then each species from the faces' multipliers and seeds (the species flux is the multiplier times the species
+// value).
 template <int DIM, int KM>
 __global__ __launch_bounds__(kBlock) void k_vjp_gather(MeshView<double> m, Phys ph, const double* __restrict__ Rb,
                                                        const double* __restrict__ fr,
                                                        const int32_t* __restrict__ ghost_slot,
                                                        const int32_t* __restrict__ slot_kind, double* __restrict__ Ub) {
     constexpr int NE = DIM + 2;
+    constexpr int SW = VjpRec<DIM>::SW;
     const int64_t c = xcd_cell_index();
     if (c >= m.NI) return;
-    const int64_t N = m.N, F = m.F, NI = m.NI;
-    double ub[NE], coef[KM], cghost[KM];
-    int64_t sf[KM], sR[KM];
-#pragma unroll
-    for (int p = 0; p < NE; p++) ub[p] = 0.0;
+    const int64_t N = m.N, NI = m.NI;
+    double ub[NE], ug[NE], coef[KM], cghost[KM], ivn[KM];
+    int32_t e[KM], nb[KM];  // neighbour across the slot: the cell itself for padding slots and ghosts
+    bool any_ghost = false;
 #pragma unroll
     for (int k = 0; k < KM; k++) {
-        const Slot sl = face_slot(m, k, c);
-        const int64_t f = sl.f;
-        sf[k] = f;
-        sR[k] = m.fcell[F + f];
-        cghost[k] = 0.0;
-        coef[k] = 0.0;
-        if (!sl.valid) continue;
-        const int64_t Rc = sR[k];
-        double cf = fr[(2 * NE + sl.s) * F + f];
+        e[k] = k < m.K ? m.ell[k * NI + c] : -1;
+        nb[k] = m.snbr[k * NI + c];
+    }
+    const double ivc = m.inv_vol[c];
 #pragma unroll
-        for (int p = 0; p < NE; p++) ub[p] += fr[(sl.s * NE + p) * F + f];
-        if (Rc >= NI) {
-            const int gk = slot_kind[ghost_slot[Rc - NI]];
-            if (gk == ABL_FV_BC_OUTFLOW) {
-#pragma unroll
-                for (int p = 0; p < NE; p++) ub[p] += fr[(NE + p) * F + f];
-                cf += fr[(2 * NE + 1) * F + f];
-            } else if (gk == kBcInflowAtFace) {
-#pragma unroll
-                for (int p = 0; p < NE; p++) ub[p] -= fr[(NE + p) * F + f];
-                cf -= fr[(2 * NE + 1) * F + f];
-            } else if (gk == ABL_FV_BC_GHOST) {
-#pragma unroll
-                for (int p = 0; p < NE; p++) Ub[p * N + Rc] = fr[(NE + p) * F + f];
-                cghost[k] = fr[(2 * NE + 1) * F + f];
-            }
-        }
-        coef[k] = cf;
+    for (int p = 0; p < NE; p++) {
+        ub[p] = 0.0;
+        ug[p] = 0.0;
     }
 #pragma unroll
-    for (int p = 0; p < NE; p++) Ub[p * N + c] = ub[p];
-    if (ph.ns == 0) return;
-    const double* __restrict__ gs = fr + (2 * NE + 2) * F;
-#pragma unroll 2
-    for (int sp = 0; sp < ph.ns; sp++) {
-        const int64_t comp = NE + sp;
-        double a = 0.0;
+    for (int k = 0; k < KM; k++) {
+        const bool valid = e[k] >= 0;
+        const double2* half = reinterpret_cast<const double2*>(fr) + face_pair(valid ? (int64_t)(e[k] >> 1) : 0, SW) +
+                              64 * (SW / 2) * (e[k] & 1);
+        double w[SW];
+#pragma unroll
+        for (int i = 0; i < SW / 2; i++) {
+            const double2 t = half[64 * i];
+            w[2 * i] = t.x;
+            w[2 * i + 1] = t.y;
+        }
+#pragma unroll
+        for (int p = 0; p < NE; p++) ub[p] += valid ? w[p] : 0.0;
+        coef[k] = valid ? w[NE] : 0.0;
+        cghost[k] = 0.0;
+        const bool inner = valid && nb[k] < NI;
+        any_ghost |= valid && nb[k] >= NI;
+        ivn[k] = m.inv_vol[inner ? nb[k] : c];
+        ivn[k] = inner ? ivn[k] : 0.0;
+    }
+    bool any_caller = false;
+    if (any_ghost) {
 #pragma unroll
         for (int k = 0; k < KM; k++) {
-            const double g = gs[(int64_t)sp * F + sf[k]];
-            a += coef[k] * g;
-            if (cghost[k] != 0.0) Ub[comp * N + sR[k]] = cghost[k] * g;
+            if (e[k] < 0 || nb[k] < NI) continue;
+            // the ghost is the right side
+            const double2* half = reinterpret_cast<const double2*>(fr) + face_pair(e[k] >> 1, SW) + 64 * (SW / 2);
+            double right[SW];
+#pragma unroll
+            for (int i = 0; i < SW / 2; i++) {
+                const double2 t = half[64 * i];
+                right[2 * i] = t.x;
+                right[2 * i + 1] = t.y;
+            }
+            const int gk = slot_kind[ghost_slot[nb[k] - NI]];
+            if (gk == ABL_FV_BC_OUTFLOW) {
+#pragma unroll
+                for (int p = 0; p < NE; p++) ug[p] += right[p];
+                coef[k] += right[NE];
+            } else if (gk == kBcInflowAtFace) {
+#pragma unroll
+                for (int p = 0; p < NE; p++) ug[p] -= right[p];
+                coef[k] -= right[NE];
+            } else if (gk == ABL_FV_BC_GHOST) {
+#pragma unroll
+                for (int p = 0; p < NE; p++) Ub[p * N + nb[k]] = right[p];
+                cghost[k] = right[NE];
+                any_caller |= cghost[k] != 0.0;
+            }
         }
-        Ub[comp * N + c] = a;
+    }
+#pragma unroll
+    for (int p = 0; p < NE; p++) Ub[p * N + c] = ub[p] + ug[p];
+    // species, the next one's seeds in flight while one is summed
+    double rc, rn[KM];
+    auto load = [&](int sp) {
+        const int64_t row = (int64_t)(NE + sp) * N;
+        rc = Rb[row + c];
+#pragma unroll
+        for (int k = 0; k < KM; k++) rn[k] = Rb[row + (e[k] >= 0 && nb[k] < NI ? (int64_t)nb[k] : c)];
+    };
+    if (ph.ns) load(0);
+    for (int sp = 0; sp < ph.ns; sp++) {
+        const int64_t row = (int64_t)(NE + sp) * N;
+        double r0 = rc, r[KM], g[KM], a = 0.0;
+#pragma unroll
+        for (int k = 0; k < KM; k++) r[k] = rn[k];
+        if (sp + 1 < ph.ns) load(sp + 1);
+#pragma unroll
+        for (int k = 0; k < KM; k++) {
+            const bool right = e[k] & 1;  // the cell is the right one
+            g[k] = right ? face_seed_of(r0, ivc, r[k], ivn[k]) : face_seed_of(r[k], ivn[k], r0, ivc);
+            a += coef[k] * (e[k] >= 0 ? g[k] : 0.0);
+        }
+        Ub[row + c] = a;
+        if (any_caller)
+#pragma unroll
+            for (int k = 0; k < KM; k++)
+                if (cghost[k] != 0.0) Ub[row + nb[k]] = cghost[k] * g[k];
     }
 }
 
@@ -2001,7 +2153,6 @@ struct AdjFaceRec {
     __host__ __device__ static int words(int ns) { return GS + ns; }
     __host__ __device__ static int pairs(int ns) { return (words(ns) + 1) / 2; }
 };
-__device__ inline int64_t adjw_pair(int64_t f, int nwp) { return (f >> 6) * 64 * (int64_t)nwp + (f & 63); }
 
 // Reverse of one face flux (advection, viscous, species advection and diffusion), both sides at once.  One lane per
 // face (interior and boundary).  The face's ghost-cell adjoints go straight to Ughost (a ghost has one face).
@@ -2071,7 +2222,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
     }
     // species sums of the face values; each species' g_sp = Rbar_sp(R) / V_R - Rbar_sp(L) / V_L goes straight into
     // the face record (read back below instead of the scattered Rbar rows)
-    double2* __restrict__ W = reinterpret_cast<double2*>(b.W) + adjw_pair(f, b.nwp);
+    double2* __restrict__ W = reinterpret_cast<double2*>(b.W) + face_pair(f, b.nwp);
     constexpr int NFIX = AW::GS / 2;  // pairs holding only fixed words
     // On interior faces the species diffusion flux's density adjoint (the face density 1/2 (rho_L + rho_R) times
     // n.(grad Y_L + grad Y_R)) is summed here too, while both sides' gradient words are in registers; boundary faces
@@ -2419,7 +2570,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_cells_e(MeshView<double> m, Phys
         // face density adjoint, and on a boundary face the right-side words (the left cell's extras)
         constexpr int NPS = (NE + 1) / 2;                      // pairs covering NE words from either parity
         constexpr int V0 = AW::TQ / 2, V1 = (AW::VL + DIM - 1) / 2;
-        const int64_t wb = adjw_pair(f, b.nwp);
+        const int64_t wb = face_pair(f, b.nwp);
         const int o = s ? AW::UR : AW::UL;
         const int p0 = o / 2;
         double sw_[2 * NPS], vw[2 * (V1 - V0 + 1)];
@@ -2583,7 +2734,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
         nb[k] = valid[k] ? (int64_t)n : c;
         bnd[k] = nb[k] >= NI;
         gi[k] = (valid[k] && bnd[k]) ? nb[k] - NI : -1;
-        wb[k] = adjw_pair(f, b.nwp);
+        wb[k] = face_pair(f, b.nwp);
         double x[2][DIM], nh[3], area;
         const int64_t geo = geometry_row(m, f);
         load_face_pair<DIM>(m.fdx, geo, x);
@@ -2928,6 +3079,7 @@ using FluxKernel = void (*)(MeshView<double>, Phys, const double*, const double*
                             double*, int);
 using FaceFluxKernel = void (*)(MeshView<double>, Phys, const double*, const double*, const double*, const double*,
                                 double*, double*);
+using GatherCoefKernel = void (*)(MeshView<double>, int, const double*, const double*, double*, int);
 using GatherKernel = void (*)(MeshView<double>, int, const double*, const double*, double*, int);
 
 template <typename G, int DIM, int KM, bool TAB, bool GHOSTS>
@@ -3099,6 +3251,14 @@ template <int DIM>
 TileKernel pick_tile(bool recon, bool visc, bool species, int K) {
     if (recon) return visc ? pick_tile2<DIM, true, true>(species, K) : pick_tile2<DIM, true, false>(species, K);
     return visc ? pick_tile2<DIM, false, true>(species, K) : pick_tile2<DIM, false, false>(species, K);
+}
+template <int DIM>
+GatherCoefKernel pick_gather_coef(int K) {
+    switch (slot_width(K)) {
+        case 4: return k_gather_coef<DIM, 4>;
+        case 6: return k_gather_coef<DIM, 6>;
+        default: return k_gather_coef<DIM, 8>;
+    }
 }
 template <int DIM>
 GatherKernel pick_gather(bool species, int K) {
@@ -3516,7 +3676,7 @@ struct abl_fv_solver {
     abl::VjpKernel vjp_kernel = nullptr;         // cell-centric first-order VJP (allocation-free entry)
     abl::VjpFacesKernel vjp_faces = nullptr;     // face-centric first-order VJP: face rows, then per-cell sums
     abl::VjpGatherKernel vjp_gather = nullptr;
-    abl::DevBuf<double> vjp_rows;                // [2 NE + 2 + ns][F] face rows of vjp_faces (first call allocates)
+    abl::DevBuf<double> vjp_rows;                // [F] VjpRec halves of vjp_faces (first call allocates)
     // second-order adjoint: kernels, mirror-slot table, workspace (allocated by the first such call)
     abl::AdjFacesKernel adj_faces = nullptr;
     abl::DevBuf<double> adjW, adjGL;  // face adjoint records, boundary-face species extras
@@ -3531,6 +3691,7 @@ struct abl_fv_solver {
     abl::FluxKernel flux_kernel = nullptr;
     abl::FaceFluxKernel face_flux_kernel = nullptr;
     abl::GatherKernel gather_kernel = nullptr;
+    abl::GatherCoefKernel gather_coef = nullptr;  // set for first-order inviscid species (in place of gather_kernel)
     int strategy = ABL_FV_STRATEGY_TILE;
     abl::DevBuf<unsigned long long> counter;
     abl::DevBuf<double> rmin, cfl_partial, cfl_out;  // MIN_CELL_RADIUS per interior cell; CFL reduction scratch
@@ -3645,8 +3806,9 @@ struct abl_fv_solver {
         const int nrow = host.dim + 2 + host.ns;
         if (form == ABL_FV_FORM_FP64) {
             if (face_flux_e.ptr) return;
-            face_flux_e.alloc((size_t)(((host.dim + 2) + 1) & ~1) * host.F);
-            if (host.ns) {  // species pairs interleaved per face (k_gather); an odd count's last slot stays zero
+            // euler fluxes and, for first-order inviscid species, the two species coefficients; an even record
+            face_flux_e.alloc((size_t)2 * abl::face_pairs_total(host.F, (host.dim + 2 + (gather_coef ? 2 : 0) + 1) / 2));
+            if (host.ns && !gather_coef) {  // species pairs interleaved per face (k_gather); an odd count's last slot stays zero
                 face_flux_s.alloc((size_t)(host.ns + 1) / 2 * 2 * host.F);
                 HIP_CHECK(hipMemset(face_flux_s.ptr, 0, face_flux_s.bytes()));
             }
@@ -3992,6 +4154,7 @@ extern "C" int abl_fv_create(const abl_fv_mesh_desc* mesh, const abl_fv_physics_
             s->face_flux_kernel = abl::pick_face_flux<3>(s->recon, s->visc, species);
             s->tile_kernel = abl::pick_tile<3>(s->recon, s->visc, species, L.K);
             s->gather_kernel = abl::pick_gather<3>(species, L.K);
+            if (species && !s->recon && !s->visc) s->gather_coef = abl::pick_gather_coef<3>(L.K);
             if (form == ABL_FV_FORM_FP64 && !species && !suth) s->fused_kernel = abl::pick_fused<3>(s->recon, s->visc, lim, L.K);
             if (form == ABL_FV_FORM_FP64 && !species && !suth) s->march_kernel = abl::pick_march<3>(s->recon, s->visc, lim, L.K);
         } else {
@@ -4002,6 +4165,7 @@ extern "C" int abl_fv_create(const abl_fv_mesh_desc* mesh, const abl_fv_physics_
             s->face_flux_kernel = abl::pick_face_flux<2>(s->recon, s->visc, species);
             s->tile_kernel = abl::pick_tile<2>(s->recon, s->visc, species, L.K);
             s->gather_kernel = abl::pick_gather<2>(species, L.K);
+            if (species && !s->recon && !s->visc) s->gather_coef = abl::pick_gather_coef<2>(L.K);
             if (form == ABL_FV_FORM_FP64 && !species && !suth) s->fused_kernel = abl::pick_fused<2>(s->recon, s->visc, lim, L.K);
             if (form == ABL_FV_FORM_FP64 && !species && !suth) s->march_kernel = abl::pick_march<2>(s->recon, s->visc, lim, L.K);
         }
@@ -4339,8 +4503,12 @@ extern "C" int abl_fv_rhs(abl_fv_handle h, double time, double* U, double* R, in
                                    h->gradA.ptr, h->rec.ptr, h->face_flux_e.ptr, h->face_flux_s.ptr);
             });
             h->timed(ABL_FV_PHASE_GATHER, st, [&] {
-                hipLaunchKernelGGL(h->gather_kernel, grid, block, 0, st, v, L.ns, h->face_flux_e.ptr, h->face_flux_s.ptr,
-                                   R, accumulate);
+                if (h->gather_coef)
+                    hipLaunchKernelGGL(h->gather_coef, grid, block, 0, st, v, L.ns, U, h->face_flux_e.ptr, R,
+                                       accumulate);
+                else
+                    hipLaunchKernelGGL(h->gather_kernel, grid, block, 0, st, v, L.ns, h->face_flux_e.ptr,
+                                       h->face_flux_s.ptr, R, accumulate);
             });
         } else {
             h->timed(ABL_FV_PHASE_FLUX, st, [&] {
@@ -4541,7 +4709,7 @@ extern "C" int abl_fv_rhs_vjp(abl_fv_handle h, double time, double* U, const dou
         if (theta_bar && h->n_bfaces && !h->theta_contrib.ptr) h->theta_contrib.alloc((size_t)3 * h->n_bfaces);
         if (theta_bar && h->n_bfaces && !h->theta_sum.ptr) h->theta_sum.alloc((size_t)3 * abl::kMaxBcSlots);
         if (fl != ABL_FV_FLUX_OFF && fl != ABL_FV_FLUX_NONE && L.F > 0 && !h->vjp_rows.ptr)
-            h->vjp_rows.alloc((size_t)(2 * (L.dim + 2) + 2 + L.ns) * L.F);
+            h->vjp_rows.alloc((size_t)2 * abl::face_pairs_total(L.F, L.dim == 3 ? abl::VjpRec<3>::SW : abl::VjpRec<2>::SW));
     } catch (const std::exception& e) {
         return fail(h, std::string("abl_fv_rhs_vjp: ") + e.what());
     }

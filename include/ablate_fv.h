@@ -247,8 +247,8 @@ int abl_fv_rhs(abl_fv_handle h, double time, double* U, double* R, int32_t accum
  *   any it leaves theta_bar as it is and returns without waiting).  Fluxes are recomputed, not stored.  Supported
  *   for the FP64 form with the
  *   Ausm, Rusanov or Off calculators, first order or least squares with the Barth-Jespersen limiter (or none),
- *   viscous and species fluxes; the first call allocates its workspace (first order: 2 n_euler + 2 + n_species
- *   doubles per face). */
+ *   viscous and species fluxes; the first call allocates its workspace (first order: 2 (n_euler + 1
+ *   rounded up to even) doubles per face). */
 int abl_fv_rhs_vjp(abl_fv_handle h, double time, double* U, const double* Rbar, double* Ubar, double* theta_bar,
                    abl_fv_stream stream);
 
@@ -341,7 +341,9 @@ enum {
     ABL_FV_STRATEGY_RECOMPUTE = 1, /* one lane per cell evaluates each of its faces: every face flux computed twice
                                       (mixed form: no species) */
     ABL_FV_STRATEGY_FACE_FLUX = 2, /* one lane per face stores its flux once; a second pass gathers per cell
-                                      (FP64: 8 * (n_euler + n_species rounded up to even) bytes per face; mixed:
+                                      (FP64: 8 * (n_euler + n_species rounded up to even) bytes per face, or for
+                                      first-order inviscid species 8 * (n_euler + 2) rounded up to even: the gather
+                                      forms the species fluxes from two coefficients per face; mixed:
                                       8 * (n_euler + n_species)) */
     ABL_FV_STRATEGY_TILE = 3,      /* one workgroup per tile of consecutive cells evaluates the tile's faces once into
                                       LDS and gathers its cells; bitwise equal to FACE_FLUX */
