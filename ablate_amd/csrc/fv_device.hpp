@@ -181,6 +181,13 @@ __device__ inline void load_slot_vec(const MeshView<G>& m, int k, int64_t c, G* 
     for (int d = 0; d < DIM; d++) v[d] = arr ? arr[(k * DIM + d) * m.NI + c] : G(0);
 }
 
+// Entry (face << 1) | side of slot k (< KM, which may exceed the table's width) of cell c, -1 = none; no branch.
+template <typename MV>
+__device__ inline int32_t slot_entry(const MV& m, int k, int64_t c) {
+    const int32_t e = m.ell[(int64_t)(k < m.K ? k : 0) * m.NI + c];
+    return k < m.K ? e : -1;
+}
+
 // Face slot k of interior cell c in the cell -> face table.  Loops over slots are unrolled to a compile-time
 // width so that every slot's loads issue up front; padding slots map to face 0 / the cell itself (valid addresses)
 // and are masked out of the arithmetic.

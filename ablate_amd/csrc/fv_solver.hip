@@ -2171,103 +2171,112 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
     const int64_t N = m.N, F = m.F, NI = m.NI, NG = N - NI;
     const int ns = ph.ns;
     const bool recon = ph.recon != 0, visc = ph.visc != 0, sdiff = ph.sdiff != 0;
-    const bool useRec = recon || visc;
     const int64_t L = m.fcell[f], Rc = m.fcell[F + f];
     const bool ghost = Rc >= NI;
+    const int64_t Rr = ghost ? L : Rc;  // a ghost has no record, gradients or Rbar: the left cell's are read, unused
     double nh[3], area, x[2][DIM];
     const int64_t geo = geometry_row(m, f);
     load_face_na(m.fna, geo, nh, area);
     load_face_pair<DIM>(m.fdx, geo, x);
-    const double ivL = m.inv_vol[L], ivR = ghost ? 0.0 : m.inv_vol[Rc];
-    double g[NE];
-#pragma unroll
-    for (int p = 0; p < NE; p++) g[p] = (ghost ? 0.0 : Rb[p * N + Rc] * ivR) - Rb[p * N + L] * ivL;
-    // both sides: cell state, face state and viscous terms
-    double uL[NE], uR[NE], fL[NE], fR[NE], tqL[NT], tqR[NT];
-#pragma unroll
-    for (int sd = 0; sd < 2; sd++) {
-        const int64_t cc = sd == 0 ? L : Rc;
-        double* u = sd == 0 ? uL : uR;
-        double* fu = sd == 0 ? fL : fR;
-        double* tq = sd == 0 ? tqL : tqR;
-        if (useRec && !(sd == 1 && ghost)) {
-            double r[CR::RS];
-            const double2* __restrict__ rb = reinterpret_cast<const double2*>(rec) + rec_pair<DIM>(cc);
-#pragma unroll
-            for (int q = 0; q < CR::NP; q++) {
-                const double2 v = rb[CR::BLOCK * q];
-                r[2 * q] = v.x;
-                r[2 * q + 1] = v.y;
-            }
-#pragma unroll
-            for (int p = 0; p < NE; p++) {
-                u[p] = r[p];
-                double a = 0.0;
-                if (recon)
-#pragma unroll
-                    for (int d = 0; d < DIM; d++) a += r[CR::G0 + p * DIM + d] * x[sd][d];
-                fu[p] = u[p] + a;
-            }
-#pragma unroll
-            for (int q = 0; q < NT; q++) tq[q] = r[CR::T0 + q];
-        } else {
-#pragma unroll
-            for (int p = 0; p < NE; p++) {
-                u[p] = U[p * N + cc];
-                fu[p] = u[p];
-            }
-#pragma unroll
-            for (int q = 0; q < NT; q++) tq[q] = 0.0;
-        }
-    }
-    // species sums of the face values; each species' g_sp = Rbar_sp(R) / V_R - Rbar_sp(L) / V_L goes straight into
-    // the face record (read back below instead of the scattered Rbar rows)
+    const double ivL = m.inv_vol[L], ivN = m.inv_vol[Rr], ivR = ghost ? 0.0 : ivN;
+    // Species sums of the face values, before the euler records take their registers, with the next species' loads in
+    // flight (they took the state records' and the species' rounds of latency one after the other before).  Each
+    // species' g_sp = Rbar_sp(R) / V_R - Rbar_sp(L) / V_L goes straight into the face record.  On interior faces the
+    // species diffusion flux's density adjoint (the face density 1/2 (rho_L + rho_R) times n.(grad Y_L + grad Y_R)) is
+    // summed here too; boundary faces take it in the ghost pass below.
     double2* __restrict__ W = reinterpret_cast<double2*>(b.W) + face_pair(f, b.nwp);
     constexpr int NFIX = AW::GS / 2;  // pairs holding only fixed words
-    // On interior faces the species diffusion flux's density adjoint (the face density 1/2 (rho_L + rho_R) times
-    // n.(grad Y_L + grad Y_R)) is summed here too, while both sides' gradient words are in registers; boundary faces
-    // take it in the ghost pass below.
     double QL = 0.0, QR = 0.0, QdL = 0.0, rhob = 0.0;
-    const double2* __restrict__ gS2 = reinterpret_cast<const double2*>(gS);
-    for (int q = 0; 2 * q < ns; q++) {
-        double gp0 = 0.0, gp1 = 0.0;
-#pragma unroll 1
-        for (int h = 0; h < 2; h++) {
-            const int sp = 2 * q + h;
-            if (sp >= ns) break;
+    if (ns) {
+        const double2* __restrict__ gS2 = reinterpret_cast<const double2*>(gS);
+        double xR[DIM];  // a ghost's face value is its state
+#pragma unroll
+        for (int d = 0; d < DIM; d++) xR[d] = ghost || !recon ? 0.0 : x[1][d];
+        const double cdiff = sdiff && !ghost ? -ph.diff * 0.25 * area : 0.0;
+        struct Sp {
+            double rl, rr, yl, yr;
+            double2 a[DIM], c[DIM];  // gradient words in pairs: [0, DIM) limited densityYi, [DIM, 2 DIM) Yi gradient
+        } nx;
+        auto load = [&](int sp) {
             const int64_t comp = NE + sp;
-            const double gsp = (ghost ? 0.0 : Rb[comp * N + Rc] * ivR) - Rb[comp * N + L] * ivL;
-            if (h) gp1 = gsp;
-            else gp0 = gsp;
-            double yl = U[comp * N + L], yr = U[comp * N + Rc], dot = 0.0;
-            // each side's gradient words in pairs: [0, DIM) limited densityYi gradient, [DIM, 2 DIM) Yi gradient
+            nx.rl = Rb[comp * N + L];
+            nx.rr = Rb[comp * N + Rr];
+            nx.yl = U[comp * N + L];
+            nx.yr = U[comp * N + Rc];
 #pragma unroll
-            for (int j = 0; j < DIM; j++) {
-                const bool need = (recon && 2 * j < DIM) || (sdiff && 2 * j + 1 >= DIM);
-                if (!need) continue;
-                const double2 a = gS2[((int64_t)sp * DIM + j) * N + L];
-                const double2 c2 = ghost ? make_double2(0.0, 0.0) : gS2[((int64_t)sp * DIM + j) * N + Rc];
+            for (int q = 0; q < DIM; q++) {
+                nx.a[q] = gS2[((int64_t)sp * DIM + q) * N + L];
+                nx.c[q] = gS2[((int64_t)sp * DIM + q) * N + Rr];
+            }
+        };
+        load(0);
+        double first = 0.0;
+        for (int sp = 0; sp < ns; sp++) {
+            const Sp v = nx;
+            if (sp + 1 < ns) load(sp + 1);
+            const double gsp = face_seed_of(ghost ? 0.0 : v.rr, ivR, v.rl, ivL);
+            double wl[2 * DIM], wr[2 * DIM], yl = v.yl, yr = v.yr, dot = 0.0;
 #pragma unroll
-                for (int h2 = 0; h2 < 2; h2++) {
-                    const int w = 2 * j + h2;
-                    const double wl = h2 ? a.y : a.x, wr = h2 ? c2.y : c2.x;
-                    if (w < DIM) {
-                        if (recon) {
-                            yl += wl * x[0][w];
-                            yr += wr * x[1][w];
-                        }
-                    } else {
-                        dot += nh[w - DIM] * (wl + wr);
-                    }
-                }
+            for (int q = 0; q < DIM; q++) {
+                wl[2 * q] = v.a[q].x;
+                wl[2 * q + 1] = v.a[q].y;
+                wr[2 * q] = v.c[q].x;
+                wr[2 * q + 1] = v.c[q].y;
+            }
+#pragma unroll
+            for (int d = 0; d < DIM; d++) {
+                yl += wl[d] * (recon ? x[0][d] : 0.0);
+                yr += wr[d] * xR[d];
+                dot += nh[d] * (wl[DIM + d] + wr[DIM + d]);
             }
             QL += gsp * yl;
             QR += gsp * yr;
             QdL += gsp * (yr - yl);
-            // rho_L and rho_R enter the face density alike
-            if (sdiff && !ghost) rhob += gsp * (-ph.diff * 0.25 * area) * dot;
+            rhob += gsp * cdiff * dot;  // rho_L and rho_R enter the face density alike
+            if (sp & 1)
+                W[64 * (NFIX + (sp >> 1))] = make_double2(first, gsp);
+            else if (sp + 1 == ns)
+                W[64 * (NFIX + (sp >> 1))] = make_double2(gsp, 0.0);
+            first = gsp;
         }
-        W[64 * (NFIX + q)] = make_double2(gp0, gp1);
+    }
+    double g[NE];
+#pragma unroll
+    for (int p = 0; p < NE; p++) g[p] = face_seed_of(ghost ? 0.0 : Rb[p * N + Rr], ivR, Rb[p * N + L], ivL);
+    // both sides: cell state, face state and viscous terms from the cell records
+    double uL[NE], uR[NE], fL[NE], fR[NE], tqL[NT], tqR[NT];
+#pragma unroll
+    for (int sd = 0; sd < 2; sd++) {
+        double* u = sd == 0 ? uL : uR;
+        double* fu = sd == 0 ? fL : fR;
+        double* tq = sd == 0 ? tqL : tqR;
+        double r[CR::RS];
+        const double2* __restrict__ rb = reinterpret_cast<const double2*>(rec) + rec_pair<DIM>(sd == 0 ? L : Rr);
+#pragma unroll
+        for (int q = 0; q < CR::NP; q++) {
+            const double2 v = rb[CR::BLOCK * q];
+            r[2 * q] = v.x;
+            r[2 * q + 1] = v.y;
+        }
+#pragma unroll
+        for (int p = 0; p < NE; p++) {
+            u[p] = r[p];
+            double a = 0.0;
+#pragma unroll
+            for (int d = 0; d < DIM; d++) a += r[CR::G0 + p * DIM + d] * x[sd][d];
+            fu[p] = recon ? u[p] + a : u[p];
+        }
+#pragma unroll
+        for (int q = 0; q < NT; q++) tq[q] = r[CR::T0 + q];
+    }
+    if (ghost) {
+#pragma unroll
+        for (int p = 0; p < NE; p++) {
+            uR[p] = U[p * N + Rc];
+            fR[p] = uR[p];
+        }
+#pragma unroll
+        for (int q = 0; q < NT; q++) tqR[q] = 0.0;
     }
     double ubL[NE], ubR[NE], cL = 0.0, cR = 0.0;
 #pragma unroll
@@ -2408,113 +2417,78 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
     for (int q = 0; q < NFIX; q++) W[64 * q] = make_double2(w[2 * q], w[2 * q + 1]);
 }
 
-// Barth-Jespersen limiter of one component with its active pieces: phi = min(1, (umax - uc) / dpos, (umin - uc) /
-// dneg); imax / imin = slot of the extreme neighbour (-1: the cell itself), kpos / kneg = slot of the extreme face
-// projection.
-struct BJFwd {
-    double umax, umin, dpos, dneg, phi;
-    int imax, imin, kpos, kneg, active;  // active: 0 none (phi = 1), 1 max side, 2 min side
-};
-__device__ inline void bj_finish(double uc, BJFwd& L) {
-    L.phi = 1.0;
-    L.active = 0;
-    if (L.dpos > 0.0) {
-        const double r = (L.umax - uc) / L.dpos;
-        if (r < L.phi) {
-            L.phi = r;
-            L.active = 1;
-        }
-    }
-    if (L.dneg < 0.0) {
-        const double r = (L.umin - uc) / L.dneg;
-        if (r < L.phi) {
-            L.phi = r;
-            L.active = 2;
-        }
-    }
-}
-
 // Reverse of one component's limited least-squares gradient g = phi(G) G, G = sum_k w_k (u_n - u_c), given the
 // adjoint gbl of g: adds the adjoint of the cell's own value to ubc and of each neighbour's to cn[k] (ghost
-// neighbours through to_ghost).  unv[k] = the component's value in the neighbour across slot k, x[k] = x_f - x_c of
-// slot k (the Barth-Jespersen projection vector).
+// neighbours through to_ghost).  unv[k] = the component's value in the neighbour across slot k (the cell's own in
+// padding slots), x[k] = x_f - x_c of slot k (the Barth-Jespersen projection vector, zero in padding slots).  The limiter is phi = min(1,
+// (umax - uc) / dpos, (umin - uc) / dneg); its active pieces are the slot of the extreme neighbour (imax / imin, -1: the
+// cell itself) and of the extreme face projection (kpos / kneg).  Conditions are selects (see gradients_body).
 template <int DIM, int KM, typename ToGhost>
-__device__ inline void limited_lsq_vjp(const double* unv, double uc, const double (*w)[DIM], const double (*x)[DIM],
-                                       const int64_t* nb, const bool* valid, const bool* bnd, bool bj,
-                                       const double* gbl, double& ubc, double* cn, ToGhost&& to_ghost) {
+__device__ __forceinline__ void limited_lsq_vjp(const double* unv, double uc, const double (*w)[DIM],
+                                                const double (*x)[DIM], const bool* bnd, bool any_bnd, bool bj,
+                                                const double* gbl, double& ubc, double* cn, ToGhost&& to_ghost) {
     double G[DIM], Gb[DIM];
 #pragma unroll
     for (int d = 0; d < DIM; d++) G[d] = 0.0;
-    BJFwd lim{uc, uc, 0.0, 0.0, 1.0, -1, -1, -1, -1, 0};
+    double umax = uc, umin = uc;
+    int imax = -1, imin = -1;
 #pragma unroll
     for (int k = 0; k < KM; k++) {
-        if (!valid[k]) continue;
-        const double un = unv[k];
-        if (!bnd[k])
+        const double delta = bnd[k] ? 0.0 : unv[k] - uc;
 #pragma unroll
-            for (int d = 0; d < DIM; d++) G[d] += w[k][d] * (un - uc);
-        if (un > lim.umax) {
-            lim.umax = un;
-            lim.imax = k;
-        }
-        if (un < lim.umin) {
-            lim.umin = un;
-            lim.imin = k;
-        }
+        for (int d = 0; d < DIM; d++) G[d] += w[k][d] * delta;
+        imax = unv[k] > umax ? k : imax;
+        umax = unv[k] > umax ? unv[k] : umax;
+        imin = unv[k] < umin ? k : imin;
+        umin = unv[k] < umin ? unv[k] : umin;
     }
-    if (bj) {
+    double dpos = 0.0, dneg = 0.0;
+    int kpos = -1, kneg = -1;
 #pragma unroll
-        for (int k = 0; k < KM; k++) {
-            if (!valid[k]) continue;
-            double D = 0.0;
+    for (int k = 0; k < KM; k++) {
+        double D = 0.0;
 #pragma unroll
-            for (int d = 0; d < DIM; d++) D += G[d] * x[k][d];
-            if (D > lim.dpos) {
-                lim.dpos = D;
-                lim.kpos = k;
-            }
-            if (D < lim.dneg) {
-                lim.dneg = D;
-                lim.kneg = k;
-            }
-        }
-        bj_finish(uc, lim);
+        for (int d = 0; d < DIM; d++) D += G[d] * x[k][d];
+        kpos = D > dpos ? k : kpos;
+        dpos = D > dpos ? D : dpos;
+        kneg = D < dneg ? k : kneg;
+        dneg = D < dneg ? D : dneg;
     }
+    const double rp = (umax - uc) / dpos, rn = (umin - uc) / dneg;
+    double phi = 1.0;
+    const bool ap = bj && dpos > 0.0 && rp < phi;
+    phi = ap ? rp : phi;
+    const bool an = bj && dneg < 0.0 && rn < phi;
+    phi = an ? rn : phi;
+    const double den = an ? dneg : (ap ? dpos : 1.0);
+    const int ext = an ? imin : imax, kd = an ? kneg : kpos;  // extreme neighbour and projection of the active bound
     double phib = 0.0;
 #pragma unroll
     for (int d = 0; d < DIM; d++) {
-        Gb[d] = lim.phi * gbl[d];
+        Gb[d] = phi * gbl[d];
         phib += gbl[d] * G[d];
     }
-    if (bj && lim.active) {
-        const bool mx = lim.active == 1;
-        const double den = mx ? lim.dpos : lim.dneg;
-        const int ext = mx ? lim.imax : lim.imin;
-        const int kd = mx ? lim.kpos : lim.kneg;
-        const double ub_ext = phib / den;
-        ubc -= ub_ext;
-        if (ext < 0) ubc += ub_ext;
-        const double den_b = -lim.phi * phib / den;
+    const double ub_ext = ap || an ? phib / den : 0.0;
+    ubc -= ext < 0 ? 0.0 : ub_ext;  // an extreme at the cell itself returns what it takes
+    const double den_b = -phi * ub_ext;
 #pragma unroll
-        for (int k = 0; k < KM; k++) {  // selects, not runtime register indices (which would spill)
-            if (k == ext) {
-                if (bnd[k])
-                    to_ghost(nb[k], ub_ext);
-                else
-                    cn[k] += ub_ext;
-            }
-            if (k == kd)
+    for (int k = 0; k < KM; k++) {  // selects, not runtime register indices (which would spill)
+        cn[k] += k == ext && !bnd[k] ? ub_ext : 0.0;
+        const double t = k == kd ? den_b : 0.0;
 #pragma unroll
-                for (int d = 0; d < DIM; d++) Gb[d] += den_b * x[k][d];
-        }
+        for (int d = 0; d < DIM; d++) Gb[d] += t * x[k][d];
     }
+    if (any_bnd && ub_ext != 0.0)
+#pragma unroll
+        for (int k = 0; k < KM; k++)
+            if (k == ext && bnd[k]) to_ghost(k, ub_ext);
     // least-squares gradient: G = sum_k w_k (u_n - u_c)
 #pragma unroll
     for (int k = 0; k < KM; k++) {
-        if (!valid[k] || bnd[k]) continue;
         double t = 0.0;
 #pragma unroll
         for (int d = 0; d < DIM; d++) t += w[k][d] * Gb[d];
+        t = bnd[k] ? 0.0 : t;
         cn[k] += t;
         ubc -= t;
     }
@@ -2524,9 +2498,14 @@ __device__ inline void limited_lsq_vjp(const double* unv, double uc, const doubl
 // gradients through the face state U + G dx, viscous terms, face velocity and density, boundary-face extras), then
 // reverses the limiter, the least-squares gradients and the aux (temperature / velocity) gradients of the cell;
 // writes its own adjoint and, per face slot, the contribution for the neighbour across the face.
-template <int DIM, int KM>
-__global__ __launch_bounds__(kBlock) void k_adj_cells_e(MeshView<double> m, Phys ph, const double* __restrict__ U,
-                                                        AdjBufs b) {
+// The reverse walks the components: a component needs its own neighbour values, its gradient adjoint and, for the aux
+// gradients, 1 / rho and the temperature adjoint of every neighbour, so only those stay in registers (two waves per SIMD
+// for hexes; with all neighbours' states and all contributions live they took 288 VGPRs, one wave per SIMD, and a
+// branch per slot made the record loads of the six slots six dependent rounds).  The density comes last: the other
+// components' aux terms add to it.
+template <int DIM, int KM, bool RECON, bool VISC, bool TAB>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_adj_cells_e(
+    MeshView<double> m, Phys ph, const double* __restrict__ U, AdjBufs b) {
     constexpr int NE = DIM + 2;
     constexpr int NT = ViscTerms<DIM>::NT;
     using AW = AdjFaceRec<DIM>;
@@ -2534,10 +2513,33 @@ __global__ __launch_bounds__(kBlock) void k_adj_cells_e(MeshView<double> m, Phys
     if (c >= m.NI) return;
     const int64_t N = m.N, NI = m.NI, NG = N - NI;
     const int nc = NE + ph.ns;
-    const bool recon = ph.recon != 0, visc = ph.visc != 0;
     const bool bj = ph.limiter == ABL_FV_LIMITER_BARTH_JESPERSEN;
     const double2* __restrict__ W = reinterpret_cast<const double2*>(b.W);
-    double ub[NE], gb[NE][DIM], tqb[NT], velb[DIM], auxb[DIM + 1], rhob = 0.0;
+    int32_t e[KM], nb[KM];
+    bool valid[KM], bnd[KM], any_bnd = false;
+    uint32_t row[KM];  // word offsets of the slots' table rows
+#pragma unroll
+    for (int k = 0; k < KM; k++) {
+        e[k] = slot_entry(m, k, c);
+        nb[k] = m.snbr[k * NI + c];
+        row[k] = TAB ? (uint32_t)m.srow[k * NI + c] * (uint32_t)m.sstride : 0u;
+    }
+    // geometry vectors of slot k (zero in padding slots); offsets are formed anew for each read (pin)
+    const double* __restrict__ wa_arr = m.swa ? m.swa : m.sw;
+    auto slot_vec = [&](const double* arr, int off, int k, double* v) {
+        if (TAB) pin(row[k]);
+#pragma unroll
+        for (int d = 0; d < DIM; d++) v[d] = TAB ? m.stab[row[k] + (uint32_t)(off + d)] : arr[(k * DIM + d) * NI + c];
+    };
+#pragma unroll
+    for (int k = 0; k < KM; k++) {
+        valid[k] = e[k] >= 0;
+        nb[k] = valid[k] ? nb[k] : (int32_t)c;
+        bnd[k] = nb[k] >= NI;
+        any_bnd |= bnd[k];
+    }
+    double ub[NE], gb[NE][DIM], tqb[NT], velb[DIM], rhob = 0.0;
+    double xs[KM][DIM];  // x_f - x_c of the slots
 #pragma unroll
     for (int p = 0; p < NE; p++) {
         ub[p] = 0.0;
@@ -2548,161 +2550,210 @@ __global__ __launch_bounds__(kBlock) void k_adj_cells_e(MeshView<double> m, Phys
     for (int q = 0; q < NT; q++) tqb[q] = 0.0;
 #pragma unroll
     for (int d = 0; d < DIM; d++) velb[d] = 0.0;
-#pragma unroll
-    for (int q = 0; q <= DIM; q++) auxb[q] = 0.0;
-    int64_t nb[KM];
-    bool valid[KM], bnd[KM];
-    double xs[KM][DIM];
-#pragma unroll
-    for (int k = 0; k < KM; k++) {
-        const int32_t e = k < m.K ? m.ell[k * NI + c] : -1;
-        valid[k] = e >= 0;
-        const int64_t f = valid[k] ? (int64_t)(e >> 1) : 0;
-        const int s = e & 1;
-        const int32_t n = m.snbr[k * NI + c];
-        nb[k] = valid[k] ? (int64_t)n : c;
-        bnd[k] = nb[k] >= NI;
-        double x[2][DIM];
-        load_face_pair<DIM>(m.fdx, geometry_row(m, f), x);
-#pragma unroll
-        for (int d = 0; d < DIM; d++) xs[k][d] = s ? x[1][d] : x[0][d];
-        // the record pairs this cell needs: its side's face-state adjoint, the viscous terms and face velocity, the
-        // face density adjoint, and on a boundary face the right-side words (the left cell's extras)
-        constexpr int NPS = (NE + 1) / 2;                      // pairs covering NE words from either parity
-        constexpr int V0 = AW::TQ / 2, V1 = (AW::VL + DIM - 1) / 2;
-        const int64_t wb = face_pair(f, b.nwp);
-        const int o = s ? AW::UR : AW::UL;
-        const int p0 = o / 2;
-        double sw_[2 * NPS], vw[2 * (V1 - V0 + 1)];
+    // the record pairs a cell needs of a face: its side's face-state adjoint, the viscous terms and face velocity, the
+    // face density adjoint
+    constexpr int NPS = (NE + 1) / 2;  // pairs covering NE words from either parity
+    constexpr int V0 = AW::TQ / 2, V1 = (AW::VL + DIM - 1) / 2;
+    double sd[2][2 * NPS], vw[2][2 * (V1 - V0 + 1)], rh[2];  // two slots in flight, as in gradients_body
+    auto load_face = [&](int k) {
+        // a padding slot reads the cell's first face and counts it zero times
+        const double2* __restrict__ rec = W + face_pair((valid[k] ? e[k] : e[0]) >> 1, b.nwp);
+        const int o = (e[k] & 1) ? AW::UR : AW::UL;
 #pragma unroll
         for (int i = 0; i < NPS; i++) {
-            const double2 v = W[wb + 64 * (p0 + i)];
-            sw_[2 * i] = v.x;
-            sw_[2 * i + 1] = v.y;
+            const double2 v = rec[64 * (o / 2 + i)];
+            sd[k & 1][2 * i] = v.x;
+            sd[k & 1][2 * i + 1] = v.y;
         }
-        if (visc)
+        if (VISC)
 #pragma unroll
             for (int q = V0; q <= V1; q++) {
-                const double2 v = W[wb + 64 * q];
-                vw[2 * (q - V0)] = v.x;
-                vw[2 * (q - V0) + 1] = v.y;
+                const double2 v = rec[64 * q];
+                vw[k & 1][2 * (q - V0)] = v.x;
+                vw[k & 1][2 * (q - V0) + 1] = v.y;
             }
-        const double2 rp = W[wb + 64 * (AW::RH / 2)];
-        const double rh = (AW::RH & 1) ? rp.y : rp.x;
-        if (!valid[k]) continue;
+        const double2 rp = rec[64 * (AW::RH / 2)];
+        rh[k & 1] = (AW::RH & 1) ? rp.y : rp.x;
+        if (RECON) slot_vec(m.slim, DIM, k, xs[k]);
+    };
+    load_face(0);
+#pragma unroll
+    for (int k = 0; k < KM; k++) {
+        if (k + 1 < KM) load_face(k + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        const int s = e[k] & 1, h = k & 1;
+        const double count = valid[k] ? 1.0 : 0.0;
 #pragma unroll
         for (int p = 0; p < NE; p++) {
-            const double wp = sw_[o + p - 2 * p0];
-            ub[p] += wp;
-            if (recon)
+            // words [o, o + NE) start in either half of a pair
+            const double w0 = sd[h][p], w1 = sd[h][p + 1 < 2 * NPS ? p + 1 : p];
+            const double v = count * ((s ? (AW::UR & 1) : (AW::UL & 1)) ? w1 : w0);
+            ub[p] += v;
+            if (RECON)
 #pragma unroll
-                for (int d = 0; d < DIM; d++) gb[p][d] += wp * xs[k][d];
+                for (int d = 0; d < DIM; d++) gb[p][d] += v * xs[k][d];
         }
-        if (visc) {
+        if (VISC) {
 #pragma unroll
-            for (int q = 0; q < NT; q++) tqb[q] += vw[AW::TQ + q - 2 * V0];
+            for (int q = 0; q < NT; q++) tqb[q] += count * vw[h][AW::TQ + q - 2 * V0];
 #pragma unroll
-            for (int d = 0; d < DIM; d++) velb[d] += vw[AW::VL + d - 2 * V0];
+            for (int d = 0; d < DIM; d++) velb[d] += count * vw[h][AW::VL + d - 2 * V0];
+            rhob += count * rh[h];
         }
-        rhob += rh;
-        if (bnd[k]) {  // boundary face: the left cell's extras from the ghost's viscous gradient
+        pin(ub);
+        if (RECON) pin(gb);
+        if (VISC) {
+            pin(tqb);
+            pin(velb);
+            pin(rhob);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    double ab[DIM + 1];  // aux adjoint of the cell: the face velocities', the extras below, then the gradients'
+#pragma unroll
+    for (int q = 0; q <= DIM; q++) ab[q] = q == 0 ? 0.0 : velb[q - 1];
+    if (VISC && any_bnd) {  // boundary faces: the left cell's extras from the ghost's viscous gradient
+#pragma unroll
+        for (int k = 0; k < KM; k++) {
+            if (!bnd[k]) continue;
+            const double2* __restrict__ rec = W + face_pair(e[k] >> 1, b.nwp);
             constexpr int R0 = AW::UR / 2;
             double rw[2 * NPS];
 #pragma unroll
             for (int i = 0; i < NPS; i++) {
-                const double2 v = W[wb + 64 * (R0 + i)];
+                const double2 v = rec[64 * (R0 + i)];
                 rw[2 * i] = v.x;
                 rw[2 * i + 1] = v.y;
             }
 #pragma unroll
-            for (int q = 0; q <= DIM; q++) auxb[q] += rw[AW::UR + q - 2 * R0];
+            for (int q = 0; q <= DIM; q++) ab[q] += rw[AW::UR + q - 2 * R0];
             rhob += rw[AW::UR + DIM + 1 - 2 * R0];
         }
     }
-    double uc[NE];
-#pragma unroll
-    for (int p = 0; p < NE; p++) uc[p] = U[p * N + c];
-    if (visc) {
-        double ab[DIM + 1];
-        ab[0] = auxb[0];
-#pragma unroll
-        for (int d = 0; d < DIM; d++) ab[1 + d] = velb[d] + auxb[1 + d];
-        aux_vjp<DIM>(uc, ph, ab, ub);
-    }
     ub[kRho] += rhob;
-    // the cell's reverse: limiter and least-squares gradients, then the aux gradients
-    double ce[KM][NE];
+    double gAb[DIM + 1][DIM], irn[KM], tn[KM], rn[KM];  // per neighbour: 1 / rho, T adjoint, rho's sum
+    if (VISC) {
 #pragma unroll
-    for (int k = 0; k < KM; k++)
-#pragma unroll
-        for (int p = 0; p < NE; p++) ce[k][p] = 0.0;
-    double unb_all[KM][NE];  // neighbour states (the limiter / least-squares and the aux reverses both read them)
-#pragma unroll
-    for (int k = 0; k < KM; k++)
-#pragma unroll
-        for (int p = 0; p < NE; p++) unb_all[k][p] = U[p * N + nb[k]];
-    if (recon) {
-        double wl[KM][DIM];
-#pragma unroll
-        for (int k = 0; k < KM; k++) load_slot_vec<DIM, KM, kSlotWeight>(m, k, c, wl[k]);
-#pragma unroll
-        for (int p = 0; p < NE; p++) {
-            double cn[KM], unv[KM];
-#pragma unroll
-            for (int k = 0; k < KM; k++) {
-                cn[k] = 0.0;
-                unv[k] = unb_all[k][p];
-            }
-            limited_lsq_vjp<DIM, KM>(unv, uc[p], wl, xs, nb, valid, bnd, bj, gb[p], ub[p], cn,
-                                     [&](int64_t g, double v) { b.Ughost[(int64_t)p * NG + (g - NI)] += v; });
-#pragma unroll
-            for (int k = 0; k < KM; k++) ce[k][p] += cn[k];
-        }
-    }
-    if (visc) {
-        double gAb[DIM + 1][DIM], acb[DIM + 1];
-#pragma unroll
-        for (int q = 0; q <= DIM; q++) {
-            acb[q] = 0.0;
+        for (int q = 0; q <= DIM; q++)
 #pragma unroll
             for (int d = 0; d < DIM; d++) gAb[q][d] = 0.0;
-        }
         stress_heat_vjp<DIM>(ph.mu, ph.k, tqb, gAb);
+        pin(gAb);
+    }
+    // the slots' weights and limiter vectors stay in registers for four slots and are read again for each component
+    // for more (from the geometry tables' cache lines on hexes)
+    constexpr bool RELOAD = KM > 4;
+    double wl[KM][DIM];
+    auto load_vectors = [&]() {
 #pragma unroll
         for (int k = 0; k < KM; k++) {
-            if (!valid[k]) continue;
-            double anb[DIM + 1], un[NE], unb[NE], wa[DIM];
-            load_slot_vec<DIM, KM, kSlotAux>(m, k, c, wa);
-#pragma unroll
-            for (int q = 0; q <= DIM; q++) {
-                double t = 0.0;
-#pragma unroll
-                for (int d = 0; d < DIM; d++) t += wa[d] * gAb[q][d];
-                anb[q] = t;
-                acb[q] -= t;
-            }
-#pragma unroll
-            for (int p = 0; p < NE; p++) {
-                un[p] = unb_all[k][p];
-                unb[p] = 0.0;
-            }
-            aux_vjp<DIM>(un, ph, anb, unb);
-#pragma unroll
-            for (int p = 0; p < NE; p++) {
-                if (bnd[k])
-                    b.Ughost[(int64_t)p * NG + (nb[k] - NI)] += unb[p];
-                else
-                    ce[k][p] += unb[p];
-            }
+            slot_vec(m.sw, 0, k, wl[k]);
+            if (RELOAD) slot_vec(m.slim, DIM, k, xs[k]);
         }
-        aux_vjp<DIM>(uc, ph, acb, ub);
+    };
+    if (RECON && !RELOAD) load_vectors();
+    double un[KM], uc;
+    auto load = [&](int p) {
+        uc = U[p * N + c];
+#pragma unroll
+        for (int k = 0; k < KM; k++) {
+            pin(nb[k]);
+            un[k] = U[p * N + nb[k]];
+        }
+    };
+    if (VISC) {
+        load(kRho);
+#pragma unroll
+        for (int k = 0; k < KM; k++) {
+            irn[k] = 1.0 / un[k];
+            rn[k] = 0.0;
+        }
+        pin(irn);
+    }
+    load(kRhoE);
+    // aux adjoint component q of every neighbour: wa_k . gAb[q]; read and formed before the next component's loads are
+    // issued (loads return in order)
+    auto aux_adjoint = [&](int q, double* t) {
+        double wv[KM][DIM];
+#pragma unroll
+        for (int k = 0; k < KM; k++) slot_vec(wa_arr, TAB ? m.saux : 0, k, wv[k]);
+#pragma unroll
+        for (int k = 0; k < KM; k++) {
+            const double* wa = wv[k];
+            t[k] = 0.0;
+#pragma unroll
+            for (int d = 0; d < DIM; d++) t[k] += wa[d] * gAb[q][d];
+            ab[q] -= t[k];
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < NE; i++) {
+        const int p = (i + 1) % NE;  // rhoE, rhoU ..., rho
+        double v[KM], cn[KM], ax[KM];
+        const double u0 = uc;
+#pragma unroll
+        for (int k = 0; k < KM; k++) {
+            v[k] = un[k];
+            cn[k] = 0.0;
+            ax[k] = 0.0;
+        }
+        double tv[KM];
+        if (VISC && p != kRho) {
+            aux_adjoint(p == kRhoE ? 0 : 1 + p - kRhoU, tv);
+            pin(tv);
+            pin(ab);
+        }
+        if (RECON && RELOAD) load_vectors();
+        if (i + 1 < NE) load((i + 2) % NE);
+        __builtin_amdgcn_sched_barrier(0);
+        if (VISC) {
+            // aux_vjp of the neighbour's state: T = (rhoE / rho - |vel|^2 / 2) / cv, vel = rhoU / rho
+            if (p == kRhoE) {
+#pragma unroll
+                for (int k = 0; k < KM; k++) {
+                    tn[k] = tv[k];
+                    ax[k] = tn[k] * ph.icv * irn[k];
+                    rn[k] -= ax[k] * v[k] * irn[k];
+                }
+                pin(tn);
+            } else if (p != kRho) {
+#pragma unroll
+                for (int k = 0; k < KM; k++) {
+                    const double vel = v[k] * irn[k];
+                    ax[k] = (tv[k] - tn[k] * vel * ph.icv) * irn[k];
+                    rn[k] -= ax[k] * vel;
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < KM; k++) ax[k] = rn[k];
+            }
+            pin(rn);
+            pin(ax);
+        }
+        if (RECON)
+            limited_lsq_vjp<DIM, KM>(v, u0, wl, xs, bnd, any_bnd, bj, gb[p], ub[p], cn, [&](int k, double t) {
+                b.Ughost[(int64_t)p * NG + (nb[k] - NI)] += t;
+            });
+        pin(ub[p]);
+#pragma unroll
+        for (int k = 0; k < KM; k++) {
+            b.contrib[((int64_t)k * nc + p) * NI + c] = bnd[k] ? 0.0 : cn[k] + ax[k];
+            pin(cn[k]);
+        }
+        if (VISC && any_bnd)
+#pragma unroll
+            for (int k = 0; k < KM; k++)
+                if (bnd[k]) b.Ughost[(int64_t)p * NG + (nb[k] - NI)] += ax[k];
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (VISC) {
+        double uo[NE];
+#pragma unroll
+        for (int p = 0; p < NE; p++) uo[p] = U[p * N + c];
+        aux_vjp<DIM>(uo, ph, ab, ub);
     }
 #pragma unroll
     for (int p = 0; p < NE; p++) b.Uself[(int64_t)p * NI + c] = ub[p];
-#pragma unroll
-    for (int k = 0; k < KM; k++)
-#pragma unroll
-        for (int p = 0; p < NE; p++) b.contrib[((int64_t)k * nc + p) * NI + c] = ce[k][p];
 }
 
 // Pass 2, species (lane per interior cell, after k_adj_cells_e): per species, sums the species factors of its faces'
@@ -2722,7 +2773,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     const bool bj = ph.limiter == ABL_FV_LIMITER_BARTH_JESPERSEN;
     const double2* __restrict__ W = reinterpret_cast<const double2*>(b.W);
     int64_t nb[KM], wb[KM], gi[KM];
-    bool valid[KM], bnd[KM];
+    bool valid[KM], bnd[KM], any_bnd = false;
     double xs[KM][DIM], cnv[KM][DIM], csk[KM], wl[KM][DIM], wa[KM][DIM];
 #pragma unroll
     for (int k = 0; k < KM; k++) {
@@ -2733,6 +2784,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
         const int32_t n = m.snbr[k * NI + c];
         nb[k] = valid[k] ? (int64_t)n : c;
         bnd[k] = nb[k] >= NI;
+        any_bnd |= bnd[k];
         gi[k] = (valid[k] && bnd[k]) ? nb[k] - NI : -1;
         wb[k] = face_pair(f, b.nwp);
         double x[2][DIM], nh[3], area;
@@ -2814,8 +2866,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
             for (int k = 0; k < KM; k++) cs[k] = 0.0;
             if (recon)
-                limited_lsq_vjp<DIM, KM>(unv[h], ycs[h], wl, xs, nb, valid, bnd, bj, gsb, usb, cs,
-                                         [&](int64_t g, double v) { b.Ughost[comp * NG + (g - NI)] += v; });
+                limited_lsq_vjp<DIM, KM>(unv[h], ycs[h], wl, xs, bnd, any_bnd, bj, gsb, usb, cs,
+                                         [&](int k, double v) { b.Ughost[comp * NG + (nb[k] - NI)] += v; });
             if (sdiff) {
                 double ycb = 0.0;
 #pragma unroll
@@ -2860,27 +2912,45 @@ __global__ __launch_bounds__(kBlock) void k_adj_gather(MeshView<double> m, Phys 
     if (c >= m.NI) return;
     const int64_t N = m.N, NI = m.NI, NG = N - NI;
     const int nc = NE + ph.ns;
-    int64_t nb[KM];
-    int mk[KM];
-    double from_ghost[KM];  // dU_ghost / dU_cell: +1 (OUTFLOW copy), -1 (enforceAtFace inflow), 0 otherwise
+    // the contribution its neighbour across slot k wrote for the cell (its mirror slot); padding slots and ghosts read
+    // the cell's own slot 0 and count it zero times, so that the slots' loads are in flight together, and with the next
+    // component's
+    const double* __restrict__ from[KM];
+    double count[KM];
+    int32_t nb[KM];
+    bool any_bnd = false;
 #pragma unroll
     for (int k = 0; k < KM; k++) {
-        const int32_t e = m.snbr[k * NI + c];
-        nb[k] = e;
-        mk[k] = b.mirror[k * NI + c];
-        const int gk = e >= NI ? slot_kind[ghost_slot[e - NI]] : ABL_FV_BC_NONE;
-        from_ghost[k] = gk == ABL_FV_BC_OUTFLOW ? 1.0 : (gk == kBcInflowAtFace ? -1.0 : 0.0);
+        nb[k] = m.snbr[k * NI + c];
+        const int mk = b.mirror[k * NI + c];
+        const bool inner = nb[k] >= 0 && nb[k] < NI;
+        any_bnd |= nb[k] >= NI;
+        from[k] = b.contrib + (inner ? (int64_t)mk * nc * NI + nb[k] : c);
+        count[k] = inner ? 1.0 : 0.0;
     }
-    for (int p = 0; p < nc; p++) {
-        double acc = b.Uself[(int64_t)p * NI + c];
+    double own, in[KM];
+    auto load = [&](int p) {
+        own = b.Uself[(int64_t)p * NI + c];
 #pragma unroll
-        for (int k = 0; k < KM; k++) {
-            if (nb[k] < 0) continue;
-            if (nb[k] < NI)
-                acc += b.contrib[((int64_t)mk[k] * nc + p) * NI + nb[k]];
-            else if (from_ghost[k] != 0.0)
-                acc += from_ghost[k] * b.Ughost[(int64_t)p * NG + (nb[k] - NI)];
-        }
+        for (int k = 0; k < KM; k++) in[k] = from[k][(int64_t)p * NI];
+    };
+    load(0);
+    for (int p = 0; p < nc; p++) {
+        double acc = own, v[KM];
+#pragma unroll
+        for (int k = 0; k < KM; k++) v[k] = in[k];
+        if (p + 1 < nc) load(p + 1);
+#pragma unroll
+        for (int k = 0; k < KM; k++) acc += count[k] * v[k];
+        if (any_bnd)
+#pragma unroll
+            for (int k = 0; k < KM; k++) {
+                if (nb[k] < NI) continue;
+                // dU_ghost / dU_cell: +1 (OUTFLOW copy), -1 (enforceAtFace inflow), 0 otherwise
+                const int gk = slot_kind[ghost_slot[nb[k] - NI]];
+                const double g = b.Ughost[(int64_t)p * NG + (nb[k] - NI)];
+                acc += gk == ABL_FV_BC_OUTFLOW ? g : (gk == kBcInflowAtFace ? -g : 0.0);
+            }
         Ub[(int64_t)p * N + c] = acc;
     }
 }
@@ -3056,9 +3126,20 @@ using AdjFacesKernel = void (*)(MeshView<double>, Phys, const double*, const dou
                                 const double*, AdjBufs);
 using AdjGatherKernel = void (*)(MeshView<double>, Phys, const int32_t*, const int32_t*, AdjBufs, double*);
 template <int DIM, int KM>
-void pick_adj_k(bool rusanov, AdjFacesKernel& fk, AdjCellsKernel& ce, AdjCellsKernel& cs, AdjGatherKernel& gk) {
+void pick_adj_k(bool rusanov, bool recon, bool visc, bool tab, AdjFacesKernel& fk, AdjCellsKernel& ce,
+                AdjCellsKernel& cs, AdjGatherKernel& gk) {
     fk = rusanov ? k_adj_face_rev<DIM, true> : k_adj_face_rev<DIM, false>;
-    ce = k_adj_cells_e<DIM, KM>;
+    auto cells = [&](auto table) {
+        constexpr bool TAB = decltype(table)::value;
+        ce = recon ? (visc ? k_adj_cells_e<DIM, KM, true, true, TAB> : k_adj_cells_e<DIM, KM, true, false, TAB>)
+                   : k_adj_cells_e<DIM, KM, false, true, TAB>;
+    };
+    if constexpr (kSlotRows<DIM, KM>) {
+        if (tab) cells(std::true_type());
+        else cells(std::false_type());
+    } else {
+        cells(std::false_type());
+    }
     cs = k_adj_cells_s<DIM, KM>;
     gk = k_adj_gather<DIM, KM>;
 }
@@ -3101,12 +3182,12 @@ GradKernelT<G> pick_gradients_k(bool recon, bool visc, int lim) {
 // Compile-time slot width of the cell -> face table: 4 (quads, tets), 6 (hexes) or 8.
 inline int slot_width(int K) { return K <= 4 ? 4 : (K <= 6 ? 6 : 8); }
 template <int DIM>
-void pick_adj(bool rusanov, int K, AdjFacesKernel& fk, AdjCellsKernel& ce, AdjCellsKernel& cs,
+void pick_adj(bool rusanov, bool recon, bool visc, bool tab, int K, AdjFacesKernel& fk, AdjCellsKernel& ce, AdjCellsKernel& cs,
               AdjGatherKernel& gk) {
     switch (slot_width(K)) {
-        case 4: pick_adj_k<DIM, 4>(rusanov, fk, ce, cs, gk); break;
-        case 6: pick_adj_k<DIM, 6>(rusanov, fk, ce, cs, gk); break;
-        default: pick_adj_k<DIM, 8>(rusanov, fk, ce, cs, gk); break;
+        case 4: pick_adj_k<DIM, 4>(rusanov, recon, visc, tab, fk, ce, cs, gk); break;
+        case 6: pick_adj_k<DIM, 6>(rusanov, recon, visc, tab, fk, ce, cs, gk); break;
+        default: pick_adj_k<DIM, 8>(rusanov, recon, visc, tab, fk, ce, cs, gk); break;
     }
 }
 template <typename G, int DIM>
@@ -4117,6 +4198,9 @@ extern "C" int abl_fv_create(const abl_fv_mesh_desc* mesh, const abl_fv_physics_
         const int lim = p.limiter == ABL_FV_LIMITER_NONE ? abl::kLimNone
                         : p.limiter == ABL_FV_LIMITER_BARTH_JESPERSEN ? abl::kLimBJ : abl::kLimPetsc;
         const bool species = p.n_species > 0;
+        // the adjoint takes the face vectors of the reconstruction from the limiter geometry: without a limiter they are
+        // kept too
+        const int lim_geometry = lim == abl::kLimNone && s->recon && form == ABL_FV_FORM_FP64 ? abl::kLimBJ : lim;
         // geometry tables of meshes with few distinct face and slot records (else every face and slot keeps its own)
         std::vector<uint16_t> face_rows;
         std::vector<double> face_table;  // 4 words of fna, 2 dim of fdx
@@ -4130,8 +4214,8 @@ extern "C" int abl_fv_create(const abl_fv_mesh_desc* mesh, const abl_fv_physics_
             s->frow.upload(face_rows);
         abl::SlotRows<double> slots;
         abl::SlotRows<float> slots_f;
-        s->slot_rows = form == ABL_FV_FORM_FP64 ? abl::build_slot_rows<double>(L, abl::slot_width(L.K), lim, slots)
-                                                : abl::build_slot_rows<float>(L, abl::slot_width(L.K), lim, slots_f);
+        s->slot_rows = form == ABL_FV_FORM_FP64 ? abl::build_slot_rows<double>(L, abl::slot_width(L.K), lim_geometry, slots)
+                                                : abl::build_slot_rows<float>(L, abl::slot_width(L.K), lim_geometry, slots_f);
         if (s->slot_rows) {
             s->srow.upload(form == ABL_FV_FORM_FP64 ? slots.row : slots_f.row);
             s->slot_stride = form == ABL_FV_FORM_FP64 ? slots.stride : slots_f.stride;
@@ -4179,7 +4263,7 @@ extern "C" int abl_fv_create(const abl_fv_mesh_desc* mesh, const abl_fv_physics_
             s->fna.upload(face_array(L.fna, 0, 4));
             s->fdx.upload(face_array(L.fdx, 4, 2 * L.dim));
             abl::SlotGeometry<double> sg;
-            abl::build_slot_geometry<double>(L, abl::slot_width(L.K), lim, !s->slot_rows, sg);
+            abl::build_slot_geometry<double>(L, abl::slot_width(L.K), lim_geometry, !s->slot_rows, sg);
             s->stab.upload(slots.table);
             s->snbr.upload(sg.nbr);
             s->sw.upload(sg.w);
@@ -4199,7 +4283,7 @@ extern "C" int abl_fv_create(const abl_fv_mesh_desc* mesh, const abl_fv_physics_
             s->fna_f.upload(to_f(face_array(L.fna, 0, 4)));
             s->fdx_f.upload(to_f(face_array(L.fdx, 4, 2 * L.dim)));
             abl::SlotGeometry<float> sg;
-            abl::build_slot_geometry<float>(L, abl::slot_width(L.K), lim, !s->slot_rows, sg);
+            abl::build_slot_geometry<float>(L, abl::slot_width(L.K), lim_geometry, !s->slot_rows, sg);
             s->stab_f.upload(slots_f.table);
             s->snbr.upload(sg.nbr);
             s->sw_f.upload(sg.w);
@@ -4257,13 +4341,13 @@ extern "C" int abl_fv_create(const abl_fv_mesh_desc* mesh, const abl_fv_physics_
                 s->vjp_faces = abl::pick_vjp_faces<3>(rus);
                 s->vjp_gather = abl::pick_vjp_gather<3>(L.K);
                 s->vjp_theta_kernel = abl::pick_vjp_theta<3>(rus);
-                abl::pick_adj<3>(rus, L.K, s->adj_faces, s->adj_cells_e, s->adj_cells_s, s->adj_gather);
+                abl::pick_adj<3>(rus, s->recon, s->visc, s->slot_rows, L.K, s->adj_faces, s->adj_cells_e, s->adj_cells_s, s->adj_gather);
             } else {
                 s->vjp_kernel = abl::pick_vjp<2>(rus, L.K);
                 s->vjp_faces = abl::pick_vjp_faces<2>(rus);
                 s->vjp_gather = abl::pick_vjp_gather<2>(L.K);
                 s->vjp_theta_kernel = abl::pick_vjp_theta<2>(rus);
-                abl::pick_adj<2>(rus, L.K, s->adj_faces, s->adj_cells_e, s->adj_cells_s, s->adj_gather);
+                abl::pick_adj<2>(rus, s->recon, s->visc, s->slot_rows, L.K, s->adj_faces, s->adj_cells_e, s->adj_cells_s, s->adj_gather);
             }
             if (s->recon || s->visc) {
                 // mirror slots: for slot k of cell c, the slot of the same face in the neighbour's list
