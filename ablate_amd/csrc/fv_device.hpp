@@ -80,7 +80,14 @@ struct MeshView {
     const uint16_t* __restrict__ srow;  // [KM][NI]
     const G* __restrict__ stab;         // [rows][sstride]
     int sstride, saux;
+    // Not null: every kernel of the right-hand side returns at once when *halt is set (the device-side time loop
+    // enqueues steps ahead of the one that ends it).
+    const int32_t* halt;
 };
+template <typename MV>
+__device__ inline bool halted(const MV& m) {
+    return m.halt && *m.halt;
+}
 // Slot tables exist for quads and hexes only (the kernels of the other cell shapes have no table path).
 template <int DIM, int KM>
 constexpr bool kSlotRows = DIM == 2 ? KM == 4 : KM == 6;

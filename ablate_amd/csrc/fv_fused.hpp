@@ -287,6 +287,7 @@ __global__ __launch_bounds__(256) void k_fused(MeshView<double> m, Phys ph, cons
     using SD = SideData<DIM, VISC>;
     constexpr int NE = DIM + 2;
     extern __shared__ double lds[];
+    if (halted(m)) return;
     const int T = fv.T, nem = fv.nem, nfm = fv.nfm;
     double* rec = lds;                    // [RW][T]
     double* hal = rec + FL::RW * T;       // [HW][nem]
@@ -497,6 +498,7 @@ __global__ __launch_bounds__(kMarchBlock) __attribute__((amdgpu_waves_per_eu(2))
     using FL = FusedLayout<DIM, RECON, VISC>;
     constexpr int NE = DIM + 2;
     extern __shared__ double lds[];
+    if (halted(m)) return;
     const int T = mv.T, nem = mv.nem, nfm = mv.nfm;
     double* rec = lds;                      // [2][RW][T]
     double* hal = rec + 2 * FL::RW * T;     // [HW][nem]

@@ -49,29 +49,38 @@ constexpr int kCuLdsBytes = 160 * 1024;  // LDS of one gfx950 compute unit
 
 // ============================================================================================ kernels
 
-// Ghost rows of the state, and (Z not null) zeros in the ghost rows of the result, which every ghost cell's one
-// boundary face covers.  One lane per boundary face and component (blockIdx.y), the cells straight from bcell: two
-// dependent loads deep.  A lane per face that walked the components took 22 us for 62208 faces of 15 components (each
-// store to U may alias the next component's load), and the zeros were a launch of their own.
-__global__ __launch_bounds__(kBlock) void k_ghost_fill(int64_t nb, const int2* __restrict__ bcell,
-                                                       const int32_t* __restrict__ bslot, int64_t N, int nc,
-                                                       const int32_t* __restrict__ slot_kind,
-                                                       const double* __restrict__ slot_state, double* __restrict__ U,
-                                                       double* __restrict__ Z) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nb) return;
-    const int p = blockIdx.y;
-    const int2 cells = bcell[i];  // interior, ghost
-    const int32_t s = bslot[i];
-    const int kind = slot_kind[s];
-    const double ui = U[(int64_t)p * N + cells.x], state = slot_state[s * nc + p];
-    const int64_t g = (int64_t)p * N + cells.y;
-    if (Z) Z[g] = 0.0;
+// Boundary faces as the ghost fill takes them.
+struct GhostView {
+    int64_t nb, N;
+    int nc;
+    const int2* __restrict__ bcell;  // interior and ghost cell
+    const int32_t* __restrict__ bslot;
+    const int32_t* __restrict__ slot_kind;
+    const double* __restrict__ slot_state;
+};
+// Component p of boundary face i: the ghost row of U from its condition, and zero in that of Z (unless null).
+__device__ inline void ghost_fill(const GhostView& g, int64_t i, int p, double* __restrict__ U, double* __restrict__ Z) {
+    const int2 cells = g.bcell[i];
+    const int32_t s = g.bslot[i];
+    const int kind = g.slot_kind[s];
+    const double ui = U[(int64_t)p * g.N + cells.x], state = g.slot_state[s * g.nc + p];
+    const int64_t o = (int64_t)p * g.N + cells.y;
+    if (Z) Z[o] = 0.0;
     if (kind == ABL_FV_BC_GHOST) return;  // caller-filled: the ghost rows are inputs
     double v = ui;  // OUTFLOW: zero-gradient extrapolation
     if (kind == ABL_FV_BC_INFLOW) v = state;
     if (kind == kBcInflowAtFace) v = 2.0 * state - ui;  // essentialGhost.cpp:17-20
-    U[g] = v;
+    U[o] = v;
+}
+// Ghost rows of the state, and (Z not null) zeros in the ghost rows of the result, which every ghost cell's one
+// boundary face covers.  One lane per boundary face and component (blockIdx.y): two dependent loads deep.  A lane per
+// face that walked the components took 22 us for 62208 faces of 15 components (each store to U may alias the next
+// component's load), and the zeros were a launch of their own.
+__global__ __launch_bounds__(kBlock) void k_ghost_fill(GhostView g, double* __restrict__ U, double* __restrict__ Z,
+                                                       const int32_t* halt) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= g.nb || (halt && *halt)) return;
+    ghost_fill(g, i, blockIdx.y, U, Z);
 }
 
 // Aux values of a cell: temperature (PerfectGas TemperatureFunction, perfectGas.cpp:76-86) and velocity.
@@ -206,7 +215,7 @@ __device__ __forceinline__ void gradients_body(MeshView<G> m, Phys ph, const dou
     constexpr int NE = DIM + 2;
     constexpr int NA = DIM + 1;
     const int64_t c = xcd_cell_index();
-    if (c >= m.NI) return;
+    if (c >= m.NI || halted(m)) return;
     const int64_t N = m.N, NI = m.NI;
     const G* __restrict__ wa_arr = m.swa ? m.swa : m.sw;
     int32_t nb[KM];
@@ -477,7 +486,7 @@ __device__ __forceinline__ void species_body(MeshView<G> m, Phys ph, const doubl
                                              G* __restrict__ gradC, G* __restrict__ gradA) {
     constexpr int NE = DIM + 2;
     const int64_t c = xcd_cell_index();
-    if (c >= m.NI) return;
+    if (c >= m.NI || halted(m)) return;
     const int64_t N = m.N, NI = m.NI;
     const bool recon = ph.recon != 0;
     const bool aux = ph.sdiff != 0;
@@ -854,7 +863,7 @@ __global__ __launch_bounds__(kBlock) void k_flux(MeshView<double> m, Phys ph, co
     constexpr int NE = DIM + 2;
     using SD = SideData<DIM, VISC>;
     const int64_t c = xcd_cell_index();
-    if (c >= m.NI) return;
+    if (c >= m.NI || halted(m)) return;
     const int64_t N = m.N, F = m.F, NI = m.NI;
     double acc[NE];
 #pragma unroll
@@ -969,7 +978,7 @@ __device__ __forceinline__ void face_flux_body(MeshView<double> m, Phys ph, cons
     constexpr int NW = NE + (kCoefGather<RECON, VISC, SPECIES> ? 2 : 0);
     constexpr int FS = (NW + 1) & ~1;
     const int64_t f = xcd_cell_index();
-    if (f >= m.F) return;
+    if (f >= m.F || halted(m)) return;
     double flux[FS];
     eval_face<DIM, RECON, VISC, SPECIES, true>(m, ph, U, gradC, gradA, rec, face_ref(m, f), flux, Fs + 2 * f, 2 * m.F);
     if (FS > NW) flux[FS - 1] = 0.0;
@@ -1006,6 +1015,7 @@ __global__ __launch_bounds__(kTileMax) void k_tile_flux(MeshView<double> m, Phys
                                                         double* __restrict__ R, int accumulate) {
     constexpr int NE = DIM + 2;
     extern __shared__ double lds[];
+    if (halted(m)) return;
     double* le = lds;              // [NE][nfm]
     double* ls = lds + NE * nfm;   // [ns][nfm]
     const int64_t t = xcd_block_index();
@@ -1068,7 +1078,7 @@ __global__ __launch_bounds__(kBlock) void k_gather(MeshView<double> m, int ns, c
     constexpr int NE = DIM + 2;
     constexpr int FS = (NE + 1) & ~1;
     const int64_t c = xcd_cell_index();
-    if (c >= m.NI) return;
+    if (c >= m.NI || halted(m)) return;
     const int64_t N = m.N, F = m.F, NI = m.NI;
     int64_t fk[KM];
     double sg[KM];
@@ -1135,7 +1145,7 @@ __global__ __launch_bounds__(kBlock) void k_gather_coef(MeshView<double> m, int 
     constexpr int NE = DIM + 2;
     constexpr int FS = (NE + 3) & ~1;
     const int64_t c = xcd_cell_index();
-    if (c >= m.NI) return;
+    if (c >= m.NI || halted(m)) return;
     const int64_t N = m.N, NI = m.NI;
     int32_t e[KM], nb[KM];
 #pragma unroll
@@ -1616,7 +1626,7 @@ __global__ __launch_bounds__(kBlock) void k_flux_mixed(MeshView<float> m, Phys p
                                                        int accumulate) {
     constexpr int NE = DIM + 2;
     const int64_t c = xcd_cell_index();
-    if (c >= m.NI) return;
+    if (c >= m.NI || halted(m)) return;
     const int64_t N = m.N, NI = m.NI;
     double acc[NE];
 #pragma unroll
@@ -1657,6 +1667,7 @@ __global__ __launch_bounds__(kTileMax) void k_tile_flux_mixed(MeshView<float> m,
                                                               double* __restrict__ R, int accumulate) {
     constexpr int NE = DIM + 2;
     extern __shared__ double lds_d[];
+    if (halted(m)) return;
     float* lf = reinterpret_cast<float*>(lds_d);
     const int nrow = NE + (SPECIES ? ph.ns : 0);
     const int64_t t = xcd_block_index();
@@ -1710,7 +1721,7 @@ __global__ __launch_bounds__(kBlock) void k_face_flux_mixed(MeshView<float> m, P
                                                             int nrow) {
     constexpr int NE = DIM + 2;
     const int64_t f = xcd_cell_index();
-    if (f >= m.F) return;
+    if (f >= m.F || halted(m)) return;
     const int64_t F = m.F;
     float dFL[NE], dFR[NE];
     mixed_face<DIM, RECON, VISC, SPECIES, RUS>(m, ph, U, rec, gS, gY, face_ref(m, f), dFL, dFR, Fm + NE * F + f,
@@ -1728,7 +1739,7 @@ template <int DIM, int KM>
 __global__ __launch_bounds__(kBlock) void k_gather_mixed(MeshView<float> m, int nrow, const float* __restrict__ Fm,
                                                          double* __restrict__ R, int accumulate) {
     const int64_t c = xcd_cell_index();
-    if (c >= m.NI) return;
+    if (c >= m.NI || halted(m)) return;
     const int64_t N = m.N, NI = m.NI;
     int64_t off[KM];
     double sg[KM];
@@ -3438,35 +3449,127 @@ __device__ inline double block_min(double v) {
     for (int i = 1; i < (int)(blockDim.x >> 6); i++) m = fmin(m, wmin[i]);
     return m;
 }
+// CFL step of cell c, the reference's starting minimum (utilities::Constants::large) past the end.
+__device__ inline double cfl_of(const double* __restrict__ U, const double* __restrict__ rmin, int64_t N, int64_t NI, int dim,
+                                const Phys& ph, double cfl, double alpha, int64_t c) {
+    if (c >= NI) return 1e10;
+    const double rho = U[c];
+    double ke = 0.0, velSum = 0.0;
+    for (int d = 0; d < dim; d++) {
+        const double v = U[(kRhoU + d) * N + c] / rho;
+        ke += v * v;
+        velSum += fabs(U[(kRhoU + d) * N + c]) / rho;
+    }
+    ke *= 0.5;
+    const double T = (U[kRhoE * N + c] / rho - ke) / ph.cv;
+    const double p = ph.R * rho * T;
+    const double a = sqrt(ph.gamma * p / rho);
+    return cfl * (2.0 * rmin[c]) / (a / alpha + velSum);
+}
 __global__ __launch_bounds__(kBlock) void k_cfl_partial(const double* __restrict__ U, const double* __restrict__ rmin,
                                                         int64_t N, int64_t NI, int dim, Phys ph, double cfl,
                                                         double alpha, double* __restrict__ partial) {
     const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    double dt = 1e10;  // utilities::Constants::large, the reference's starting minimum
-    if (c < NI) {
-        const double rho = U[c];
-        double ke = 0.0, velSum = 0.0;
-        for (int d = 0; d < dim; d++) {
-            const double v = U[(kRhoU + d) * N + c] / rho;
-            ke += v * v;
-            velSum += fabs(U[(kRhoU + d) * N + c]) / rho;
-        }
-        ke *= 0.5;
-        const double T = (U[kRhoE * N + c] / rho - ke) / ph.cv;
-        const double p = ph.R * rho * T;
-        const double a = sqrt(ph.gamma * p / rho);
-        dt = cfl * (2.0 * rmin[c]) / (a / alpha + velSum);
-    }
-    const double m = block_min(dt);
+    const double m = block_min(cfl_of(U, rmin, N, NI, dim, ph, cfl, alpha, c));
     if (threadIdx.x == 0) partial[blockIdx.x] = m;
+}
+__device__ inline double partial_min(const double* __restrict__ partial, int64_t n) {
+    double v = 1e10;
+    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) v = fmin(v, partial[i]);
+    return block_min(v);
 }
 __global__ __launch_bounds__(kBlock) void k_min_final(const double* __restrict__ partial, int64_t n,
                                                       double* __restrict__ out) {
-    double v = 1e10;
-    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) v = fmin(v, partial[i]);
-    const double m = block_min(v);
+    const double m = partial_min(partial, n);
     if (threadIdx.x == 0) out[0] = m;
 }
+
+// Forward-Euler loop on the device (abl_fv_ts_euler): the clock of the run.  `halt` ends it: the maximum time or step
+// count is reached, or (bad) the step size is not positive.
+struct TsClock {
+    double t, dt;
+    int64_t steps;
+    int32_t halt, bad;
+};
+struct TsLimits {
+    double max_time, safety;
+    int64_t max_steps;
+};
+// The physics step of U_n (TSStep_Euler asks the adaptor while the solution still holds U_n) and U += dt R, one lane per
+// cell: the state is read once for both, and R before the block's minimum.
+template <int DIM>
+__global__ __launch_bounds__(kBlock) void k_ts_update(double* __restrict__ U, const double* __restrict__ R,
+                                                      const double* __restrict__ rmin, int64_t N, int64_t NI, int nc,
+                                                      Phys ph, double cfl, double alpha,
+                                                      const TsClock* __restrict__ clock, double* __restrict__ partial) {
+    constexpr int NE = DIM + 2;
+    if (clock->halt) return;
+    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, ca = c < NI ? c : NI - 1;
+    const double dt = clock->dt;
+    double r[NE];
+#pragma unroll
+    for (int p = 0; p < NE; p++) r[p] = R[p * N + ca];
+    const double m = block_min(cfl_of(U, rmin, N, NI, DIM, ph, cfl, alpha, c));
+    if (threadIdx.x == 0) partial[blockIdx.x] = m;
+    if (c >= NI) return;
+#pragma unroll
+    for (int p = 0; p < NE; p++) U[p * N + c] += dt * r[p];
+#pragma unroll 4
+    for (int p = NE; p < nc; p++) U[p * N + c] += dt * R[p * N + c];
+}
+// End of a step: the clock after it, with `physics` the step of U_n: the next step size and TSAdaptChoose with
+// ts_exact_final_time matchstep (matchstep factors 0.01, 2).
+__device__ inline TsClock ts_advance(TsClock k, double physics, const TsLimits& lim) {
+    double next = lim.safety * fmin(1e10, physics);
+    const double t_end = k.t + k.dt, remaining = lim.max_time - t_end;
+    if (t_end < lim.max_time && t_end + next > lim.max_time) next = remaining;
+    if (t_end < lim.max_time && t_end + next < lim.max_time && next * 2.0 > remaining) next = remaining / 2.0;
+    if (t_end < lim.max_time && t_end + next < lim.max_time && next * 1.01 > remaining) next = remaining;
+    k.t = t_end;
+    k.dt = next;
+    k.steps++;
+    return k;
+}
+__device__ inline TsClock ts_check(TsClock k, const TsLimits& lim) {
+    const bool more = k.t < lim.max_time && k.steps < lim.max_steps;
+    k.bad = more && !(k.dt > 0.0);
+    k.halt = !more || k.bad;
+    return k;
+}
+// The start of the run (first: t0 and min(dt0, physics step), AdaptPhysics::AdaptInitializer) or the end of a step, from
+// clock `from` into clock `to` and its pinned host copy; `partial` holds the block minima of the physics step.
+__global__ __launch_bounds__(kBlock) void k_ts_advance(const double* __restrict__ partial, int64_t n, TsLimits lim, bool first,
+                                                       double t0, double dt0, const TsClock* __restrict__ from,
+                                                       TsClock* __restrict__ to, TsClock* __restrict__ host) {
+    const double physics = partial_min(partial, n);
+    if (threadIdx.x != 0) return;
+    TsClock k;
+    if (first) {
+        const double p = lim.safety * fmin(1e10, physics);
+        k = ts_check({t0, p < dt0 ? p : dt0, 0, 0, 0}, lim);
+    } else {
+        k = *from;
+        if (!k.halt) k = ts_check(ts_advance(k, physics, lim), lim);
+    }
+    *to = k;
+    *host = k;
+}
+// The end of a step and the ghost rows of the next one in one launch: every block forms the new clock for itself from
+// the few block minima, the first one stores it.  (Clocks alternate, so that no block reads the one being stored.)
+__global__ __launch_bounds__(kBlock) void k_ts_advance_ghosts(const double* __restrict__ partial, int64_t n, TsLimits lim,
+                                                              const TsClock* __restrict__ from,
+                                                              TsClock* __restrict__ to, GhostView g,
+                                                              double* __restrict__ U, double* __restrict__ Z) {
+    const double physics = partial_min(partial, n);
+    TsClock k = *from;
+    if (!k.halt) k = ts_check(ts_advance(k, physics, lim), lim);
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *to = k;
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= g.nb || k.halt) return;
+    ghost_fill(g, i, blockIdx.y, U, Z);
+}
+// Block minima that every block of k_ts_advance_ghosts reads again: a few per lane.
+constexpr int64_t kTsGhostPartials = 1024;
 // NavierStokesTransport::ComputeConductionTimeStep and ComputeViscousDiffusionTimeStep
 // (navierStokesTransport.cpp:287-450): per interior cell |f (2 r_min)^2 / alpha| with alpha = k / (rho cv) and
 // |f (2 r_min)^2 / nu| with nu = mu / rho, k and mu of the transport model at the cell temperature (the aux T);
@@ -3710,6 +3813,7 @@ struct abl_fv_solver {
     abl::DevBuf<double> stab;
     abl::DevBuf<float> stab_f;
     int slot_stride = 0, slot_aux = 0;
+    const int32_t* halt = nullptr;  // set while abl_fv_ts_euler enqueues steps (MeshView::halt)
     bool slot_rows = false;
     abl::DevBuf<double> rec;            // cell records of the FP64 form (rec_pair blocks)
     // face fluxes (allocated when that strategy is selected): FP64 euler records [F][FS] and species pairs
@@ -3775,6 +3879,8 @@ struct abl_fv_solver {
     abl::GatherCoefKernel gather_coef = nullptr;  // set for first-order inviscid species (in place of gather_kernel)
     int strategy = ABL_FV_STRATEGY_TILE;
     abl::DevBuf<unsigned long long> counter;
+    abl::DevBuf<abl::TsClock> ts_clock;      // device-side time loop (allocated by its first run): two clocks
+    abl::TsClock* ts_host = nullptr;         // and a pinned host copy
     abl::DevBuf<double> rmin, cfl_partial, cfl_out;  // MIN_CELL_RADIUS per interior cell; CFL reduction scratch
     abl::DevBuf<double> dt_partial;                  // conduction / viscous time-step block minima [2][blocks]
     // PressureGradientScaling attached by abl_fv_set_pgs: its state (alpha in ph.pgs_alpha) and reduction scratch
@@ -3827,6 +3933,7 @@ struct abl_fv_solver {
         pending.clear();
     }
     ~abl_fv_solver() {
+        if (ts_host) (void)hipHostFree(ts_host);
         for (auto& e : pending) {
             (void)hipEventSynchronize(e.stop);
             (void)hipEventDestroy(e.start);
@@ -3856,6 +3963,7 @@ struct abl_fv_solver {
         v.stab = stab.ptr;
         v.sstride = slot_stride;
         v.saux = slot_aux;
+        v.halt = halt;
         return v;
     }
     abl::MeshView<float> view_f() const {
@@ -3880,7 +3988,11 @@ struct abl_fv_solver {
         v.stab = stab_f.ptr;
         v.sstride = slot_stride;
         v.saux = slot_aux;
+        v.halt = halt;
         return v;
+    }
+    abl::GhostView ghost_view() const {
+        return {n_bfaces, host.N, host.nc, bcell.ptr, bslot.ptr, slot_kind.ptr, slot_state.ptr};
     }
     // Face-flux storage of strategy 2 (see the members).
     void ensure_face_flux() {
@@ -4120,9 +4232,8 @@ std::string unset_boundary(abl_fv_handle h) {
 // passes (and their copy back to the host) are skipped.
 // Ghost rows of U from the boundary conditions; zeros in the ghost rows of Z (null: none).
 void fill_ghosts(abl_fv_handle h, hipStream_t st, double* U, double* Z) {
-    const abl::Layout& L = h->host;
-    hipLaunchKernelGGL(abl::k_ghost_fill, dim3(grid_for(h->n_bfaces), (unsigned)L.nc), dim3(abl::kBlock), 0, st,
-                       h->n_bfaces, h->bcell.ptr, h->bslot.ptr, L.N, L.nc, h->slot_kind.ptr, h->slot_state.ptr, U, Z);
+    hipLaunchKernelGGL(abl::k_ghost_fill, dim3(grid_for(h->n_bfaces), (unsigned)h->host.nc), dim3(abl::kBlock), 0, st,
+                       h->ghost_view(), U, Z, h->halt);
 }
 
 bool has_inflow(abl_fv_handle h) {
@@ -4504,6 +4615,98 @@ extern "C" int abl_fv_set_boundary(abl_fv_handle h, int32_t slot, const abl_fv_b
     return 0;
 }
 
+namespace {
+// The kernels of one right-hand side after the ghost fill.
+void launch_rhs(abl_fv_handle h, double* U, double* R, int32_t accumulate, hipStream_t st) {
+    const abl::Layout& L = h->host;
+    const dim3 grid(grid_for(L.NI)), block(abl::kBlock);
+    if (h->form == ABL_FV_FORM_MIXED) {
+        const auto vf = h->view_f();
+        if (h->recon || h->visc)
+            h->timed(ABL_FV_PHASE_GRADIENTS, st, [&] {
+                hipLaunchKernelGGL(h->grad_kernel_f, grid, block, 0, st, vf, h->ph, U, nullptr, nullptr,
+                                   (void*)h->recf.ptr);
+            });
+        if (L.ns && (h->recon || h->visc))
+            h->timed(ABL_FV_PHASE_SPECIES_GRADIENTS, st, [&] {
+                hipLaunchKernelGGL(h->species_kernel_f, grid, block, 0, st, vf, h->ph, U, h->gS_f.ptr, h->gY_f.ptr);
+            });
+        if (h->strategy == ABL_FV_STRATEGY_FACE_FLUX) {
+            const int nrow = L.dim + 2 + L.ns;
+            h->timed(ABL_FV_PHASE_FLUX, st, [&] {
+                hipLaunchKernelGGL(h->face_flux_kernel_mixed, dim3(grid_for(L.F)), block, 0, st, vf, h->ph, U,
+                                   h->recf.ptr,
+                                   h->gS_f.ptr, h->gY_f.ptr, h->face_flux_m.ptr, nrow);
+            });
+            h->timed(ABL_FV_PHASE_GATHER, st, [&] {
+                hipLaunchKernelGGL(h->gather_kernel_mixed, grid, block, 0, st, vf, nrow, h->face_flux_m.ptr, R,
+                                   accumulate);
+            });
+        } else if (h->strategy == ABL_FV_STRATEGY_TILE) {
+            h->timed(ABL_FV_PHASE_FLUX, st, [&] {
+                hipLaunchKernelGGL(h->tile_kernel_mixed, dim3((unsigned)h->tile_n), dim3(h->tile_threads), h->tile_lds, st,
+                                   vf, h->ph, U, h->recf.ptr, h->gS_f.ptr, h->gY_f.ptr, h->tile_start.ptr,
+                                   h->tile_faces.ptr, h->tile_slot.ptr, h->tile_T, h->tile_nfm, R, accumulate);
+            });
+        } else {
+            h->timed(ABL_FV_PHASE_FLUX, st, [&] {
+                hipLaunchKernelGGL(h->flux_kernel_mixed, grid, block, 0, st, vf, h->ph, U, h->recf.ptr, R,
+                                   accumulate);
+            });
+        }
+    } else if (h->strategy == ABL_FV_STRATEGY_MARCH) {
+        h->timed(ABL_FV_PHASE_FLUX, st, [&] {
+            hipLaunchKernelGGL(h->march_kernel, dim3((unsigned)h->mr_nseq), dim3(abl::kMarchBlock), h->mr_lds, st,
+                               h->view(), h->ph, U, h->march_view(), R, accumulate);
+        });
+    } else if (h->strategy == ABL_FV_STRATEGY_FUSED) {
+        h->timed(ABL_FV_PHASE_FLUX, st, [&] {
+            hipLaunchKernelGGL(h->fused_kernel, dim3((unsigned)h->fu_n), dim3(256), h->fu_lds, st, h->view(), h->ph, U,
+                               h->fused_view(), R, accumulate);
+        });
+    } else {
+    const auto v = h->view();
+    if (h->recon || h->visc) {
+        h->timed(ABL_FV_PHASE_GRADIENTS, st, [&] {
+            hipLaunchKernelGGL(h->grad_kernel, grid, block, 0, st, v, h->ph, U, h->gradC.ptr, h->gradA.ptr,
+                               (void*)h->rec.ptr);
+        });
+        if (L.ns)
+            h->timed(ABL_FV_PHASE_SPECIES_GRADIENTS, st, [&] {
+                hipLaunchKernelGGL(h->species_kernel, grid, block, 0, st, v, h->ph, U, h->gradC.ptr, h->gradA.ptr);
+            });
+    }
+    if (h->strategy == ABL_FV_STRATEGY_TILE) {
+        h->timed(ABL_FV_PHASE_FLUX, st, [&] {
+            hipLaunchKernelGGL(h->tile_kernel, dim3((unsigned)h->tile_n), dim3(h->tile_threads), h->tile_lds, st, v, h->ph,
+                               U, h->gradC.ptr, h->gradA.ptr, h->rec.ptr, h->tile_start.ptr,
+                               h->tile_faces.ptr,
+                               h->tile_slot.ptr, h->tile_T, h->tile_nfm, R, accumulate);
+        });
+    } else if (h->strategy == ABL_FV_STRATEGY_FACE_FLUX) {
+        h->timed(ABL_FV_PHASE_FLUX, st, [&] {
+            hipLaunchKernelGGL(h->face_flux_kernel, dim3(grid_for(L.F)), block, 0, st, v, h->ph, U, h->gradC.ptr,
+                               h->gradA.ptr, h->rec.ptr, h->face_flux_e.ptr, h->face_flux_s.ptr);
+        });
+        h->timed(ABL_FV_PHASE_GATHER, st, [&] {
+            if (h->gather_coef)
+                hipLaunchKernelGGL(h->gather_coef, grid, block, 0, st, v, L.ns, U, h->face_flux_e.ptr, R,
+                                   accumulate);
+            else
+                hipLaunchKernelGGL(h->gather_kernel, grid, block, 0, st, v, L.ns, h->face_flux_e.ptr,
+                                   h->face_flux_s.ptr, R, accumulate);
+        });
+    } else {
+        h->timed(ABL_FV_PHASE_FLUX, st, [&] {
+            hipLaunchKernelGGL(h->flux_kernel, grid, block, 0, st, v, h->ph, U, h->gradC.ptr, h->gradA.ptr,
+                               h->rec.ptr, R, accumulate);
+        });
+    }
+    }
+    HIP_CHECK(hipGetLastError());
+}
+}  // namespace
+
 extern "C" int abl_fv_rhs(abl_fv_handle h, double time, double* U, double* R, int32_t accumulate, abl_fv_stream stream) {
     (void)time;  // constant-state conditions do not depend on it; caller-filled ghosts were evaluated at it
     if (!h || !U || !R) return fail(h, "abl_fv_rhs: null argument");
@@ -4513,95 +4716,9 @@ extern "C" int abl_fv_rhs(abl_fv_handle h, double time, double* U, double* R, in
     }
     try {
         hipStream_t st = (hipStream_t)stream;
-        const abl::Layout& L = h->host;
-        if (h->n_bfaces) {
+        if (h->n_bfaces)
             h->timed(ABL_FV_PHASE_GHOST, st, [&] { fill_ghosts(h, st, U, accumulate ? nullptr : R); });
-        }
-        const dim3 grid(grid_for(L.NI)), block(abl::kBlock);
-        if (h->form == ABL_FV_FORM_MIXED) {
-            const auto vf = h->view_f();
-            if (h->recon || h->visc)
-                h->timed(ABL_FV_PHASE_GRADIENTS, st, [&] {
-                    hipLaunchKernelGGL(h->grad_kernel_f, grid, block, 0, st, vf, h->ph, U, nullptr, nullptr,
-                                       (void*)h->recf.ptr);
-                });
-            if (L.ns && (h->recon || h->visc))
-                h->timed(ABL_FV_PHASE_SPECIES_GRADIENTS, st, [&] {
-                    hipLaunchKernelGGL(h->species_kernel_f, grid, block, 0, st, vf, h->ph, U, h->gS_f.ptr, h->gY_f.ptr);
-                });
-            if (h->strategy == ABL_FV_STRATEGY_FACE_FLUX) {
-                const int nrow = L.dim + 2 + L.ns;
-                h->timed(ABL_FV_PHASE_FLUX, st, [&] {
-                    hipLaunchKernelGGL(h->face_flux_kernel_mixed, dim3(grid_for(L.F)), block, 0, st, vf, h->ph, U,
-                                       h->recf.ptr,
-                                       h->gS_f.ptr, h->gY_f.ptr, h->face_flux_m.ptr, nrow);
-                });
-                h->timed(ABL_FV_PHASE_GATHER, st, [&] {
-                    hipLaunchKernelGGL(h->gather_kernel_mixed, grid, block, 0, st, vf, nrow, h->face_flux_m.ptr, R,
-                                       accumulate);
-                });
-            } else if (h->strategy == ABL_FV_STRATEGY_TILE) {
-                h->timed(ABL_FV_PHASE_FLUX, st, [&] {
-                    hipLaunchKernelGGL(h->tile_kernel_mixed, dim3((unsigned)h->tile_n), dim3(h->tile_threads), h->tile_lds, st,
-                                       vf, h->ph, U, h->recf.ptr, h->gS_f.ptr, h->gY_f.ptr, h->tile_start.ptr,
-                                       h->tile_faces.ptr, h->tile_slot.ptr, h->tile_T, h->tile_nfm, R, accumulate);
-                });
-            } else {
-                h->timed(ABL_FV_PHASE_FLUX, st, [&] {
-                    hipLaunchKernelGGL(h->flux_kernel_mixed, grid, block, 0, st, vf, h->ph, U, h->recf.ptr, R,
-                                       accumulate);
-                });
-            }
-        } else if (h->strategy == ABL_FV_STRATEGY_MARCH) {
-            h->timed(ABL_FV_PHASE_FLUX, st, [&] {
-                hipLaunchKernelGGL(h->march_kernel, dim3((unsigned)h->mr_nseq), dim3(abl::kMarchBlock), h->mr_lds, st,
-                                   h->view(), h->ph, U, h->march_view(), R, accumulate);
-            });
-        } else if (h->strategy == ABL_FV_STRATEGY_FUSED) {
-            h->timed(ABL_FV_PHASE_FLUX, st, [&] {
-                hipLaunchKernelGGL(h->fused_kernel, dim3((unsigned)h->fu_n), dim3(256), h->fu_lds, st, h->view(), h->ph, U,
-                                   h->fused_view(), R, accumulate);
-            });
-        } else {
-        const auto v = h->view();
-        if (h->recon || h->visc) {
-            h->timed(ABL_FV_PHASE_GRADIENTS, st, [&] {
-                hipLaunchKernelGGL(h->grad_kernel, grid, block, 0, st, v, h->ph, U, h->gradC.ptr, h->gradA.ptr,
-                                   (void*)h->rec.ptr);
-            });
-            if (L.ns)
-                h->timed(ABL_FV_PHASE_SPECIES_GRADIENTS, st, [&] {
-                    hipLaunchKernelGGL(h->species_kernel, grid, block, 0, st, v, h->ph, U, h->gradC.ptr, h->gradA.ptr);
-                });
-        }
-        if (h->strategy == ABL_FV_STRATEGY_TILE) {
-            h->timed(ABL_FV_PHASE_FLUX, st, [&] {
-                hipLaunchKernelGGL(h->tile_kernel, dim3((unsigned)h->tile_n), dim3(h->tile_threads), h->tile_lds, st, v, h->ph,
-                                   U, h->gradC.ptr, h->gradA.ptr, h->rec.ptr, h->tile_start.ptr,
-                                   h->tile_faces.ptr,
-                                   h->tile_slot.ptr, h->tile_T, h->tile_nfm, R, accumulate);
-            });
-        } else if (h->strategy == ABL_FV_STRATEGY_FACE_FLUX) {
-            h->timed(ABL_FV_PHASE_FLUX, st, [&] {
-                hipLaunchKernelGGL(h->face_flux_kernel, dim3(grid_for(L.F)), block, 0, st, v, h->ph, U, h->gradC.ptr,
-                                   h->gradA.ptr, h->rec.ptr, h->face_flux_e.ptr, h->face_flux_s.ptr);
-            });
-            h->timed(ABL_FV_PHASE_GATHER, st, [&] {
-                if (h->gather_coef)
-                    hipLaunchKernelGGL(h->gather_coef, grid, block, 0, st, v, L.ns, U, h->face_flux_e.ptr, R,
-                                       accumulate);
-                else
-                    hipLaunchKernelGGL(h->gather_kernel, grid, block, 0, st, v, L.ns, h->face_flux_e.ptr,
-                                       h->face_flux_s.ptr, R, accumulate);
-            });
-        } else {
-            h->timed(ABL_FV_PHASE_FLUX, st, [&] {
-                hipLaunchKernelGGL(h->flux_kernel, grid, block, 0, st, v, h->ph, U, h->gradC.ptr, h->gradA.ptr,
-                                   h->rec.ptr, R, accumulate);
-            });
-        }
-        }
-        HIP_CHECK(hipGetLastError());
+        launch_rhs(h, U, R, accumulate, st);
     } catch (const std::exception& e) {
         return fail(h, std::string("abl_fv_rhs: ") + e.what());
     }
@@ -5068,6 +5185,77 @@ extern "C" int abl_fv_set_pgs_alpha(abl_fv_handle h, double alpha) {
     return 0;
 }
 
+namespace {
+// abl_fv_ts_euler with the CFL step alone.  A step is the right-hand side, k_ts_update and k_ts_advance, enqueued without
+// waiting: the clock lives on the device, and steps enqueued past the end do nothing (their kernels see `halt`).  The
+// host waits once for the first step size and then once per batch, sized from the time left and the last step size.
+// With a wait per step for its size, and separate step-size and update kernels, 150 x 95 quads took 36 us a step.
+int ts_euler_device(abl_fv_handle h, double* U, double* R, double t0, double max_time, double dt0, double safety,
+                    int64_t max_steps, double* t_out, int64_t* steps_out, hipStream_t st) {
+    constexpr int64_t kMaxBatch = 256;
+    struct Halt {  // the kernels of abl_fv_rhs look at the clock only inside this loop
+        abl_fv_handle h;
+        ~Halt() { h->halt = nullptr; }
+    } guard{h};
+    try {
+        const abl::Layout& L = h->host;
+        if (!h->ts_clock.ptr) h->ts_clock.alloc(2);
+        if (!h->ts_host) HIP_CHECK(hipHostMalloc((void**)&h->ts_host, sizeof(abl::TsClock)));
+        const unsigned nb = grid_for(L.NI);
+        const double alpha = h->ph.compact ? h->ph.pgs_alpha : 1.0;
+        const abl::TsLimits lim{max_time, safety, max_steps};
+        const auto update = L.dim == 3 ? abl::k_ts_update<3> : abl::k_ts_update<2>;
+        const bool merged = h->n_bfaces && (int64_t)nb <= abl::kTsGhostPartials;
+        abl::TsClock* clock = h->ts_clock.ptr;  // of the step being enqueued; the other one follows
+        auto other = [&] { return clock == h->ts_clock.ptr ? clock + 1 : h->ts_clock.ptr; };
+        auto advance = [&](bool first) {
+            hipLaunchKernelGGL(abl::k_ts_advance, dim3(1), dim3(abl::kBlock), 0, st, h->cfl_partial.ptr, (int64_t)nb, lim,
+                               first, t0, dt0, clock, other(), h->ts_host);
+            clock = other();
+        };
+        hipLaunchKernelGGL(abl::k_cfl_partial, dim3(nb), dim3(abl::kBlock), 0, st, U, h->rmin.ptr, L.N, L.NI, L.dim, h->ph,
+                           h->phys.cfl, alpha, h->cfl_partial.ptr);
+        advance(true);
+        HIP_CHECK(hipGetLastError());
+        HIP_CHECK(hipStreamSynchronize(st));
+        abl::TsClock k = *h->ts_host;
+        while (!k.halt) {
+            const double left = std::ceil((max_time - k.t) / k.dt) + 1.0;
+            int64_t batch = std::min(max_steps - k.steps, kMaxBatch);
+            if (left < (double)batch) batch = std::max<int64_t>(1, (int64_t)left);
+            for (int64_t i = 0; i < batch; i++) {
+                if (i > 0 && merged) {
+                    h->timed(ABL_FV_PHASE_GHOST, st, [&] {
+                        hipLaunchKernelGGL(abl::k_ts_advance_ghosts, dim3(grid_for(h->n_bfaces), (unsigned)L.nc),
+                                           dim3(abl::kBlock), 0, st, h->cfl_partial.ptr, (int64_t)nb, lim, clock, other(),
+                                           h->ghost_view(), U, R);
+                    });
+                    clock = other();
+                    h->halt = &clock->halt;
+                } else {
+                    if (i > 0) advance(false);
+                    h->halt = &clock->halt;
+                    if (h->n_bfaces) h->timed(ABL_FV_PHASE_GHOST, st, [&] { fill_ghosts(h, st, U, R); });
+                }
+                launch_rhs(h, U, R, 0, st);
+                hipLaunchKernelGGL(update, dim3(nb), dim3(abl::kBlock), 0, st, U, R, h->rmin.ptr, L.N, L.NI, L.nc, h->ph,
+                                   h->phys.cfl, alpha, clock, h->cfl_partial.ptr);
+            }
+            advance(false);
+            HIP_CHECK(hipGetLastError());
+            HIP_CHECK(hipStreamSynchronize(st));
+            k = *h->ts_host;
+        }
+        if (k.bad) throw std::runtime_error("non-positive or NaN step size at t = " + std::to_string(k.t));
+        if (t_out) *t_out = k.t;
+        if (steps_out) *steps_out = k.steps;
+    } catch (const std::exception& e) {
+        return fail(h, std::string("abl_fv_ts_euler: ") + e.what());
+    }
+    return 0;
+}
+}  // namespace
+
 extern "C" int abl_fv_ts_euler(abl_fv_handle h, double* U, double* R, double t0, double max_time, double dt0,
                                double safety, int64_t max_steps, double* t_out, int64_t* steps_out,
                                abl_fv_stream stream) {
@@ -5081,6 +5269,11 @@ extern "C" int abl_fv_ts_euler(abl_fv_handle h, double* U, double* R, double t0,
     hipStream_t st = (hipStream_t)stream;
     double t = t0;
     int64_t steps = 0;
+    // The CFL step alone (no diffusion step, no pressure-gradient scaling): the whole loop runs on the device.
+    const bool diffusion_steps =
+        h->visc && (h->phys.conduction_stability_factor > 0.0 || h->phys.viscous_stability_factor > 0.0);
+    if (h->phys.flux_calculator != ABL_FV_FLUX_NONE && !diffusion_steps && !h->pgs_on)
+        return ts_euler_device(h, U, R, t0, max_time, dt0, safety, max_steps, t_out, steps_out, st);
     try {
         double dt = std::min(dt0, safety * physics_dt_impl(h, U, st));  // AdaptPhysics::AdaptInitializer
         while (t < max_time && steps < max_steps) {
