@@ -493,18 +493,20 @@ __device__ __forceinline__ void species_body(MeshView<G> m, Phys ph, const doubl
     const bool bj = ph.limiter == ABL_FV_LIMITER_BARTH_JESPERSEN;
     const double irho_c = 1.0 / U[kRho * N + c];
     // arithmetic of the gradient sums and the limiter: FP64 in the FP64 form; FP32 in the mixed form (which stores
-    // these gradients in FP32), on FP64 state differences rounded once
+    // these gradients in FP32), on FP64 state differences rounded once.  Conditions are selects (see gradients_body).
     using A = G;
-    int64_t nb[KM];
-    bool valid[KM], inner[KM];
+    int32_t nb[KM];  // the cell itself in padding slots
+    bool inner[KM];
     G w[KM][DIM], wa[KM][DIM], xl[KM][DIM];
     double irn[KM];
 #pragma unroll
     for (int k = 0; k < KM; k++) {
-        const int32_t e = m.snbr[k * NI + c];
-        valid[k] = e >= 0;
-        nb[k] = valid[k] ? (int64_t)e : c;
-        inner[k] = valid[k] && nb[k] < NI;
+        nb[k] = m.snbr[k * NI + c];
+        nb[k] = nb[k] >= 0 ? nb[k] : (int32_t)c;
+        inner[k] = nb[k] < NI;
+    }
+#pragma unroll
+    for (int k = 0; k < KM; k++) {
 #pragma unroll
         for (int d = 0; d < DIM; d++) {
             w[k][d] = G(0);
@@ -516,16 +518,24 @@ __device__ __forceinline__ void species_body(MeshView<G> m, Phys ph, const doubl
             load_slot_vec<DIM, KM, kSlotLimiter>(m, k, c, xl[k]);
         }
         if (aux) load_slot_vec<DIM, KM, kSlotAux>(m, k, c, wa[k]);
-        irn[k] = aux ? 1.0 / U[kRho * N + nb[k]] : 0.0;
+        irn[k] = 1.0 / U[kRho * N + nb[k]];
     }
     bool cancel = false;
+    double uc_next, un_next[KM];
+    auto load = [&](int sp) {
+        const int64_t row = (int64_t)(NE + sp) * N;
+        uc_next = U[row + c];
+#pragma unroll
+        for (int k = 0; k < KM; k++) un_next[k] = U[row + nb[k]];
+    };
+    load(0);
     for (int sp = 0; sp < ph.ns; sp++) {
-        const int64_t comp = NE + sp;
-        const double uc = U[comp * N + c];
-        const double yc = uc * irho_c;
+        const double uc = uc_next, yc = uc * irho_c;
         double un[KM];
 #pragma unroll
-        for (int k = 0; k < KM; k++) un[k] = U[comp * N + nb[k]];
+        for (int k = 0; k < KM; k++) un[k] = un_next[k];
+        if (sp + 1 < ph.ns) load(sp + 1);
+        __builtin_amdgcn_sched_barrier(0);
         A g[DIM], ga[DIM];
         double umin = uc, umax = uc;
 #pragma unroll
@@ -534,22 +544,18 @@ __device__ __forceinline__ void species_body(MeshView<G> m, Phys ph, const doubl
             ga[d] = A(0);
         }
 #pragma unroll
-        for (int k = 0; k < KM; k++) {
-            if (!valid[k]) continue;
-            if (recon) {
-                umin = fmin(umin, un[k]);
-                umax = fmax(umax, un[k]);
-                if (inner[k]) {
-                    const A delta = A(un[k] - uc);  // both sides: + w.(u_n - u_c), see k_gradients
+        for (int k = 0; k < KM; k++) {  // a padding slot's neighbour is the cell: differences and weights are zero
+            umin = fmin(umin, un[k]);
+            umax = fmax(umax, un[k]);
+            const A delta = inner[k] ? A(un[k] - uc) : A(0);  // both sides: + w.(u_n - u_c), see gradients_body
+            const A dY = A(un[k] * irn[k] - yc);
 #pragma unroll
-                    for (int d = 0; d < DIM; d++) g[d] += w[k][d] * delta;
-                }
+            for (int d = 0; d < DIM; d++) {
+                g[d] += w[k][d] * delta;
+                ga[d] += wa[k][d] * dY;
             }
-            if (aux) {
-                const A delta = A(un[k] * irn[k] - yc);
-#pragma unroll
-                for (int d = 0; d < DIM; d++) ga[d] += wa[k][d] * delta;
-            }
+            pin(g);
+            pin(ga);
         }
         if (recon) {
             A phi = sizeof(A) == 8 ? A(DBL_MAX) : A(FLT_MAX);
@@ -557,20 +563,24 @@ __device__ __forceinline__ void species_body(MeshView<G> m, Phys ph, const doubl
                 A dpos = A(0), dneg = A(0);
 #pragma unroll
                 for (int k = 0; k < KM; k++) {
-                    if (!valid[k]) continue;
                     A D = A(0);
 #pragma unroll
                     for (int d = 0; d < DIM; d++) D += g[d] * xl[k][d];
                     dpos = fmax(dpos, D);
                     dneg = fmin(dneg, D);
                 }
+                pin(dpos);
+                pin(dneg);
+                A up = A(umax - uc) / dpos;
+                pin(up);
+                const A dn = A(umin - uc) / dneg;
                 phi = A(1);
-                if (dpos > A(0)) phi = fmin(phi, A(umax - uc) / dpos);
-                if (dneg < A(0)) phi = fmin(phi, A(umin - uc) / dneg);
+                phi = dpos > A(0) ? fmin(phi, up) : phi;
+                phi = dneg < A(0) ? fmin(phi, dn) : phi;
             } else if (ph.limiter != ABL_FV_LIMITER_NONE) {
 #pragma unroll
                 for (int k = 0; k < KM; k++) {
-                    if (!valid[k]) continue;
+                    if (nb[k] == (int32_t)c) continue;  // padding slot
                     A denom = A(0);
 #pragma unroll
                     for (int d = 0; d < DIM; d++) denom += g[d] * xl[k][d];
@@ -580,10 +590,10 @@ __device__ __forceinline__ void species_body(MeshView<G> m, Phys ph, const doubl
             } else {
                 phi = A(1);
             }
-            if (phi == A(0))
+            bool large = false;
 #pragma unroll
-                for (int d = 0; d < DIM; d++)
-                    if (fabs(double(g[d])) > ph.max_lim_grad) cancel = true;
+            for (int d = 0; d < DIM; d++) large |= fabs(double(g[d])) > ph.max_lim_grad;
+            cancel |= (phi == A(0)) & large;
 #pragma unroll
             for (int d = 0; d < DIM; d++) g[d] *= phi;  // stored with the aux gradient below
         }
@@ -604,6 +614,7 @@ __device__ __forceinline__ void species_body(MeshView<G> m, Phys ph, const doubl
                 o[((int64_t)sp * DIM + j) * N + c] = t;
             }
         }
+        __builtin_amdgcn_sched_barrier(0);
     }
     if (cancel)  // the maxLimGrad rule zeroes the whole densityYi field of the cell (cellInterpolant.cpp:459-481)
         for (int sp = 0; sp < ph.ns; sp++)
@@ -1741,22 +1752,44 @@ __global__ __launch_bounds__(kBlock) void k_gather_mixed(MeshView<float> m, int 
     const int64_t c = xcd_cell_index();
     if (c >= m.NI || halted(m)) return;
     const int64_t N = m.N, NI = m.NI;
-    int64_t off[KM];
+    const float* __restrict__ from[KM];  // this side's rows of the slots' faces (padding slots: the first one's, unused)
     double sg[KM];
+    const int32_t e0 = slot_entry(m, 0, c);
 #pragma unroll
     for (int k = 0; k < KM; k++) {
-        const int32_t e = k < m.K ? m.ell[k * NI + c] : -1;
-        off[k] = e >= 0 ? (int64_t)(e >> 1) + ((e & 1) ? (int64_t)nrow * m.F : 0) : 0;
+        const int32_t e = slot_entry(m, k, c), ea = e >= 0 ? e : e0;
+        from[k] = Fm + (ea >> 1) + ((ea & 1) ? (int64_t)nrow * m.F : 0);
         sg[k] = e < 0 ? 0.0 : ((e & 1) ? 1.0 : -1.0);
     }
     const double iv = m.inv_vol[c];
-    for (int p = 0; p < nrow; p++) {
-        double acc = 0.0;
+    // rows in pairs, the next pair's loads in flight while one is summed (a wait per row kept 95 % of the waves' cycles:
+    // 60^3 x 6 tetrahedra with ten species, 137 us)
+    float next[2][KM];
+    auto load = [&](int p) {
 #pragma unroll
-        for (int k = 0; k < KM; k++)
-            acc += sg[k] * (sg[k] != 0.0 ? double(Fm[p * m.F + off[k]]) : 0.0);
-        const double r = acc * iv;
-        R[p * N + c] = accumulate ? R[p * N + c] + r : r;
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int k = 0; k < KM; k++) next[h][k] = from[k][(int64_t)(p + h < nrow ? p + h : p) * m.F];
+    };
+    load(0);
+    for (int p = 0; p < nrow; p += 2) {
+        float v[2][KM];
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int k = 0; k < KM; k++) v[h][k] = next[h][k];
+        if (p + 2 < nrow) load(p + 2);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            if (p + h >= nrow) break;
+            double acc = 0.0;
+#pragma unroll
+            for (int k = 0; k < KM; k++) acc += sg[k] * double(v[h][k]);
+            const double r = acc * iv;
+            const int64_t o = (int64_t)(p + h) * N + c;
+            R[o] = accumulate ? R[o] + r : r;
+        }
     }
 }
 
@@ -1767,35 +1800,61 @@ __global__ __launch_bounds__(kBlock) void k_gather_mixed(MeshView<float> m, int 
 // every face contributes dF/dU_side^T g_f with g_f = Rbar_R / V_R - Rbar_L / V_L.  One lane per interior cell
 // recomputes the forward flux of each of its faces and keeps its own side's adjoint (deterministic gather).
 
-// Seed of one component of a face, Rbar_R / V_R - Rbar_L / V_L (a ghost right side: rbR = ivR = 0), in one fixed order of
-// operations: the kernels that form it per face and per cell agree bit for bit.
+// Seed of one component of a face, Rbar_R / V_R - Rbar_L / V_L, in one fixed order of operations: the kernels that form it
+// per face and per cell agree bit for bit.  A ghost right side has no Rbar: the interior cell's row is read in its
+// place, with ivR = 0 (a select around the load would become a branch, and a wait for every species).
 __device__ inline double face_seed_of(double rbR, double ivR, double rbL, double ivL) {
     return __builtin_fma(rbR, ivR, -(rbL * ivL));
 }
 
-// Adjoint seeds of face f: g[p] for euler components and the species sums QL = sum g_sp rhoY_L,
-// QR = sum g_sp rhoY_R, QdL = sum g_sp (rhoY_R - rhoY_L).
-template <int DIM, int UNR = 2>
+// Adjoint seeds of face f: fb[p] for euler components and the species sums QL = sum g_sp rhoY_L, QR = sum g_sp rhoY_R,
+// QdL = sum g_sp (rhoY_R - rhoY_L), with the next BATCH species' loads in flight while one batch is summed.  The species
+// come first, while few registers are live (k_vjp_faces at 128^3 hexes with ten species: 449 us when the compiler kept
+// two loads in flight beside the euler states).
+template <int DIM, int BATCH = 2>
 __device__ inline void face_seed(const MeshView<double>& m, const Phys& ph, const double* __restrict__ U,
                                  const double* __restrict__ Rb, int64_t L, int64_t Rc, bool ghost, double* fb,
                                  double& QL, double& QR, double& QdL) {
     constexpr int NE = DIM + 2;
     const int64_t N = m.N;
-    const double ivL = m.inv_vol[L], ivR = ghost ? 0.0 : m.inv_vol[Rc];
-#pragma unroll
-    for (int p = 0; p < NE; p++) fb[p] = face_seed_of(ghost ? 0.0 : Rb[p * N + Rc], ivR, Rb[p * N + L], ivL);
+    const int64_t Rr = ghost ? L : Rc;
+    const double ivL = m.inv_vol[L], ivN = m.inv_vol[Rr], ivR = ghost ? 0.0 : ivN;
     QL = 0.0;
     QR = 0.0;
     QdL = 0.0;
-#pragma unroll UNR
-    for (int sp = 0; sp < ph.ns; sp++) {  // UNR species' loads in flight
-        const int64_t comp = NE + sp;
-        const double g = face_seed_of(ghost ? 0.0 : Rb[comp * N + Rc], ivR, Rb[comp * N + L], ivL);
-        const double yl = U[comp * N + L], yr = U[comp * N + Rc];
-        QL += g * yl;
-        QR += g * yr;
-        QdL += g * (yr - yl);
+    if (ph.ns) {
+        double next[BATCH][4];
+        auto load = [&](int s0) {
+#pragma unroll
+            for (int b = 0; b < BATCH; b++) {
+                const int64_t row = (int64_t)(NE + (s0 + b < ph.ns ? s0 + b : s0)) * N;
+                next[b][0] = Rb[row + L];
+                next[b][1] = Rb[row + Rr];
+                next[b][2] = U[row + L];
+                next[b][3] = U[row + Rc];
+            }
+        };
+        load(0);
+        for (int s0 = 0; s0 < ph.ns; s0 += BATCH) {
+            double v[BATCH][4];
+#pragma unroll
+            for (int b = 0; b < BATCH; b++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) v[b][i] = next[b][i];
+            if (s0 + BATCH < ph.ns) load(s0 + BATCH);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int b = 0; b < BATCH; b++) {
+                const double g = s0 + b < ph.ns ? face_seed_of(v[b][1], ivR, v[b][0], ivL) : 0.0;
+                QL += g * v[b][2];
+                QR += g * v[b][3];
+                QdL += g * (v[b][3] - v[b][2]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
+#pragma unroll
+    for (int p = 0; p < NE; p++) fb[p] = face_seed_of(Rb[p * N + Rr], ivR, Rb[p * N + L], ivL);
 }
 
 template <int DIM, bool RUS>
@@ -1891,7 +1950,7 @@ __global__ __launch_bounds__(kBlock) void k_vjp(MeshView<double> m, Phys ph, con
 #pragma unroll
         for (int k = 0; k < KM; k++) {
             const bool ghost = sR[k] >= NI;
-            const double g = face_seed_of(ghost ? 0.0 : Rb[comp * N + sR[k]], ivR[k], Rb[comp * N + sL[k]], ivL[k]);
+            const double g = face_seed_of(Rb[comp * N + (ghost ? sL[k] : sR[k])], ivR[k], Rb[comp * N + sL[k]], ivL[k]);
             a += coef[k] * g;
             if (cghost[k] != 0.0) Ub[comp * N + sR[k]] = cghost[k] * g;
         }
@@ -1920,13 +1979,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     const int64_t L = m.fcell[f], Rc = m.fcell[F + f];
     const bool ghost = Rc >= NI;
     double nh[3], area, uL[NE], uR[NE], fb[NE], QL, QR, QdL;
+    face_seed<DIM, 5>(m, ph, U, Rb, L, Rc, ghost, fb, QL, QR, QdL);
     load_face_na(m.fna, geometry_row(m, f), nh, area);
 #pragma unroll
     for (int p = 0; p < NE; p++) {
         uL[p] = U[p * N + L];
         uR[p] = U[p * N + Rc];
     }
-    face_seed<DIM, 5>(m, ph, U, Rb, L, Rc, ghost, fb, QL, QR, QdL);
     double w[2][SW], cL, cR;
 #pragma unroll
     for (int i = 0; i < SW; i++) {
@@ -2225,7 +2284,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
         for (int sp = 0; sp < ns; sp++) {
             const Sp v = nx;
             if (sp + 1 < ns) load(sp + 1);
-            const double gsp = face_seed_of(ghost ? 0.0 : v.rr, ivR, v.rl, ivL);
+            const double gsp = face_seed_of(v.rr, ivR, v.rl, ivL);
             double wl[2 * DIM], wr[2 * DIM], yl = v.yl, yr = v.yr, dot = 0.0;
 #pragma unroll
             for (int q = 0; q < DIM; q++) {
@@ -2253,7 +2312,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
     }
     double g[NE];
 #pragma unroll
-    for (int p = 0; p < NE; p++) g[p] = face_seed_of(ghost ? 0.0 : Rb[p * N + Rr], ivR, Rb[p * N + L], ivL);
+    for (int p = 0; p < NE; p++) g[p] = face_seed_of(Rb[p * N + Rr], ivR, Rb[p * N + L], ivL);
     // both sides: cell state, face state and viscous terms from the cell records
     double uL[NE], uR[NE], fL[NE], fR[NE], tqL[NT], tqR[NT];
 #pragma unroll
