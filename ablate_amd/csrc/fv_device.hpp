@@ -80,6 +80,7 @@ struct MeshView {
     const uint16_t* __restrict__ srow;  // [KM][NI]
     const G* __restrict__ stab;         // [rows][sstride]
     int sstride, saux;
+    int rec_swap;  // order of the cells in a record block (rec_lane)
     // Not null: every kernel of the right-hand side returns at once when *halt is set (the device-side time loop
     // enqueues steps ahead of the one that ends it).
     const int32_t* halt;

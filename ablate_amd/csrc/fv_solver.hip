@@ -15,6 +15,7 @@
 //                          being stored: no float atomics, no face-flux array, bitwise deterministic.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <array>
 #include <cmath>
 #include <cstdio>
@@ -107,6 +108,13 @@ enum : int { kLimNone = 0, kLimPetsc = 1, kLimBJ = 2 };
 // consecutive cells) store each pair with one coalesced 1 KB store, and the faces of a wave, whose cells cluster,
 // read each pair from a few cache lines with one 16-byte load (a per-cell record made every load of the wave touch
 // up to 64 lines; single words per load took twice the load instructions).
+// Position of cell c in its 64-cell block: c mod 64, with bits 2 and 3 exchanged when `swap` (0 or 1) is set.  A line
+// of 128 bytes holds the pair of 8 cells: 8 in a row by number, or (swap) 4 in a row of two rows 8 apart.  In bricks of
+// 8 x 8 x 8 cells the latter halves the lines that the faces across a brick's x sides touch (see choose_rec_swap).
+__device__ __host__ inline int32_t rec_lane(int64_t c, int swap) {
+    const int32_t l = (int32_t)(c & 63);
+    return l ^ (12 * (((l >> 2) ^ (l >> 3)) & swap));
+}
 template <int DIM>
 struct CellRec {
     static constexpr int NE = DIM + 2;
@@ -118,15 +126,9 @@ struct CellRec {
     static constexpr int BLOCK = 64;
 };
 template <int DIM>
-__device__ inline int64_t rec_pair(int64_t c) {
-    return (c >> 6) * (int64_t)(CellRec<DIM>::BLOCK * CellRec<DIM>::NP) + (c & 63);
+__device__ inline int64_t rec_pair(int64_t c, int swap) {
+    return (c >> 6) * (int64_t)(CellRec<DIM>::BLOCK * CellRec<DIM>::NP) + rec_lane(c, swap);
 }
-// Word i of cell c's record.
-template <int DIM>
-__device__ inline double rec_word(const double* __restrict__ rec, int64_t c, int i) {
-    return rec[2 * (rec_pair<DIM>(c) + (int64_t)CellRec<DIM>::BLOCK * (i >> 1)) + (i & 1)];
-}
-
 // Face records (fluxes, adjoints) of np word pairs, in blocks of 64 consecutive faces: pair q of face f is the double2 at
 // face_pair(f, np) + 64 q.  A wave of consecutive faces stores each pair with one coalesced 1 KB access, and the gather
 // of a wave of consecutive cells, whose faces cluster, reads it from a few lines.  With one contiguous record per face
@@ -156,8 +158,8 @@ struct CellRecF {
     static constexpr int RS = 4 * NP;                                 // floats per cell (with padding)
 };
 template <int DIM>
-__device__ inline int64_t recf_pair(int64_t c) {
-    return (c >> 6) * (int64_t)(64 * CellRecF<DIM>::NP) + (c & 63);
+__device__ inline int64_t recf_pair(int64_t c, int swap) {
+    return (c >> 6) * (int64_t)(64 * CellRecF<DIM>::NP) + rec_lane(c, swap);
 }
 
 template <int DIM, bool RECON, bool VISC>
@@ -168,10 +170,11 @@ struct RecF {
 };
 // Loads a mixed-form cell record (FP64 state, FP32 gradients and viscous terms).
 template <int DIM, bool RECON, bool VISC>
-__device__ inline void load_rec_f(const float* __restrict__ rec, int64_t c, RecF<DIM, RECON, VISC>& r) {
+__device__ inline void load_rec_f(const MeshView<float>& m, const float* __restrict__ rec, int64_t c,
+                                  RecF<DIM, RECON, VISC>& r) {
     using CR = CellRecF<DIM>;
     constexpr int NE = DIM + 2;
-    const ulonglong2* __restrict__ b = reinterpret_cast<const ulonglong2*>(rec) + recf_pair<DIM>(c);
+    const ulonglong2* __restrict__ b = reinterpret_cast<const ulonglong2*>(rec) + recf_pair<DIM>(c, m.rec_swap);
     constexpr int NF = VISC ? CR::TF + ViscTerms<DIM>::NT : (RECON ? CR::TF : 0);
     constexpr int NFW = (NF + 1) / 2;  // words holding the FP32 values needed
     uint64_t wd[2 * CR::NP];
@@ -430,7 +433,7 @@ __device__ __forceinline__ void gradients_body(MeshView<G> m, Phys ph, const dou
             for (int q = 0; q < ViscTerms<DIM>::NT; q++) w[CR::T0 + q] = VISC ? double(tq[q]) : 0.0;
 #pragma unroll
             for (int i = CR::END; i < CR::RS; i++) w[i] = 0.0;
-            double2* __restrict__ r = reinterpret_cast<double2*>(rec) + rec_pair<DIM>(c);
+            double2* __restrict__ r = reinterpret_cast<double2*>(rec) + rec_pair<DIM>(c, m.rec_swap);
 #pragma unroll
             for (int q = 0; q < CR::NP; q++) r[CR::BLOCK * q] = make_double2(w[2 * q], w[2 * q + 1]);
         }
@@ -457,7 +460,7 @@ __device__ __forceinline__ void gradients_body(MeshView<G> m, Phys ph, const dou
             for (int p = 0; p < NE; p++) wd[CR::U0 / 2 + p] = (uint64_t)__double_as_longlong(uc[p]);
 #pragma unroll
             for (int i = CR::RSW; i < 2 * CR::NP; i++) wd[i] = 0;
-            ulonglong2* __restrict__ w = reinterpret_cast<ulonglong2*>(rec) + recf_pair<DIM>(c);
+            ulonglong2* __restrict__ w = reinterpret_cast<ulonglong2*>(rec) + recf_pair<DIM>(c, m.rec_swap);
 #pragma unroll
             for (int q = 0; q < CR::NP; q++) w[64 * q] = make_ulonglong2(wd[2 * q], wd[2 * q + 1]);
         }
@@ -671,14 +674,14 @@ __device__ inline void side_cell_values(const double* u, SideData<DIM, VISC>& sd
 // straight line and are in flight together; with the choice between record and state around the loads, the right
 // side's were issued only when the left side's had arrived.
 template <int DIM, bool RECON, bool VISC>
-__device__ inline void load_side(const double* __restrict__ U, const double* __restrict__ rec, int64_t N, int64_t c,
-                                 const double* dx, SideData<DIM, VISC>& sd) {
+__device__ inline void load_side(const MeshView<double>& m, const double* __restrict__ U,
+                                 const double* __restrict__ rec, int64_t c, const double* dx, SideData<DIM, VISC>& sd) {
     using CR = CellRec<DIM>;
     constexpr int NE = DIM + 2;
     constexpr int NL = VISC ? CR::END : (RECON ? CR::T0 : NE);
     double r[2 * ((NL + 1) / 2)];
     if constexpr (RECON || VISC) {
-        const double2* __restrict__ rb = reinterpret_cast<const double2*>(rec) + rec_pair<DIM>(c);
+        const double2* __restrict__ rb = reinterpret_cast<const double2*>(rec) + rec_pair<DIM>(c, m.rec_swap);
 #pragma unroll
         for (int q = 0; q < (NL + 1) / 2; q++) {
             // without reconstruction the pairs holding only gradient words are not read
@@ -689,7 +692,7 @@ __device__ inline void load_side(const double* __restrict__ U, const double* __r
         }
     } else {
 #pragma unroll
-        for (int p2 = 0; p2 < NE; p2++) r[p2] = U[p2 * N + c];
+        for (int p2 = 0; p2 < NE; p2++) r[p2] = U[p2 * m.N + c];
     }
 #pragma unroll
     for (int p2 = 0; p2 < NE; p2++) {
@@ -743,8 +746,8 @@ __device__ inline void load_sides(const MeshView<double>& m, const Phys& ph, con
                                   SideData<DIM, VISC>& sr) {
     constexpr bool USE_REC = RECON || VISC;  // (a first-order inviscid face reads the ghost's state row itself)
     const bool ghost = Rc >= m.NI;
-    load_side<DIM, RECON, VISC>(U, rec, m.N, L, x[0], sl);
-    load_side<DIM, RECON, VISC>(U, rec, m.N, USE_REC && ghost ? L : Rc, x[1], sr);
+    load_side<DIM, RECON, VISC>(m, U, rec, L, x[0], sl);
+    load_side<DIM, RECON, VISC>(m, U, rec, USE_REC && ghost ? L : Rc, x[1], sr);
     if (USE_REC && ghost) {
         ghost_side<DIM, VISC>(U, m.N, Rc, sr);
         if (VISC) {
@@ -1328,13 +1331,13 @@ __device__ inline void mixed_face(const MeshView<float>& m, const Phys& ph, cons
     for (int d = 0; d < DIM; d++) nhat[d] = nh[d];
     RecF<DIM, RECON, VISC> rl, rr;
     if (USE_REC) {
-        load_rec_f<DIM, RECON, VISC>(rec, L, rl);
+        load_rec_f<DIM, RECON, VISC>(m, rec, L, rl);
     } else {
 #pragma unroll
         for (int p = 0; p < NE; p++) rl.u[p] = U[p * N + L];
     }
     if (USE_REC) {  // a ghost has no record: the left cell's stands in, so that both loads are in flight together
-        load_rec_f<DIM, RECON, VISC>(rec, ghost ? L : Rc, rr);
+        load_rec_f<DIM, RECON, VISC>(m, rec, ghost ? L : Rc, rr);
         if (ghost)
 #pragma unroll
             for (int p = 0; p < NE; p++) rr.u[p] = U[p * N + Rc];
@@ -2321,7 +2324,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
         double* fu = sd == 0 ? fL : fR;
         double* tq = sd == 0 ? tqL : tqR;
         double r[CR::RS];
-        const double2* __restrict__ rb = reinterpret_cast<const double2*>(rec) + rec_pair<DIM>(sd == 0 ? L : Rr);
+        const double2* __restrict__ rb = reinterpret_cast<const double2*>(rec) + rec_pair<DIM>(sd == 0 ? L : Rr, m.rec_swap);
 #pragma unroll
         for (int q = 0; q < CR::NP; q++) {
             const double2 v = rb[CR::BLOCK * q];
@@ -3855,6 +3858,28 @@ bool build_slot_rows(const Layout& L, int KM, int lim, SlotRows<G>& out) {
     return true;
 }
 
+// Whether the cell records exchange bits 2 and 3 of the cell number inside their 64-cell blocks (rec_lane): the order in
+// which the cells across a tile's faces touch fewer 128-byte lines, counted over up to 256 tiles of the mesh.  Bricks of
+// 8 x 8 x 8 cells numbered x first: 120 lines per word pair of a 256-cell tile without the exchange, 96 with it; the
+// tile pass takes 2.33 and 2.15 ms at 256^3 (Navier-Stokes FP64), 546 and 513 us at 200 x 161 x 150 (mixed).
+int choose_rec_swap(const Layout& L, const Tiles& tl) {
+    int64_t lines[2] = {0, 0};
+    std::vector<int64_t> key;
+    const int64_t stride = std::max<int64_t>(1, tl.n / 256);
+    for (int64_t t = 0; t < tl.n; t += stride)
+        for (int swap = 0; swap < 2; swap++) {
+            key.clear();
+            for (int32_t i = tl.start[(size_t)t]; i < tl.start[(size_t)t + 1]; i++)
+                for (int s = 0; s < 2; s++) {
+                    const int64_t c = L.fcell[(size_t)(s * L.F + tl.faces[(size_t)i])];
+                    if (c < L.NI) key.push_back((c >> 6) * 8 + (rec_lane(c, swap) >> 3));
+                }
+            std::sort(key.begin(), key.end());
+            lines[swap] += std::unique(key.begin(), key.end()) - key.begin();
+        }
+    return lines[1] < lines[0] ? 1 : 0;
+}
+
 }  // namespace abl
 
 struct abl_fv_solver {
@@ -3872,6 +3897,7 @@ struct abl_fv_solver {
     abl::DevBuf<double> stab;
     abl::DevBuf<float> stab_f;
     int slot_stride = 0, slot_aux = 0;
+    int rec_swap = 0;  // rec_lane order of the cell records (choose_rec_swap)
     const int32_t* halt = nullptr;  // set while abl_fv_ts_euler enqueues steps (MeshView::halt)
     bool slot_rows = false;
     abl::DevBuf<double> rec;            // cell records of the FP64 form (rec_pair blocks)
@@ -4023,6 +4049,7 @@ struct abl_fv_solver {
         v.sstride = slot_stride;
         v.saux = slot_aux;
         v.halt = halt;
+        v.rec_swap = rec_swap;
         return v;
     }
     abl::MeshView<float> view_f() const {
@@ -4048,6 +4075,7 @@ struct abl_fv_solver {
         v.sstride = slot_stride;
         v.saux = slot_aux;
         v.halt = halt;
+        v.rec_swap = rec_swap;
         return v;
     }
     abl::GhostView ghost_view() const {
@@ -4110,6 +4138,7 @@ struct abl_fv_solver {
                                    face_rows.empty() ? f : (int32_t)face_rows[(size_t)f]);
         }
         tile_faces.upload(entries);
+        if (!only_T) rec_swap = abl::choose_rec_swap(lay, tl);
         tile_slot.upload(tl.slot);
         tile_T = tl.T;
         tile_threads = tl.n <= 4 * (int64_t)cus ? std::max(tl.T, abl::kBlock) : tl.T;
