@@ -2845,25 +2845,28 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     const bool recon = ph.recon != 0, sdiff = ph.sdiff != 0;
     const bool bj = ph.limiter == ABL_FV_LIMITER_BARTH_JESPERSEN;
     const double2* __restrict__ W = reinterpret_cast<const double2*>(b.W);
-    int64_t nb[KM], wb[KM], gi[KM];
-    bool valid[KM], bnd[KM], any_bnd = false;
+    // Conditions are selects (see gradients_body); a padding slot reads the cell's first face and its own state, with zero
+    // coefficients and weights.
+    int32_t nb[KM], e[KM];
+    int64_t wb[KM];
+    bool bnd[KM], any_bnd = false;
     double xs[KM][DIM], cnv[KM][DIM], csk[KM], wl[KM][DIM], wa[KM][DIM];
 #pragma unroll
     for (int k = 0; k < KM; k++) {
-        const int32_t e = k < m.K ? m.ell[k * NI + c] : -1;
-        valid[k] = e >= 0;
-        const int64_t f = valid[k] ? (int64_t)(e >> 1) : 0;
-        const int s = e & 1;
-        const int32_t n = m.snbr[k * NI + c];
-        nb[k] = valid[k] ? (int64_t)n : c;
+        e[k] = slot_entry(m, k, c);
+        nb[k] = m.snbr[k * NI + c];
+    }
+#pragma unroll
+    for (int k = 0; k < KM; k++) {
+        const bool valid = e[k] >= 0;
+        nb[k] = valid ? nb[k] : (int32_t)c;
         bnd[k] = nb[k] >= NI;
         any_bnd |= bnd[k];
-        gi[k] = (valid[k] && bnd[k]) ? nb[k] - NI : -1;
+        const int64_t f = (valid ? e[k] : e[0]) >> 1;
+        const int s = e[k] & 1;
         wb[k] = face_pair(f, b.nwp);
-        double x[2][DIM], nh[3], area;
-        const int64_t geo = geometry_row(m, f);
-        load_face_pair<DIM>(m.fdx, geo, x);
-        load_face_na(m.fna, geo, nh, area);
+        double nh[3], area;
+        load_face_na(m.fna, geometry_row(m, f), nh, area);
         double cw[4];  // words CL, CR, CD of the record (two pairs from CL's pair on)
         {
             const double2 v0 = W[wb[k] + 64 * (AW::CL / 2)], v1 = W[wb[k] + 64 * (AW::CL / 2 + 1)];
@@ -2872,106 +2875,120 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
             cw[2] = v1.x;
             cw[3] = v1.y;
         }
-        const int o = AW::CL & 1;
-        csk[k] = valid[k] ? (s ? cw[o + 1] : cw[o]) : 0.0;
-        const double cd = valid[k] ? cw[o + 2] : 0.0;
+        constexpr int o = AW::CL & 1;
+        const double cs = s ? cw[o + 1] : cw[o];
+        csk[k] = valid ? cs : 0.0;
+        const double cd = valid ? cw[o + 2] : 0.0;
 #pragma unroll
         for (int d = 0; d < DIM; d++) {
-            xs[k][d] = s ? x[1][d] : x[0][d];
+            xs[k][d] = 0.0;
             cnv[k][d] = cd * nh[d];
             wl[k][d] = 0.0;
             wa[k][d] = 0.0;
         }
-        if (recon) load_slot_vec<DIM, KM, kSlotWeight>(m, k, c, wl[k]);
+        if (recon) {
+            load_slot_vec<DIM, KM, kSlotLimiter>(m, k, c, xs[k]);
+            load_slot_vec<DIM, KM, kSlotWeight>(m, k, c, wl[k]);
+        }
         if (sdiff) load_slot_vec<DIM, KM, kSlotAux>(m, k, c, wa[k]);
     }
-    const double rho_c = U[c];
-    double rbc = 0.0, rbn[KM], rho_n[KM];
+    const double irho_c = 1.0 / U[c];
+    double rbc = 0.0, rbn[KM], irn[KM];
 #pragma unroll
     for (int k = 0; k < KM; k++) {
         rbn[k] = 0.0;
-        rho_n[k] = sdiff ? U[nb[k]] : 1.0;
+        irn[k] = 1.0 / U[nb[k]];
     }
-    const double* __restrict__ GL = b.GL;
-    // species in pairs: both species' loads (own and neighbour densities, the record pair) are issued before either
-    // is reversed, so two dependent rounds of memory latency overlap
-    for (int sp0 = 0; sp0 < ns; sp0 += 2) {
-        const int nh = sp0 + 1 < ns ? 2 : 1;
-        double ycs[2], unv[2][KM], gsp[2][KM];
+    // the next species' densities and seeds are in flight while one is reversed
+    double yc_next, un_next[KM], gs_next[KM];
+    auto load = [&](int sp) {
+        const int64_t row = (int64_t)(NE + sp) * N;
+        const double* __restrict__ Ws = b.W + ((sp & 1) + 128 * (int64_t)(AW::GS / 2 + (sp >> 1)));
+        yc_next = U[row + c];
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int64_t comp = NE + sp0 + (h < nh ? h : 0);
-            ycs[h] = U[comp * N + c];
+        for (int k = 0; k < KM; k++) {
+            pin(nb[k]);
+            un_next[k] = U[row + nb[k]];
+            gs_next[k] = Ws[2 * wb[k]];
+        }
+    };
+    load(0);
+    for (int sp = 0; sp < ns; sp++) {
+        const int64_t comp = NE + sp;
+        const double yc = yc_next;
+        double un[KM], gsp[KM];
 #pragma unroll
-            for (int k = 0; k < KM; k++) unv[h][k] = U[comp * N + nb[k]];
+        for (int k = 0; k < KM; k++) {
+            un[k] = un_next[k];
+            gsp[k] = gs_next[k];
+        }
+        if (sp + 1 < ns) load(sp + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        // the faces' species factors
+        double usb = 0.0, gsb[DIM], gyb[DIM], cs[KM];
+#pragma unroll
+        for (int d = 0; d < DIM; d++) {
+            gsb[d] = 0.0;
+            gyb[d] = 0.0;
         }
 #pragma unroll
         for (int k = 0; k < KM; k++) {
-            const double2 v = W[wb[k] + 64 * (AW::GS / 2 + (sp0 >> 1))];
-            gsp[0][k] = v.x;
-            gsp[1][k] = v.y;
-        }
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            if (h >= nh) break;
-            const int sp = sp0 + h;
-            const int64_t comp = NE + sp;
-            // the faces' species factors
-            double usb = 0.0, gsb[DIM], gyb[DIM];
+            const double yb = csk[k] * gsp[k];
+            usb += yb;
+            cs[k] = 0.0;
 #pragma unroll
             for (int d = 0; d < DIM; d++) {
-                gsb[d] = 0.0;
-                gyb[d] = 0.0;
+                gsb[d] += yb * xs[k][d];
+                gyb[d] += gsp[k] * cnv[k][d];
             }
+        }
+        if (any_bnd)  // the boundary faces' extras from the ghosts' gradients
+#pragma unroll
+            for (int k = 0; k < KM; k++)
+                if (bnd[k]) usb += b.GL[(int64_t)sp * NG + (nb[k] - NI)];
+        pin(gsb);
+        pin(gyb);
+        pin(usb);
+        if (recon)
+            limited_lsq_vjp<DIM, KM>(un, yc, wl, xs, bnd, any_bnd, bj, gsb, usb, cs,
+                                     [&](int k, double v) { b.Ughost[comp * NG + (nb[k] - NI)] += v; });
+        pin(cs);
+        pin(usb);
+        if (sdiff) {
+            // transpose of the aux gradient sum_k wa_k (Y_n - Y_c), then of Y = rhoY / rho (massfrac_vjp)
+            double ycb = 0.0, yn[KM], rn[KM];
 #pragma unroll
             for (int k = 0; k < KM; k++) {
-                if (!valid[k]) continue;
-                const double yb = csk[k] * gsp[h][k];
-                usb += yb;
-                if (gi[k] >= 0) usb += GL[(int64_t)sp * NG + gi[k]];
+                double t = 0.0;
 #pragma unroll
-                for (int d = 0; d < DIM; d++) {
-                    gsb[d] += yb * xs[k][d];
-                    gyb[d] += gsp[h][k] * cnv[k][d];
-                }
+                for (int d = 0; d < DIM; d++) t += wa[k][d] * gyb[d];
+                ycb -= t;
+                yn[k] = t * irn[k];
+                rn[k] = -(yn[k] * un[k]) * irn[k];
+                cs[k] += bnd[k] ? 0.0 : yn[k];
+                rbn[k] += bnd[k] ? 0.0 : rn[k];
             }
-            double cs[KM];  // this species' contributions to the neighbours
+            if (any_bnd)
 #pragma unroll
-            for (int k = 0; k < KM; k++) cs[k] = 0.0;
-            if (recon)
-                limited_lsq_vjp<DIM, KM>(unv[h], ycs[h], wl, xs, bnd, any_bnd, bj, gsb, usb, cs,
-                                         [&](int k, double v) { b.Ughost[comp * NG + (nb[k] - NI)] += v; });
-            if (sdiff) {
-                double ycb = 0.0;
-#pragma unroll
-                for (int k = 0; k < KM; k++) {
-                    if (!valid[k]) continue;
-                    double t = 0.0;
-#pragma unroll
-                    for (int d = 0; d < DIM; d++) t += wa[k][d] * gyb[d];
-                    ycb -= t;
-                    double yb_n = 0.0, rb_n = 0.0;
-                    massfrac_vjp(rho_n[k], unv[h][k], t, yb_n, rb_n);
+                for (int k = 0; k < KM; k++)
                     if (bnd[k]) {
-                        b.Ughost[comp * NG + (nb[k] - NI)] += yb_n;
-                        b.Ughost[(int64_t)kRho * NG + (nb[k] - NI)] += rb_n;
-                    } else {
-                        cs[k] += yb_n;
-                        rbn[k] += rb_n;
+                        b.Ughost[comp * NG + (nb[k] - NI)] += yn[k];
+                        b.Ughost[(int64_t)kRho * NG + (nb[k] - NI)] += rn[k];
                     }
-                }
-                massfrac_vjp(rho_c, ycs[h], ycb, usb, rbc);
-            }
-            b.Uself[comp * NI + c] = usb;
-#pragma unroll
-            for (int k = 0; k < KM; k++) b.contrib[((int64_t)k * nc + comp) * NI + c] = cs[k];
+            usb += ycb * irho_c;
+            rbc -= ycb * yc * irho_c * irho_c;
+            pin(rbn);
         }
+        b.Uself[comp * NI + c] = usb;
+#pragma unroll
+        for (int k = 0; k < KM; k++) b.contrib[((int64_t)k * nc + comp) * NI + c] = cs[k];
+        __builtin_amdgcn_sched_barrier(0);
     }
     if (sdiff) {
         b.Uself[(int64_t)kRho * NI + c] += rbc;
 #pragma unroll
         for (int k = 0; k < KM; k++)
-            if (valid[k] && !bnd[k]) b.contrib[((int64_t)k * nc + kRho) * NI + c] += rbn[k];
+            if (e[k] >= 0 && !bnd[k]) b.contrib[((int64_t)k * nc + kRho) * NI + c] += rbn[k];
     }
 }
 
