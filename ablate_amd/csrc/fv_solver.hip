@@ -2210,20 +2210,25 @@ struct AdjBufs {
 //   [NE, 2 NE)          right face state; on a boundary face (ghost right cell, whose adjoint goes to Ughost) the
 //                       left cell's extra aux adjoint [NE, NE + DIM + 1) and density adjoint (NE + DIM + 1) from the
 //                       ghost's one-neighbour viscous gradient
-//   [2 NE, 2 NE + NT)   half the adjoint of the face-averaged viscous terms (each side's share)
+//   [2 NE, 2 NE + DIM)  h: half (momentum seed + face velocity x energy seed)
+//   + 1                 half the energy seed e.  With the area normal n, each side's share of the adjoint of the
+//                       face-averaged viscous terms is -(h n^T + n h^T) (its diagonal halved) and -e n: four words and the
+//                       normal instead of the nine terms
 //   + DIM               half the adjoint of the face velocity
-//   + 4                 species coefficients cL, cR (F_sp = cL rhoY_L,f + cR rhoY_R,f), the diffusion coefficient
+//   + 4                 (with species) coefficients cL, cR (F_sp = cL rhoY_L,f + cR rhoY_R,f), the diffusion coefficient
 //                       cd = -D rho_face A / 2 and the face density adjoint summed over species
-//   + ns                per species g_sp = Rbar_sp(R) / V_R - Rbar_sp(L) / V_L
+//   + ns                (from an even word on) per species g_sp = Rbar_sp(R) / V_R - Rbar_sp(L) / V_L
 // Stored as word pairs in blocks of 64 faces (pair q of face f at double2 index (f / 64) 64 NWP + 64 q + f % 64):
-// each store of a wave (64 consecutive faces) is one coalesced 1 KB access.
+// each store of a wave (64 consecutive faces) is one coalesced 1 KB access.  The passes are bound by these records'
+// traffic and latency: with h and e in the nine viscous terms' place and no words after them without species (208 ->
+// 144 bytes per face) 100 x 75 x 61 hexes took k_adj_face_rev 117 -> 104 and k_adj_cells_e 200 -> 176 us, and
+// k_adj_face_rev on 47^3 x 6 tetrahedra with ten species 341 -> 318 us.
 template <int DIM>
 struct AdjFaceRec {
     static constexpr int NE = DIM + 2;
-    static constexpr int NT = ViscTerms<DIM>::NT;
-    static constexpr int UL = 0, UR = NE, TQ = 2 * NE, VL = TQ + NT, CL = VL + DIM, CR = CL + 1, CD = CL + 2,
+    static constexpr int UL = 0, UR = NE, H = 2 * NE, E = H + DIM, VL = E + 1, CL = VL + DIM, CR = CL + 1, CD = CL + 2,
                          RH = CL + 3, GS = (CL + 5) & ~1;  // species factors start on a pair boundary
-    __host__ __device__ static int words(int ns) { return GS + ns; }
+    __host__ __device__ static int words(int ns) { return ns ? GS + ns : CL; }
     __host__ __device__ static int pairs(int ns) { return (words(ns) + 1) / 2; }
 };
 
@@ -2360,9 +2365,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
     if (ph.flux == ABL_FV_FLUX_AUSM || ph.flux == ABL_FV_FLUX_RUSANOV)
         face_vjp<DIM, RUS>(fL, fR, QL, QR, QdL, nh, area, ph, g, ubL, ubR, cL, cR);
     // viscous flux
-    double tqbf[NT], velbf[DIM], wg[2][DIM];
+    double tqbf[NT], velbf[DIM], wg[2][DIM], h[DIM];
 #pragma unroll
     for (int q = 0; q < NT; q++) tqbf[q] = 0.0;
+#pragma unroll
+    for (int d = 0; d < DIM; d++) h[d] = 0.0;
 #pragma unroll
     for (int d = 0; d < DIM; d++) velbf[d] = 0.0;
     if (visc) {
@@ -2398,6 +2405,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
 #pragma unroll
         for (int q = 0; q < NT; q++) tqf[q] = 0.5 * tqL[q] + 0.5 * tqR[q];
         viscous_flux_vjp<DIM>(normal, vf, tqf, g, tqbf, velbf);
+#pragma unroll
+        for (int d = 0; d < DIM; d++) h[d] = 0.5 * (g[kRhoU + d] + vf[d] * g[kRhoE]);
     }
     double tqh[NT], velh[DIM];
 #pragma unroll
@@ -2472,22 +2481,25 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
     }
     // the record, pair by pair
     double w[AW::GS];
-    w[AW::GS - 1] = 0.0;  // padding word (2-D)
+    w[AW::GS - 1] = 0.0;  // padding word
 #pragma unroll
     for (int p = 0; p < NE; p++) {
         w[AW::UL + p] = ubL[p];
         w[AW::UR + p] = ghost ? extra[p] : ubR[p];
     }
 #pragma unroll
-    for (int q = 0; q < NT; q++) w[AW::TQ + q] = tqh[q];
-#pragma unroll
-    for (int d = 0; d < DIM; d++) w[AW::VL + d] = velh[d];
+    for (int d = 0; d < DIM; d++) {
+        w[AW::H + d] = h[d];
+        w[AW::VL + d] = velh[d];
+    }
+    w[AW::E] = 0.5 * g[kRhoE];
     w[AW::CL] = cL;
     w[AW::CR] = cR;
     w[AW::CD] = cdf;
     w[AW::RH] = rhob;
 #pragma unroll
-    for (int q = 0; q < NFIX; q++) W[64 * q] = make_double2(w[2 * q], w[2 * q + 1]);
+    for (int q = 0; q < NFIX; q++)
+        if (2 * q < AW::CL || ns) W[64 * q] = make_double2(w[2 * q], w[2 * q + 1]);
 }
 
 // Reverse of one component's limited least-squares gradient g = phi(G) G, G = sum_k w_k (u_n - u_c), given the
@@ -2626,8 +2638,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     // the record pairs a cell needs of a face: its side's face-state adjoint, the viscous terms and face velocity, the
     // face density adjoint
     constexpr int NPS = (NE + 1) / 2;  // pairs covering NE words from either parity
-    constexpr int V0 = AW::TQ / 2, V1 = (AW::VL + DIM - 1) / 2;
-    double sd[2][2 * NPS], vw[2][2 * (V1 - V0 + 1)], rh[2];  // two slots in flight, as in gradients_body
+    constexpr int V0 = AW::H / 2, V1 = (AW::VL + DIM - 1) / 2;
+    // two slots in flight, as in gradients_body
+    double sd[2][2 * NPS], vw[2][2 * (V1 - V0 + 1)], rh[2], nh[2][3], area[2];
+    int32_t geo[VISC ? KM : 1];
+    if (VISC)
+#pragma unroll
+        for (int k = 0; k < KM; k++) geo[k] = (int32_t)geometry_row(m, (valid[k] ? e[k] : e[0]) >> 1);
     auto load_face = [&](int k) {
         // a padding slot reads the cell's first face and counts it zero times
         const double2* __restrict__ rec = W + face_pair((valid[k] ? e[k] : e[0]) >> 1, b.nwp);
@@ -2645,8 +2662,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
                 vw[k & 1][2 * (q - V0)] = v.x;
                 vw[k & 1][2 * (q - V0) + 1] = v.y;
             }
-        const double2 rp = rec[64 * (AW::RH / 2)];
-        rh[k & 1] = (AW::RH & 1) ? rp.y : rp.x;
+        if (VISC) {
+            load_face_na(m.fna, geo[k], nh[k & 1], area[k & 1]);
+            const double2 rp = rec[64 * (ph.ns ? AW::RH / 2 : V1)];  // a record without species ends at V1
+            rh[k & 1] = ph.ns ? ((AW::RH & 1) ? rp.y : rp.x) : 0.0;
+        }
         if (RECON) slot_vec(m.slim, DIM, k, xs[k]);
     };
     load_face(0);
@@ -2667,10 +2687,20 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
                 for (int d = 0; d < DIM; d++) gb[p][d] += v * xs[k][d];
         }
         if (VISC) {
+            double na[DIM];
 #pragma unroll
-            for (int q = 0; q < NT; q++) tqb[q] += count * vw[h][AW::TQ + q - 2 * V0];
+            for (int d = 0; d < DIM; d++) {
+                na[d] = -count * (area[h] * nh[h][d]);
+                velb[d] += count * vw[h][AW::VL + d - 2 * V0];
+            }
+            constexpr int NTAU = ViscTerms<DIM>::NTAU;
 #pragma unroll
-            for (int d = 0; d < DIM; d++) velb[d] += count * vw[h][AW::VL + d - 2 * V0];
+            for (int i = 0; i < DIM; i++) {
+                // sym_index(i, i) is one term: both halves of the outer product's diagonal go into it
+#pragma unroll
+                for (int j = 0; j < DIM; j++) tqb[sym_index(DIM, i, j)] += na[j] * vw[h][AW::H + i - 2 * V0];
+                tqb[NTAU + i] += na[i] * vw[h][AW::E - 2 * V0];
+            }
             rhob += count * rh[h];
         }
         pin(ub);
