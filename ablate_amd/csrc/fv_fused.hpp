@@ -25,7 +25,7 @@
 // Per-tile lists of the fused strategy (built on the host by build_fused_tiles).
 struct FusedView {
     const int32_t* __restrict__ fstart;  // [n + 1]: faces of tile t at [fstart[t], fstart[t + 1])
-    const int32_t* __restrict__ ffaces;  // face numbers, ascending within a tile
+    const int32_t* __restrict__ ffaces;  // face numbers, in the mesh's order within a tile
     const int32_t* __restrict__ fcode;   // per tile face: left side code | right side code << 16
     const int32_t* __restrict__ fslot;   // [KM][NI]: tile-local face index << 1 | side, -1 padding
     const int32_t* __restrict__ hstart;  // [n + 1]: halo cells of tile t at [hstart[t], hstart[t + 1])

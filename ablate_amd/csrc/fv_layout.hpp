@@ -29,6 +29,15 @@ struct Layout {
     std::vector<double> fwa;       // [F][2][dim] (empty: same as fw)
     std::vector<double> inv_vol;   // [N]
     std::vector<BoundaryFace> bfaces;
+    std::vector<int32_t> face_src;  // [F] the mesh's number of each face, or empty: the mesh's order (face_order)
+};
+
+// The mesh's order of two faces of the layout.
+struct FaceBefore {
+    const Layout& L;
+    bool operator()(int64_t a, int64_t b) const {
+        return L.face_src.empty() ? a < b : L.face_src[(size_t)a] < L.face_src[(size_t)b];
+    }
 };
 
 // Validates the descriptor and fills the layout; throws std::invalid_argument on bad input.
@@ -82,7 +91,7 @@ bool distinct_rows(int64_t n, int width, Fetch&& fetch, std::vector<uint16_t>& i
 }
 
 // Cell tiles for the fused face-flux + gather kernel: tile t owns interior cells [t*T, min((t+1)*T, NI)).
-//   start[t] .. start[t+1]   its faces (every face with a cell in the tile), ascending face number
+//   start[t] .. start[t+1]   its faces (every face with a cell in the tile), in the mesh's face order
 //   slot[k * NI + c]         (tile-local index of the k-th face of c) << 1 | side, -1 padding; KM slots
 //   nf_max                   largest face count of a tile (sizes the workgroup's LDS)
 struct Tiles {
@@ -95,7 +104,7 @@ void build_tiles(const Layout& L, int KM, int T, Tiles& out);
 
 // Cell tiles of the fused strategy (gradients + face fluxes + gather in one kernel): tile t owns interior cells
 // [t*T, min((t+1)*T, NI)); its halo is the interior cells outside the tile that share a face with it.
-//   fstart / ffaces   the tile's faces (every face with a cell in the tile), ascending face number
+//   fstart / ffaces   the tile's faces (every face with a cell in the tile), in the mesh's face order
 //   fcode             per tile face: left side code | right side code << 16; a code is a tile cell's local index,
 //                     T + the halo face entry of that side, or 0xFFFF for a ghost cell
 //   fslot[k * NI + c] (tile-local index of the k-th face of c) << 1 | side, -1 padding; KM slots
@@ -122,7 +131,7 @@ void check_fused_tiles(const Layout& L, int KM, const FusedTiles& ft);
 // the faces between the two.
 //   seq[w] .. seq[w+1]          steps of sequence w; pro[w] its prologue tile or -1
 //   stile[s], snext[s]          tile handled by step s, tile whose records step s computes (-1: none)
-//   fstart / ffaces / fcode     per step: faces evaluated (ascending), side codes lc | rc << 16 with
+//   fstart / ffaces / fcode     per step: faces evaluated (the mesh's order), side codes lc | rc << 16 with
 //                               [0, T) a cur cell, [T, 2T) a next cell, [2T, 2T + nem) a halo entry, 0xFFFF a ghost
 //   pfstart / pffaces / pfcode  per sequence: prologue faces, codes [0, T) first-tile cell, [T, 2T) prologue cell
 //   hstart / hcell / hinfo      per step: halo cells and entries (slot mask | first entry << 8), as FusedTiles

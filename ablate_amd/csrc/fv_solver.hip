@@ -1151,7 +1151,8 @@ __global__ __launch_bounds__(kBlock) void k_gather(MeshView<double> m, int ns, c
 // The same for first-order inviscid species: the face records hold the two species coefficients after the euler fluxes,
 // and each cell forms its faces' species fluxes from its own and its neighbours' densities (k_gather's order and
 // values).  A face then moves 8 words instead of 6 + ns, written once and read twice: 128^3 hexes with ten species,
-// k_face_flux 333 -> 132 us, gather 295 -> 272 us.
+// k_face_flux 333 -> 132 us, gather 295 -> 272 us, and 250 us with the faces in rounds of 64
+// cells (face_order).
 template <int DIM, int KM>
 __global__ __launch_bounds__(kBlock) void k_gather_coef(MeshView<double> m, int ns, const double* __restrict__ U,
                                                         const double* __restrict__ Fe, double* __restrict__ R,
@@ -1965,8 +1966,8 @@ __global__ __launch_bounds__(kBlock) void k_vjp(MeshView<double> m, Phys ph, con
 // reverses the face's flux once for both sides and stores a record of two halves, one per side: the side's euler adjoint
 // and its species multiplier (VjpRec).  k_vjp_gather sums each cell's halves in slot order and forms the species
 // seeds from its own and its neighbours' Rbar, exactly as k_vjp does, so both forms give the same Ubar bit for bit.
-// With the seeds stored as ns more words per face the two kernels took 624 + 387 us at 128^3 hexes with ten species,
-// so 449 + 290 us.
+// With the seeds stored as ns more words per face the two kernels took 624 + 387 us at 128^3 hexes with ten species, in
+// this form 388 + 290 us, and with the faces of boxes in rounds of 64 cells (face_order) 374 + 248 us.
 template <int DIM>
 struct VjpRec {
     static constexpr int SW = (DIM + 4) & ~1;  // words per side: NE adjoints, the multiplier, padding to a pair
@@ -3183,7 +3184,8 @@ __device__ inline double face_interp_value(const double* __restrict__ U, int64_t
 }
 template <int DIM, int KM>
 __global__ __launch_bounds__(kBlock) void k_face_interpolate(MeshView<double> m, Phys ph, const double* __restrict__ U,
-                                                             int nc, double* __restrict__ fsol,
+                                                             int nc, const int32_t* __restrict__ face_src,
+                                                             double* __restrict__ fsol,
                                                              double* __restrict__ fsolg, double* __restrict__ faux,
                                                              double* __restrict__ fauxg) {
     const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -3191,6 +3193,7 @@ __global__ __launch_bounds__(kBlock) void k_face_interpolate(MeshView<double> m,
     const int64_t N = m.N, NI = m.NI, F = m.F;
     const int64_t L = m.fcell[f], R = m.fcell[F + f];
     const bool ghost = R >= NI;
+    const int64_t out = face_src ? face_src[f] : f;  // results are in the mesh's face order
     const int nq = nc + 1 + DIM + ph.ns;
     for (int q = 0; q < nq; q++) {
         const double vL = face_interp_value<DIM, KM>(U, N, nc, ph, q, L);
@@ -3224,13 +3227,14 @@ __global__ __launch_bounds__(kBlock) void k_face_interpolate(MeshView<double> m,
         double* val = q < nc ? fsol : faux;
         double* grd = q < nc ? fsolg : fauxg;
         const int qq = q < nc ? q : q - nc;
-        if (val) val[(int64_t)qq * F + f] = 0.5 * vL + 0.5 * vR;
+        if (val) val[(int64_t)qq * F + out] = 0.5 * vL + 0.5 * vR;
         if (grd)
 #pragma unroll
-            for (int d = 0; d < DIM; d++) grd[((int64_t)qq * DIM + d) * F + f] = g[d];
+            for (int d = 0; d < DIM; d++) grd[((int64_t)qq * DIM + d) * F + out] = g[d];
     }
 }
-using FaceInterpKernel = void (*)(MeshView<double>, Phys, const double*, int, double*, double*, double*, double*);
+using FaceInterpKernel = void (*)(MeshView<double>, Phys, const double*, int, const int32_t*, double*, double*, double*,
+                                  double*);
 template <int DIM>
 FaceInterpKernel pick_face_interpolate(int K) {
     switch (K <= 4 ? 4 : (K <= 6 ? 6 : 8)) {
@@ -3935,7 +3939,7 @@ struct abl_fv_solver {
     int form = 0;
     abl::Layout host;  // metadata only after upload (arrays released)
     abl::Phys ph{};
-    abl::DevBuf<int32_t> ell, fcell, bface, bslot, slot_kind, snbr;
+    abl::DevBuf<int32_t> ell, fcell, bface, bslot, slot_kind, snbr, face_src;
     abl::DevBuf<int2> bcell;  // interior and ghost cell of every boundary face
     abl::DevBuf<double> fna, fdx, fwa, inv_vol, gradC, gradA, slot_state;
     abl::DevBuf<double> sw, swa, slim;  // slot-major gradient geometry (FP64 form)
@@ -4337,7 +4341,7 @@ struct abl_fv_solver {
         return ABL_FV_STRATEGY_FACE_FLUX;
     }
     int64_t device_bytes() const {
-        return (int64_t)(frow.bytes() + srow.bytes() + stab.bytes() + stab_f.bytes() + bcell.bytes() + ell.bytes() + fcell.bytes() + bface.bytes() + bslot.bytes() + slot_kind.bytes() + fna.bytes() + fdx.bytes() + face_flux_e.bytes() + face_flux_s.bytes() + face_flux_m.bytes() + tile_start.bytes() + tile_faces.bytes() + tile_slot.bytes() + fu_start.bytes() + fu_faces.bytes() + fu_code.bytes() + fu_slot.bytes() + fu_hstart.bytes() + fu_hcell.bytes() + fu_hinfo.bytes() + mr_seq.bytes() + mr_pro.bytes() + mr_stile.bytes() + mr_snext.bytes() + mr_fstart.bytes() + mr_ffaces.bytes() + mr_fcode.bytes() + mr_pfstart.bytes() + mr_pffaces.bytes() + mr_pfcode.bytes() + mr_hstart.bytes() + mr_hcell.bytes() + mr_hinfo.bytes() + mr_gslot.bytes() + snbr.bytes() + vjp_rows.bytes() + sw.bytes() + swa.bytes() + slim.bytes() + sw_f.bytes() + swa_f.bytes() + slim_f.bytes() + fwa.bytes() + inv_vol.bytes() + gradC.bytes() +
+        return (int64_t)(face_src.bytes() + frow.bytes() + srow.bytes() + stab.bytes() + stab_f.bytes() + bcell.bytes() + ell.bytes() + fcell.bytes() + bface.bytes() + bslot.bytes() + slot_kind.bytes() + fna.bytes() + fdx.bytes() + face_flux_e.bytes() + face_flux_s.bytes() + face_flux_m.bytes() + tile_start.bytes() + tile_faces.bytes() + tile_slot.bytes() + fu_start.bytes() + fu_faces.bytes() + fu_code.bytes() + fu_slot.bytes() + fu_hstart.bytes() + fu_hcell.bytes() + fu_hinfo.bytes() + mr_seq.bytes() + mr_pro.bytes() + mr_stile.bytes() + mr_snext.bytes() + mr_fstart.bytes() + mr_ffaces.bytes() + mr_fcode.bytes() + mr_pfstart.bytes() + mr_pffaces.bytes() + mr_pfcode.bytes() + mr_hstart.bytes() + mr_hcell.bytes() + mr_hinfo.bytes() + mr_gslot.bytes() + snbr.bytes() + vjp_rows.bytes() + sw.bytes() + swa.bytes() + slim.bytes() + sw_f.bytes() + swa_f.bytes() + slim_f.bytes() + fwa.bytes() + inv_vol.bytes() + gradC.bytes() +
                          gradA.bytes() + rec.bytes() + adjUghost.bytes() + adjUself.bytes() + adjContrib.bytes() + adjW.bytes() + adjGL.bytes() + mirror.bytes() + recf.bytes() + gS_f.bytes() + gY_f.bytes() + rmin.bytes() + cfl_partial.bytes() + dt_partial.bytes() + cfl_out.bytes() + slot_state.bytes() + counter.bytes() + fna_f.bytes() + fdx_f.bytes() +
                          fwa_f.bytes());
     }
@@ -4500,6 +4504,7 @@ extern "C" int abl_fv_create(const abl_fv_mesh_desc* mesh, const abl_fv_physics_
             if (form == ABL_FV_FORM_FP64 && !species && !suth) s->march_kernel = abl::pick_march<2>(s->recon, s->visc, lim, L.K);
         }
 
+        s->face_src.upload(L.face_src);
         s->ell.upload(L.ell);
         s->fcell.upload(L.fcell);
         s->inv_vol.upload(L.inv_vol);
@@ -4661,6 +4666,7 @@ extern "C" int abl_fv_create(const abl_fv_mesh_desc* mesh, const abl_fv_physics_
         // release the host copies of the big arrays
         L.ell.clear(); L.ell.shrink_to_fit();
         L.fcell.clear(); L.fcell.shrink_to_fit();
+        L.face_src.clear(); L.face_src.shrink_to_fit();
         L.fna.clear(); L.fna.shrink_to_fit();
         L.fdx.clear(); L.fdx.shrink_to_fit();
         L.fw.clear(); L.fw.shrink_to_fit();
@@ -4897,12 +4903,15 @@ extern "C" int abl_fv_set_tile_size(abl_fv_handle h, int32_t cells) {
     if (cells != 0 && cells != 64 && cells != 128 && cells != 256 && cells != 512)
         return fail(h, "abl_fv_set_tile_size: cells must be 0 (default), 64, 128, 256 or 512");
     try {
-        // the host copies of the cell -> face table and the face cells were released at creation
+        // the host copies of the cell -> face table, the face cells and the face order were released at creation
         abl::Layout lay = h->host;
         lay.ell.resize(h->ell.n);
         lay.fcell.resize(h->fcell.n);
         HIP_CHECK(hipMemcpy(lay.ell.data(), h->ell.ptr, h->ell.bytes(), hipMemcpyDeviceToHost));
         HIP_CHECK(hipMemcpy(lay.fcell.data(), h->fcell.ptr, h->fcell.bytes(), hipMemcpyDeviceToHost));
+        lay.face_src.resize(h->face_src.n);
+        if (h->face_src.n)
+            HIP_CHECK(hipMemcpy(lay.face_src.data(), h->face_src.ptr, h->face_src.bytes(), hipMemcpyDeviceToHost));
         std::vector<uint16_t> face_rows(h->frow.n);
         if (h->frow.n)
             HIP_CHECK(hipMemcpy(face_rows.data(), h->frow.ptr, h->frow.bytes(), hipMemcpyDeviceToHost));
@@ -5112,8 +5121,8 @@ extern "C" int abl_fv_face_interpolate(abl_fv_handle h, const double* U, double*
         hipStream_t st = (hipStream_t)stream;
         const auto v = h->view();
         const auto kern = L.dim == 3 ? abl::pick_face_interpolate<3>(L.K) : abl::pick_face_interpolate<2>(L.K);
-        hipLaunchKernelGGL(kern, dim3(grid_for(L.F)), dim3(abl::kBlock), 0, st, v, h->ph, U, L.nc, face_sol,
-                           face_sol_grad, face_aux, face_aux_grad);
+        hipLaunchKernelGGL(kern, dim3(grid_for(L.F)), dim3(abl::kBlock), 0, st, v, h->ph, U, L.nc, h->face_src.ptr,
+                           face_sol, face_sol_grad, face_aux, face_aux_grad);
         HIP_CHECK(hipGetLastError());
     } catch (const std::exception& e) {
         return fail(h, std::string("abl_fv_face_interpolate: ") + e.what());
