@@ -1013,10 +1013,7 @@ __global__ __launch_bounds__(kBlock) void k_face_flux(MeshView<double> m, Phys p
 // tile once into LDS (faces shared with a neighbouring tile are evaluated by both), then each lane gathers its
 // cell's faces from LDS in face-number order.  No face-flux round trip through HBM; the face fluxes and the
 // gather order are those of strategy 2, so the residual is bitwise the same.  A tile's face list holds each face's
-// support cells, number and geometry row (TileFace), so that a face's records are one dependent load away.
-struct TileFace {
-    int32_t L, R, f, g;
-};
+// support cells, number and geometry row (an int4), so that a face's records are one dependent load away.
 __device__ inline FaceRef tile_face_ref(const int4& t) { return {t.z, t.x, t.y, t.w}; }
 template <int DIM, bool RECON, bool VISC, bool SPECIES, int KM>
 __global__ __launch_bounds__(kTileMax) void k_tile_flux(MeshView<double> m, Phys ph, const double* __restrict__ U,
@@ -3958,7 +3955,7 @@ struct abl_fv_solver {
     abl::DevBuf<double> face_flux_e, face_flux_s;
     abl::DevBuf<float> face_flux_m;
     abl::DevBuf<int32_t> tile_start, tile_slot;  // tile strategy (built when selected)
-    abl::DevBuf<int4> tile_faces;                // TileFace entries
+    abl::DevBuf<int4> tile_faces;                // left and right cell, face, geometry row
     int tile_T = 0, tile_threads = 0, tile_nfm = 0;
     int64_t tile_n = 0;
     size_t tile_lds = 0;
