@@ -142,23 +142,31 @@ static std::vector<int32_t> face_order(const abl_fv_mesh_desc& m) {
     for (int64_t f = 0; f < F; f++) start[(size_t)(m.face_cells[2 * f] >> 6) + 1]++;
     for (size_t b = 1; b < start.size(); b++) start[b] += start[b - 1];
     std::vector<int64_t> fill(start.begin(), start.end() - 1);
-    std::vector<uint8_t> own((size_t)NI, 0);
-    std::vector<std::pair<int32_t, int32_t>> key((size_t)F);  // (rank << 6) | cell in the block, face
-    for (int64_t f = 0; f < F; f++) {
-        const int32_t c = m.face_cells[2 * f];
-        key[(size_t)fill[(size_t)(c >> 6)]++] = {(own[(size_t)c]++ << 6) | (c & 63), (int32_t)f};
-    }
-    for (size_t b = 0; b + 1 < start.size(); b++) std::sort(key.begin() + start[b], key.begin() + start[b + 1]);
+    std::vector<int32_t> src((size_t)F);
+    for (int64_t f = 0; f < F; f++) src[(size_t)fill[(size_t)(m.face_cells[2 * f] >> 6)]++] = (int32_t)f;
     int64_t runs = 0;
-    for (int64_t i = 1; i < F; i++) {
-        const int32_t* a = m.face_cells + 2 * (int64_t)key[(size_t)i - 1].second;
-        const int32_t* b = m.face_cells + 2 * (int64_t)key[(size_t)i].second;
-        runs += b[0] == a[0] + 1 && b[1] == a[1] + 1;
+    int32_t pl = -2, pr = -2;  // cells of the face before
+    for (size_t b = 0; b + 1 < start.size(); b++) {
+        int32_t at[64 * kMaxFacesPerCell];  // the block's faces by rank and cell
+        uint8_t own[64] = {};
+        int ranks = 0;
+        std::fill(at, at + 64 * kMaxFacesPerCell, -1);
+        for (int64_t i = start[b]; i < start[b + 1]; i++) {
+            const int c = m.face_cells[2 * (int64_t)src[(size_t)i]] & 63;
+            at[64 * own[c] + c] = src[(size_t)i];
+            ranks = std::max(ranks, (int)++own[c]);
+        }
+        int64_t i = start[b];
+        for (int j = 0; j < 64 * ranks; j++) {
+            if (at[j] < 0) continue;
+            const int32_t l = m.face_cells[2 * (int64_t)at[j]], r = m.face_cells[2 * (int64_t)at[j] + 1];
+            runs += l == pl + 1 && r == pr + 1;
+            pl = l;
+            pr = r;
+            src[(size_t)i++] = at[j];
+        }
     }
-    std::vector<int32_t> src;
-    if (2 * runs <= F) return src;
-    src.resize((size_t)F);
-    for (int64_t i = 0; i < F; i++) src[(size_t)i] = key[(size_t)i].second;
+    if (2 * runs <= F) src.clear();
     return src;
 }
 
@@ -312,6 +320,12 @@ void build_layout(const abl_fv_mesh_desc& m, const abl_fv_physics_desc& p, Layou
     }
 }
 
+// Sort key of a layout face in the mesh's order: the mesh's number, then the layout's.
+static int64_t face_key(const Layout& L, int32_t f) {
+    return ((int64_t)(L.face_src.empty() ? f : L.face_src[(size_t)f]) << 32) | f;
+}
+static int32_t face_of_key(int64_t key) { return (int32_t)(key & 0x7FFFFFFF); }
+
 void build_tiles(const Layout& L, int KM, int T, Tiles& out) {
     const int64_t NI = L.NI;
     out.T = T;
@@ -321,31 +335,30 @@ void build_tiles(const Layout& L, int KM, int T, Tiles& out) {
     out.faces.clear();
     out.faces.reserve((size_t)NI * 4);
     out.slot.assign((size_t)KM * NI, -1);
-    // Faces of a tile in the mesh's order (FaceBefore): consecutive lanes then read the records of a cell's faces
+    // Faces of a tile in the mesh's order: consecutive lanes then read the records of a cell's faces
     // together (by rounds of one face per cell, as the layout numbers the faces of boxes, 256^3 hexes take 3.79 instead of
     // 3.69 ms, Navier-Stokes FP64).
-    const FaceBefore before{L};
-    std::vector<int32_t> list;
+    std::vector<int64_t> list;
     for (int64_t t = 0; t < out.n; t++) {
         const int64_t c0 = t * T, c1 = std::min<int64_t>(c0 + T, NI);
         list.clear();
         for (int k = 0; k < L.K; k++)
             for (int64_t c = c0; c < c1; c++) {
                 const int32_t e = L.ell[(size_t)k * NI + c];
-                if (e >= 0) list.push_back(e >> 1);
+                if (e >= 0) list.push_back(face_key(L, e >> 1));
             }
-        std::sort(list.begin(), list.end(), before);
+        std::sort(list.begin(), list.end());
         list.erase(std::unique(list.begin(), list.end()), list.end());
         for (int k = 0; k < L.K; k++)
             for (int64_t c = c0; c < c1; c++) {
                 const int32_t e = L.ell[(size_t)k * NI + c];
                 if (e < 0) continue;
-                const int32_t local = (int32_t)(std::lower_bound(list.begin(), list.end(), e >> 1, before) - list.begin());
+                const int32_t local = (int32_t)(std::lower_bound(list.begin(), list.end(), face_key(L, e >> 1)) - list.begin());
                 out.slot[(size_t)k * NI + c] = (local << 1) | (e & 1);
             }
         if (out.faces.size() + list.size() > (size_t)INT32_MAX)
             throw std::invalid_argument("mesh too large for 32-bit tile face lists");
-        out.faces.insert(out.faces.end(), list.begin(), list.end());
+        for (const int64_t q : list) out.faces.push_back(face_of_key(q));
         out.start[(size_t)t + 1] = (int32_t)out.faces.size();
         out.nf_max = std::max(out.nf_max, (int)list.size());
     }
@@ -370,22 +383,24 @@ void build_fused_tiles(const Layout& L, int KM, int T, FusedTiles& out) {
     out.ffaces.reserve((size_t)NI * 4);
     out.fcode.reserve((size_t)NI * 4);
     out.fslot.assign((size_t)KM * NI, -1);
-    const FaceBefore before{L};
     std::vector<int32_t> list, halo, entry;
+    std::vector<int64_t> key;  // of the list's faces
     auto local_face = [&](int32_t f) {
-        return (int32_t)(std::lower_bound(list.begin(), list.end(), f, before) - list.begin());
+        return (int32_t)(std::lower_bound(key.begin(), key.end(), face_key(L, f)) - key.begin());
     };
     for (int64_t t = 0; t < out.n; t++) {
         const int64_t c0 = t * T, c1 = std::min<int64_t>(c0 + T, NI);
         auto own = [&](int64_t c) { return c >= c0 && c < c1; };
-        list.clear();
+        key.clear();
         for (int k = 0; k < L.K; k++)
             for (int64_t c = c0; c < c1; c++) {
                 const int32_t e = L.ell[(size_t)k * NI + c];
-                if (e >= 0) list.push_back(e >> 1);
+                if (e >= 0) key.push_back(face_key(L, e >> 1));
             }
-        std::sort(list.begin(), list.end(), before);
-        list.erase(std::unique(list.begin(), list.end()), list.end());
+        std::sort(key.begin(), key.end());
+        key.erase(std::unique(key.begin(), key.end()), key.end());
+        list.clear();
+        for (const int64_t q : key) list.push_back(face_of_key(q));
         // halo: interior cells across the tile's faces that are not tile cells
         halo.clear();
         for (int32_t f : list)
