@@ -32,12 +32,13 @@ struct Layout {
     std::vector<int32_t> face_src;  // [F] the mesh's number of each face, or empty: the mesh's order (face_order)
 };
 
-// The mesh's order of two faces of the layout.
+// Sort key of a layout face in the mesh's order: the mesh's number, then the layout's.
+inline int64_t face_key(const Layout& L, int32_t f) {
+    return ((int64_t)(L.face_src.empty() ? f : L.face_src[(size_t)f]) << 32) | f;
+}
 struct FaceBefore {
     const Layout& L;
-    bool operator()(int64_t a, int64_t b) const {
-        return L.face_src.empty() ? a < b : L.face_src[(size_t)a] < L.face_src[(size_t)b];
-    }
+    bool operator()(int64_t a, int64_t b) const { return face_key(L, (int32_t)a) < face_key(L, (int32_t)b); }
 };
 
 // Validates the descriptor and fills the layout; throws std::invalid_argument on bad input.
