@@ -3949,6 +3949,7 @@ struct abl_fv_solver {
     const int32_t* halt = nullptr;  // set while abl_fv_ts_euler enqueues steps (MeshView::halt)
     bool slot_rows = false;
     abl::DevBuf<double> rec;            // cell records of the FP64 form (rec_pair blocks)
+    abl::DevBuf<double> U_copy, Rbar_copy;  // inputs of calls in place (apart; the first such call allocates)
     // face fluxes (allocated when that strategy is selected): FP64 euler records [F][FS] and species pairs
     // [ns/2][F][2];
     // mixed form rows [2 (n_euler + n_species)][F]
@@ -4125,6 +4126,14 @@ struct abl_fv_solver {
         v.halt = halt;
         v.rec_swap = rec_swap;
         return v;
+    }
+    // `in`, or a copy of it where the call's output is to take its place: the kernels read neighbours' rows of their
+    // inputs while others write theirs.
+    const double* apart(const double* in, const double* out, abl::DevBuf<double>& copy, hipStream_t st) {
+        if (in != out) return in;
+        if (!copy.ptr) copy.alloc((size_t)host.nc * host.N);
+        HIP_CHECK(hipMemcpyAsync(copy.ptr, in, copy.bytes(), hipMemcpyDeviceToDevice, st));
+        return copy.ptr;
     }
     abl::GhostView ghost_view() const {
         return {n_bfaces, host.N, host.nc, bcell.ptr, bslot.ptr, slot_kind.ptr, slot_state.ptr};
@@ -4338,7 +4347,7 @@ struct abl_fv_solver {
         return ABL_FV_STRATEGY_FACE_FLUX;
     }
     int64_t device_bytes() const {
-        return (int64_t)(face_src.bytes() + frow.bytes() + srow.bytes() + stab.bytes() + stab_f.bytes() + bcell.bytes() + ell.bytes() + fcell.bytes() + bface.bytes() + bslot.bytes() + slot_kind.bytes() + fna.bytes() + fdx.bytes() + face_flux_e.bytes() + face_flux_s.bytes() + face_flux_m.bytes() + tile_start.bytes() + tile_faces.bytes() + tile_slot.bytes() + fu_start.bytes() + fu_faces.bytes() + fu_code.bytes() + fu_slot.bytes() + fu_hstart.bytes() + fu_hcell.bytes() + fu_hinfo.bytes() + mr_seq.bytes() + mr_pro.bytes() + mr_stile.bytes() + mr_snext.bytes() + mr_fstart.bytes() + mr_ffaces.bytes() + mr_fcode.bytes() + mr_pfstart.bytes() + mr_pffaces.bytes() + mr_pfcode.bytes() + mr_hstart.bytes() + mr_hcell.bytes() + mr_hinfo.bytes() + mr_gslot.bytes() + snbr.bytes() + vjp_rows.bytes() + sw.bytes() + swa.bytes() + slim.bytes() + sw_f.bytes() + swa_f.bytes() + slim_f.bytes() + fwa.bytes() + inv_vol.bytes() + gradC.bytes() +
+        return (int64_t)(face_src.bytes() + frow.bytes() + srow.bytes() + stab.bytes() + stab_f.bytes() + bcell.bytes() + U_copy.bytes() + Rbar_copy.bytes() + ell.bytes() + fcell.bytes() + bface.bytes() + bslot.bytes() + slot_kind.bytes() + fna.bytes() + fdx.bytes() + face_flux_e.bytes() + face_flux_s.bytes() + face_flux_m.bytes() + tile_start.bytes() + tile_faces.bytes() + tile_slot.bytes() + fu_start.bytes() + fu_faces.bytes() + fu_code.bytes() + fu_slot.bytes() + fu_hstart.bytes() + fu_hcell.bytes() + fu_hinfo.bytes() + mr_seq.bytes() + mr_pro.bytes() + mr_stile.bytes() + mr_snext.bytes() + mr_fstart.bytes() + mr_ffaces.bytes() + mr_fcode.bytes() + mr_pfstart.bytes() + mr_pffaces.bytes() + mr_pfcode.bytes() + mr_hstart.bytes() + mr_hcell.bytes() + mr_hinfo.bytes() + mr_gslot.bytes() + snbr.bytes() + vjp_rows.bytes() + sw.bytes() + swa.bytes() + slim.bytes() + sw_f.bytes() + swa_f.bytes() + slim_f.bytes() + fwa.bytes() + inv_vol.bytes() + gradC.bytes() +
                          gradA.bytes() + rec.bytes() + adjUghost.bytes() + adjUself.bytes() + adjContrib.bytes() + adjW.bytes() + adjGL.bytes() + mirror.bytes() + recf.bytes() + gS_f.bytes() + gY_f.bytes() + rmin.bytes() + cfl_partial.bytes() + dt_partial.bytes() + cfl_out.bytes() + slot_state.bytes() + counter.bytes() + fna_f.bytes() + fdx_f.bytes() +
                          fwa_f.bytes());
     }
@@ -4364,14 +4373,20 @@ std::string unset_boundary(abl_fv_handle h) {
     return std::string();
 }
 
-// theta_bar is the adjoint of the inflow states: with no inflow slot every contribution is zero and the theta_bar
-// passes (and their copy back to the host) are skipped.
 // Ghost rows of U from the boundary conditions; zeros in the ghost rows of Z (null: none).
 void fill_ghosts(abl_fv_handle h, hipStream_t st, double* U, double* Z) {
     hipLaunchKernelGGL(abl::k_ghost_fill, dim3(grid_for(h->n_bfaces), (unsigned)h->host.nc), dim3(abl::kBlock), 0, st,
                        h->ghost_view(), U, Z, h->halt);
 }
+void zero_ghost_rows(abl_fv_handle h, hipStream_t st, double* Z) {
+    const abl::Layout& L = h->host;
+    if (L.N > L.NI)
+        hipLaunchKernelGGL(abl::k_zero_rows, dim3(grid_for((L.N - L.NI) * L.nc)), dim3(abl::kBlock), 0, st, Z, L.N, L.NI,
+                           L.nc);
+}
 
+// theta_bar is the adjoint of the inflow states: with no inflow slot every contribution is zero and the theta_bar
+// passes (and their copy back to the host) are skipped.
 bool has_inflow(abl_fv_handle h) {
     for (int v : h->bc_slots)
         if (h->h_slot_kind[v] == ABL_FV_BC_INFLOW) return true;
@@ -4755,7 +4770,7 @@ extern "C" int abl_fv_set_boundary(abl_fv_handle h, int32_t slot, const abl_fv_b
 
 namespace {
 // The kernels of one right-hand side after the ghost fill.
-void launch_rhs(abl_fv_handle h, double* U, double* R, int32_t accumulate, hipStream_t st) {
+void launch_rhs(abl_fv_handle h, const double* U, double* R, int32_t accumulate, hipStream_t st) {
     const abl::Layout& L = h->host;
     const dim3 grid(grid_for(L.NI)), block(abl::kBlock);
     if (h->form == ABL_FV_FORM_MIXED) {
@@ -4855,8 +4870,9 @@ extern "C" int abl_fv_rhs(abl_fv_handle h, double time, double* U, double* R, in
     try {
         hipStream_t st = (hipStream_t)stream;
         if (h->n_bfaces)
-            h->timed(ABL_FV_PHASE_GHOST, st, [&] { fill_ghosts(h, st, U, accumulate ? nullptr : R); });
-        launch_rhs(h, U, R, accumulate, st);
+            h->timed(ABL_FV_PHASE_GHOST, st, [&] { fill_ghosts(h, st, U, accumulate || R == U ? nullptr : R); });
+        launch_rhs(h, h->apart(U, R, h->U_copy, st), R, accumulate, st);
+        if (R == U && !accumulate) zero_ghost_rows(h, st, R);
     } catch (const std::exception& e) {
         return fail(h, std::string("abl_fv_rhs: ") + e.what());
     }
@@ -4984,7 +5000,7 @@ int vjp_second_order(abl_fv_handle h, double* U, const double* Rbar, double* Uba
         }
         const dim3 grid(grid_for(L.NI)), block(abl::kBlock);
         if (h->n_bfaces)
-            h->timed(ABL_FV_PHASE_GHOST, st, [&] { fill_ghosts(h, st, U, Ubar); });
+            h->timed(ABL_FV_PHASE_GHOST, st, [&] { fill_ghosts(h, st, U, Ubar == U ? nullptr : Ubar); });
         const auto v = h->view();
         h->timed(ABL_FV_PHASE_GRADIENTS, st, [&] {
             hipLaunchKernelGGL(h->grad_kernel, grid, block, 0, st, v, h->ph, U, h->gradC.ptr, h->gradA.ptr,
@@ -5004,6 +5020,7 @@ int vjp_second_order(abl_fv_handle h, double* U, const double* Rbar, double* Uba
             hipLaunchKernelGGL(h->adj_gather, grid, block, 0, st, v, h->ph, h->ghost_slot.ptr, h->slot_kind.ptr, b,
                                Ubar);
         });
+        if (Ubar == U) zero_ghost_rows(h, st, Ubar);
         if (NG > 0) {
             hipLaunchKernelGGL(abl::k_ghost_adjoint_out, dim3(grid_for(NG)), block, 0, st, NG, L.N, L.NI, L.nc,
                                h->ghost_slot.ptr, h->slot_kind.ptr, h->adjUghost.ptr, Ubar);
@@ -5062,7 +5079,7 @@ extern "C" int abl_fv_rhs_vjp(abl_fv_handle h, double time, double* U, const dou
 namespace {
 // First-order VJP (ghost fill, ghost rows of Ubar, the VJP kernels, theta_bar) with the theta_bar workspace
 // supplied by the caller: contrib [3 n_bfaces] and sums [3 kMaxBcSlots] device doubles (written in full before they
-// are read).  rows [2 NE + 2 + ns][F]: the face-centric kernels (each face reversed once); null: the cell-centric kernel
+// are read).  rows (VjpRec records): the face-centric kernels (each face reversed once); null: the cell-centric kernel
 // (each face reversed by both of its cells, no workspace).  Both give the same Ubar bit for bit.
 int vjp_first_order(abl_fv_handle h, double* U, const double* Rbar, double* Ubar, double* theta_bar, double* contrib,
                     double* sums, double* rows, hipStream_t st, const char* who) {
@@ -5071,7 +5088,13 @@ int vjp_first_order(abl_fv_handle h, double* U, const double* Rbar, double* Ubar
     try {
         if (h->n_bfaces) {
             // the ghost rows of Ubar are zeroed first: the VJP kernel then writes those of caller-filled ghosts
-            h->timed(ABL_FV_PHASE_GHOST, st, [&] { fill_ghosts(h, st, U, Ubar); });
+            h->timed(ABL_FV_PHASE_GHOST, st, [&] { fill_ghosts(h, st, U, Ubar == U ? nullptr : Ubar); });
+        }
+        const double* state = U;
+        if (rows) {  // (the allocation-free form takes separate buffers only)
+            state = h->apart(U, Ubar, h->U_copy, st);
+            Rbar = h->apart(Rbar, Ubar, h->Rbar_copy, st);
+            if (Ubar == U) zero_ghost_rows(h, st, Ubar);
         }
         const dim3 grid(grid_for(L.NI)), block(abl::kBlock);
         const bool noflux = fl == ABL_FV_FLUX_OFF || fl == ABL_FV_FLUX_NONE;
@@ -5081,11 +5104,11 @@ int vjp_first_order(abl_fv_handle h, double* U, const double* Rbar, double* Ubar
             const auto v = h->view();
             h->timed(ABL_FV_PHASE_VJP, st, [&] {
                 if (rows) {
-                    hipLaunchKernelGGL(h->vjp_faces, dim3(grid_for(L.F)), block, 0, st, v, h->ph, U, Rbar, rows);
+                    hipLaunchKernelGGL(h->vjp_faces, dim3(grid_for(L.F)), block, 0, st, v, h->ph, state, Rbar, rows);
                     hipLaunchKernelGGL(h->vjp_gather, grid, block, 0, st, v, h->ph, Rbar, rows, h->ghost_slot.ptr,
                                        h->slot_kind.ptr, Ubar);
                 } else {
-                    hipLaunchKernelGGL(h->vjp_kernel, grid, block, 0, st, v, h->ph, U, Rbar, h->ghost_slot.ptr,
+                    hipLaunchKernelGGL(h->vjp_kernel, grid, block, 0, st, v, h->ph, state, Rbar, h->ghost_slot.ptr,
                                        h->slot_kind.ptr, Ubar);
                 }
             });
@@ -5093,7 +5116,7 @@ int vjp_first_order(abl_fv_handle h, double* U, const double* Rbar, double* Ubar
         HIP_CHECK(hipGetLastError());
         if (theta_bar && h->n_bfaces && !noflux && has_inflow(h)) {
             const auto v = h->view();
-            hipLaunchKernelGGL(h->vjp_theta_kernel, dim3(grid_for(h->n_bfaces)), block, 0, st, v, h->ph, U, Rbar,
+            hipLaunchKernelGGL(h->vjp_theta_kernel, dim3(grid_for(h->n_bfaces)), block, 0, st, v, h->ph, state, Rbar,
                                h->n_bfaces, h->bface.ptr, h->bslot.ptr, h->slot_kind.ptr, h->slot_param.ptr,
                                h->slot_Y.ptr, contrib);
             HIP_CHECK(hipGetLastError());

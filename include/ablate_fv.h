@@ -235,7 +235,8 @@ int abl_fv_set_boundary(abl_fv_handle h, int32_t slot, const abl_fv_bc_desc* bc)
  * the residual is ADDED into R (reference semantics: locF is zeroed by the caller, timeStepper.cpp:363, and
  * ComputeRHSFunction adds into it); with accumulate = 0, R = rhs.  Ghost rows of R are left untouched
  * (accumulate = 1) or zeroed.  `time` is the time the caller's ghost values belong to; the constant-state
- * conditions do not depend on it.  Fails before any device work when a boundary slot has no condition. */
+ * conditions do not depend on it.  Fails before any device work when a boundary slot has no condition.  R may be U: the
+ * state is then copied first, into memory that the first such call allocates. */
 int abl_fv_rhs(abl_fv_handle h, double time, double* U, double* R, int32_t accumulate, abl_fv_stream stream);
 
 /* Vector-Jacobian product of the RHS (build-defined; the reference has no adjoint):
@@ -248,7 +249,8 @@ int abl_fv_rhs(abl_fv_handle h, double time, double* U, double* R, int32_t accum
  *   for the FP64 form with the
  *   Ausm, Rusanov or Off calculators, first order or least squares with the Barth-Jespersen limiter (or none),
  *   viscous and species fluxes; the first call allocates its workspace (first order: 2 (n_euler + 1
- *   rounded up to even) doubles per face). */
+ *   rounded up to even) doubles per face).  Ubar may be U or Rbar (first order: copied first, into memory that the first
+ *   such call allocates). */
 int abl_fv_rhs_vjp(abl_fv_handle h, double time, double* U, const double* Rbar, double* Ubar, double* theta_bar,
                    abl_fv_stream stream);
 
@@ -267,7 +269,8 @@ int abl_fv_face_interpolate(abl_fv_handle h, const double* U, double* face_sol, 
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  Same arguments and results as
  * abl_fv_rhs_vjp (bitwise), for first-order inviscid FP64 handles with at most 262144 boundary faces; it allocates
  * nothing: the theta_bar workspace lives in a static per-GPU device array.  Calls that overlap on one GPU race on
- * that array: serialise them.  Fails (nonzero, message in abl_fv_last_error) for other handles or larger meshes. */
+ * that array: serialise them.  Ubar must be a buffer of its own.  Fails (nonzero, message in abl_fv_last_error) for
+ * other handles or larger meshes. */
 int abl_fv_rhs_vjp_noalloc(abl_fv_handle h, double time, double* U, const double* Rbar, double* Ubar,
                            double* theta_bar, abl_fv_stream stream);
 
