@@ -424,8 +424,7 @@ class FiniteVolumeSolver:
     def compute_rhs(self, time: float, U, R, accumulate: bool = False, stream=None) -> None:
         self._check_tensor(U, "U")
         self._check_tensor(R, "R")
-        if self._ghosts:
-            self.insert_boundary_values(time, U)
+        self.insert_boundary_values(time, U)
         status = self._rhs(self._h, float(time), U.data_ptr(), R.data_ptr(), 1 if accumulate else 0,
                            self._stream_ptr(stream))
         if status:
