@@ -4066,13 +4066,18 @@ struct abl_fv_solver {
         }
         pending.clear();
     }
+    // Forgets the pending events from index `first` on (launches that found nothing to do).
+    void drop_events(size_t first) {
+        for (size_t i = first; i < pending.size(); i++) {
+            (void)hipEventSynchronize(pending[i].stop);
+            (void)hipEventDestroy(pending[i].start);
+            (void)hipEventDestroy(pending[i].stop);
+        }
+        if (first < pending.size()) pending.resize(first);
+    }
     ~abl_fv_solver() {
         if (ts_host) (void)hipHostFree(ts_host);
-        for (auto& e : pending) {
-            (void)hipEventSynchronize(e.stop);
-            (void)hipEventDestroy(e.start);
-            (void)hipEventDestroy(e.stop);
-        }
+        drop_events(0);
     }
 
     abl::MeshView<double> view() const {
@@ -5387,7 +5392,10 @@ int ts_euler_device(abl_fv_handle h, double* U, double* R, double t0, double max
             const double left = std::ceil((max_time - k.t) / k.dt) + 1.0;
             int64_t batch = std::min(max_steps - k.steps, kMaxBatch);
             if (left < (double)batch) batch = std::max<int64_t>(1, (int64_t)left);
+            size_t events[kMaxBatch];  // pending events before each step
+            const int64_t before = k.steps;
             for (int64_t i = 0; i < batch; i++) {
+                events[i] = h->pending.size();
                 if (i > 0 && merged) {
                     h->timed(ABL_FV_PHASE_GHOST, st, [&] {
                         hipLaunchKernelGGL(abl::k_ts_advance_ghosts, dim3(grid_for(h->n_bfaces), (unsigned)L.nc),
@@ -5409,6 +5417,7 @@ int ts_euler_device(abl_fv_handle h, double* U, double* R, double t0, double max
             HIP_CHECK(hipGetLastError());
             HIP_CHECK(hipStreamSynchronize(st));
             k = *h->ts_host;
+            if (k.steps - before < batch) h->drop_events(events[k.steps - before]);  // steps past the end
         }
         if (k.bad) throw std::runtime_error("non-positive or NaN step size at t = " + std::to_string(k.t));
         if (t_out) *t_out = k.t;

@@ -382,7 +382,8 @@ enum {
     ABL_FV_PHASE_GATHER = 5,
     ABL_FV_N_PHASES = 6
 };
-/* When enabled, every kernel of abl_fv_rhs / abl_fv_rhs_vjp is bracketed by events on its stream. */
+/* When enabled, every kernel of abl_fv_rhs / abl_fv_rhs_vjp is bracketed by events on its stream.  abl_fv_ts_euler counts
+ * the steps it takes; on meshes with boundaries the end of a step shares the next step's ghost launch and its time. */
 int abl_fv_set_profiling(abl_fv_handle h, int32_t enable);
 /* Accumulated device milliseconds and launch counts per phase since the last reset (waits for the events). */
 int abl_fv_get_phase_times(abl_fv_handle h, double* ms, int64_t* launches, int32_t reset);

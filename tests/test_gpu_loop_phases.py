@@ -1,0 +1,34 @@
+"""Phase counts of abl_fv_ts_euler: one launch per phase and step taken, none for the steps that its device loop enqueues
+past the end of the run, which the step sizes decide."""
+import pytest
+import torch
+
+from ablate_amd.mesh import BoxMesh
+from tests.fvcases import Case, inflow_x
+
+pytestmark = pytest.mark.gpu
+
+NS = dict(recon="leastsquares", limiter="barthjespersen", mu=0.05, k=0.5)
+CASES = {
+    "open_2d": lambda: Case("a", BoxMesh([19, 8], [0, 0], [1, 1], [False, True]), state="random2d", bcs=inflow_x()),
+    "periodic_ns": lambda: Case("b", BoxMesh([7, 6, 5], [0, 0, 0], [1, 1, 1], [True] * 3), **NS),
+}
+
+
+@pytest.mark.parametrize("steps", [3.4, 300.7])  # the last two steps halve what is left; more than one batch
+@pytest.mark.parametrize("name", CASES)
+def test_phases_count_the_steps_taken(name, steps, torch_cuda):
+    case = CASES[name]()
+    solver = case.solver()
+    U = torch.tensor(case.initial_state(), device="cuda")
+    max_time, V = steps * solver.ComputePhysicsTimeStep(U), U.clone()
+    solver.phase_times()
+    solver.set_profiling(True)
+    _, n = solver.ts_euler(U, max_time)
+    counts = {phase: launches for phase, (_, launches) in solver.phase_times().items()}
+    assert counts["flux"] == n
+    assert counts["ghost"] == (n if case.mesh.n_cells > case.mesh.n_interior else 0)
+    assert counts["gradients"] == (n if case.recon != "upwind" else 0)
+    solver.set_profiling(False)
+    _, n = solver.ts_euler(V, max_time, max_steps=2)
+    assert n == 2 and all(launches == 0 for _, launches in solver.phase_times().values())
