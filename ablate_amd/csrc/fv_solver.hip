@@ -4171,14 +4171,17 @@ struct abl_fv_solver {
                                                       : 2 * (lay.dim + 2 + lay.ns) * (int)sizeof(float);
         abl::Tiles tl;
         const size_t budget = only_T ? (size_t)abl::kTileLdsMax : (size_t)abl::kTileLdsDefault;
-        // Fewer than two default tiles per CU leave the chip part empty and one tile's rounds of faces a serial chain:
-        // small meshes take 64-cell tiles, and tiles of any size 256 lanes while there are at most four workgroups per
-        // CU (41 x 36 x 29 hexes, Navier-Stokes FP64: 16.3 us with 256-cell tiles, 13.3 us so; 96 x 90 x 77: 104.8 us
-        // with 256-cell tiles, 113.9 us with 64-cell tiles of 256 lanes).
+        // Few default tiles per CU leave the chip part empty and one tile's rounds of faces a serial chain: meshes of up to
+        // one and a half per CU (98304 cells) take 64-cell tiles, and tiles of any size 256 lanes while there are at most
+        // four workgroups per CU.  Whole calls with 64- and 256-cell tiles, us: 36720 hexes first order 5.4 / 6.8,
+        // Navier-Stokes FP64 18.7 / 21.7, mixed 15.6 / 19.2; 68880: 8.6 / 9.0, 27.3 / 30.0, 24.1 / 25.6; 95220: 9.5 / 9.2,
+        // 29.2 / 30.5, 26.5 / 26.2; 108000: 9.6 / 9.3, 30.9 / 30.9, 26.6 / 26.4; 130050: 10.6 / 9.9, 34.5 / 33.2, 28.4 / 27.0,
+        // with three species 68.4 / 60.1 (Navier-Stokes FP64); 665280: tile pass 113.9 / 104.8.  128-cell tiles of 256
+        // lanes are up to 13 % faster than either on hexes of 65536 to 131072 cells and up to 13 % slower on quads.
         int dev = 0, cus = 256;
         HIP_CHECK(hipGetDevice(&dev));
         HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        const int T0 = (lay.NI + abl::kTileDefault - 1) / abl::kTileDefault < 2 * cus ? 64 : abl::kTileDefault;
+        const int T0 = 2 * lay.NI <= 3 * (int64_t)abl::kTileDefault * cus ? 64 : abl::kTileDefault;
         for (int T = only_T ? only_T : T0; T >= 64; T /= 2) {
             abl::build_tiles(lay, KM, T, tl);
             if ((size_t)tl.nf_max * per_face <= budget) break;
@@ -4341,6 +4344,10 @@ struct abl_fv_solver {
     // LDS footprint leaves at least two waves per SIMD for latency hiding; cell orders with little locality within
     // a tile (bandwidth-reducing orders of unstructured meshes: ~2 evaluations per face) and wide species LDS rows
     // go to face flux.
+    // The waves are those of a tile's cells, also where small tiles get more lanes.  Tiles and face fluxes, us: Navier-Stokes
+    // FP64, 16 x 15 x 14 hexes, six species 29.6 / 27.6, ten 36.0 / 32.6; 32 x 31 x 30: 37.3 / 34.2 and 44.7 / 39.6; 48 x 47 x 46:
+    // 92 / 60 and 115 / 71.  First-order small meshes would do better by lanes (63960 hexes, five species 9.2 / 14.0, ten 12.0 /
+    // 17.6), larger ones not (132600 hexes, six species 25.0 / 23.6 with 128-cell tiles; 99452, mixed, ten 33.1 / 28.6).
     // The fused strategy is offered on request only: on the 256^3 hex workload it took 8.3 ms per RHS against
     // 5.3 ms for gradients + tiles (two workgroups per CU by LDS and registers; its phases wait on memory).
     int auto_strategy() const {
