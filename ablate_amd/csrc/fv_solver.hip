@@ -2586,8 +2586,17 @@ __device__ __forceinline__ void limited_lsq_vjp(const double* unv, double uc, co
 // for hexes; with all neighbours' states and all contributions live they took 288 VGPRs, one wave per SIMD, and a
 // branch per slot made the record loads of the six slots six dependent rounds).  The density comes last: the other
 // components' aux terms add to it.
+// The slots' weights and limiter vectors stay in registers for four slots and are read again for each component for more,
+// where they come from the geometry tables' cache lines.  Without tables those reads go past L2 (2 KB per cell): such
+// hexes and cells with up to eight faces keep them too where the aux terms read weights as well (without those, 182 to 256
+// VGPRs, reading again is no slower), at one wave per SIMD (282 VGPRs).  Whole adjoint of jittered hexes, Navier-Stokes:
+// read again / kept at two waves per SIMD / at one: 41 x 36 x 29 90 / 52 / 45 us, 100 x 75 x 61 600 / 402 / 363 us, 96 x 90 x
+// 77 846 / 570 / 535 us; 80 x 75 x 61 cells of eight faces 703 / - / 385 us.
+template <int KM, bool RECON, bool VISC, bool TAB>
+constexpr bool kAdjKeepVectors = KM <= 4 || (RECON && VISC && !TAB);
 template <int DIM, int KM, bool RECON, bool VISC, bool TAB>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_adj_cells_e(
+__global__ __launch_bounds__(kBlock)
+__attribute__((amdgpu_waves_per_eu(KM > 4 && kAdjKeepVectors<KM, RECON, VISC, TAB> ? 1 : 2))) void k_adj_cells_e(
     MeshView<double> m, Phys ph, const double* __restrict__ U, AdjBufs b) {
     constexpr int NE = DIM + 2;
     constexpr int NT = ViscTerms<DIM>::NT;
@@ -2741,9 +2750,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
         stress_heat_vjp<DIM>(ph.mu, ph.k, tqb, gAb);
         pin(gAb);
     }
-    // the slots' weights and limiter vectors stay in registers for four slots and are read again for each component
-    // for more (from the geometry tables' cache lines on hexes)
-    constexpr bool RELOAD = KM > 4;
+    constexpr bool RELOAD = !kAdjKeepVectors<KM, RECON, VISC, TAB>;
     double wl[KM][DIM];
     auto load_vectors = [&]() {
 #pragma unroll

@@ -36,6 +36,27 @@ def jittered(cells, periodic):
     return mesh
 
 
+def halved(cells, periodic, directions):
+    """A box whose faces across the given directions come as two halves side by side: cells of more faces."""
+    box = BoxMesh(cells, [0.0] * len(cells), [1.0] * len(cells), periodic)
+    a, dim = box.arrays, len(cells)
+    axis = np.argmax(np.abs(np.asarray(a.face_normal)), axis=1)
+    # (a boundary face stays whole: a ghost cell has one face)
+    two = np.isin(axis, directions) & (np.asarray(a.face_cells)[:, 1] < a.n_interior)
+    of = np.repeat(np.arange(a.n_faces), 1 + two)
+    half, second = two[of], np.r_[False, of[1:] == of[:-1]]
+    take = lambda x: None if x is None else np.array(x)[of]  # noqa: E731
+    normal, centroid = take(a.face_normal), take(a.face_centroid)
+    normal[half] *= 0.5
+    along = (axis[of] + 1) % dim
+    centroid[np.arange(len(of)), along] += np.where(half, np.where(second, 0.25, -0.25) / np.array(cells)[along], 0.0)
+    mesh = ArrayMesh(dataclasses.replace(a, n_faces=len(of), face_cells=take(a.face_cells), face_normal=normal,
+                                         face_centroid=centroid, face_shift=take(a.face_shift), face_bc=take(a.face_bc)),
+                     source=box.source_cells())
+    mesh.lower, mesh.upper, mesh.parent = box.lower, box.upper, box  # (box owns the arrays not replaced)
+    return mesh
+
+
 MESHES = {
     "hexes_periodic": lambda: jittered([12, 11, 10], [True] * 3),
     "hexes_open": lambda: jittered([13, 11, 9], [False, True, True]),
@@ -94,6 +115,13 @@ ADJOINT = {
     "quads_periodic": lambda: Case("g", MESHES["quads_periodic"](), **NS, limiter="barthjespersen", n_species=1, diff=0.1),
     "quads_open_species": lambda: Case("h", MESHES["quads_open"](), **NS, limiter="barthjespersen", n_species=2, diff=0.1,
                                        bcs=all_outflow(2)),
+    # cells of eight and six faces (never in tables)
+    "eight_faces": lambda: Case("i", halved([7, 6, 5], [True] * 3, [0]), **NS, limiter="barthjespersen"),
+    "eight_faces_open": lambda: Case("j", halved([7, 6, 5], [False, True, True], [0]), **NS, limiter="barthjespersen",
+                                     n_species=2, diff=0.1, bcs=ghost_and_at_face(2)),
+    "eight_sides": lambda: Case("k", halved([9, 8], [True, True], [0, 1]), **NS, limiter="barthjespersen", n_species=2,
+                                diff=0.1),
+    "six_sides_open": lambda: Case("l", halved([9, 8], [False, True], [1]), **NS, limiter="none", bcs=inflow_x()),
 }
 
 
