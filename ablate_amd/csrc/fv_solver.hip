@@ -5406,6 +5406,9 @@ int ts_euler_device(abl_fv_handle h, double* U, double* R, double t0, double max
             const double left = std::ceil((max_time - k.t) / k.dt) + 1.0;
             int64_t batch = std::min(max_steps - k.steps, kMaxBatch);
             if (left < (double)batch) batch = std::max<int64_t>(1, (int64_t)left);
+            // a first step held down by dt0 says nothing about the following ones' size (256 steps enqueued for the twelve that
+            // followed on 64 x 64 quads: 3.0 ms instead of 0.2 ms)
+            if (k.steps == 0 && k.dt >= dt0) batch = 1;
             size_t events[kMaxBatch];  // pending events before each step
             const int64_t before = k.steps;
             for (int64_t i = 0; i < batch; i++) {

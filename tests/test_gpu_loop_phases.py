@@ -1,5 +1,5 @@
-"""Phase counts of abl_fv_ts_euler: one launch per phase and step taken, none for the steps that its device loop enqueues
-past the end of the run, which the step sizes decide."""
+"""The batches of abl_fv_ts_euler's device loop: phase counts (one launch per phase and step taken, none for the steps that
+are enqueued past the end of the run, which the step sizes decide) and runs whose first step is smaller than the others."""
 import pytest
 import torch
 
@@ -13,6 +13,34 @@ CASES = {
     "open_2d": lambda: Case("a", BoxMesh([19, 8], [0, 0], [1, 1], [False, True]), state="random2d", bcs=inflow_x()),
     "periodic_ns": lambda: Case("b", BoxMesh([7, 6, 5], [0, 0, 0], [1, 1, 1], [True] * 3), **NS),
 }
+
+
+@pytest.mark.parametrize("first", [1e-4, 0.7])
+@pytest.mark.parametrize("name", CASES)
+def test_first_step_below_the_physics_step(name, first, torch_cuda):
+    """A run whose dt0 is below the physics step against the same steps taken one by one."""
+    case = CASES[name]()
+    solver = case.solver()
+    U = torch.tensor(case.initial_state(), device="cuda")
+    V, W = U.clone(), U.clone()
+    dt = solver.ComputePhysicsTimeStep(W)
+    max_time, t, n, step = 6.3 * dt, 0.0, 0, min(first * dt, dt)
+    while t < max_time:
+        R = torch.zeros_like(V)
+        solver.compute_rhs(t, V, R)
+        new = solver.ComputePhysicsTimeStep(V)
+        solver.axpy(step, R, V)
+        t, left, n = t + step, max_time - (t + step), n + 1
+        if t < max_time and t + new > max_time:
+            new = left
+        if t < max_time and t + new < max_time and new * 2.0 > left:
+            new = left / 2.0
+        if t < max_time and t + new < max_time and new * 1.01 > left:
+            new = left
+        step = new
+    end, steps = solver.ts_euler(U, max_time, dt0=first * dt)
+    assert steps == n and end == pytest.approx(t, rel=1e-14)
+    assert torch.all((U - V).abs() <= 1e-13 * V.abs().amax(dim=1, keepdim=True))
 
 
 @pytest.mark.parametrize("steps", [3.4, 300.7])  # the last two steps halve what is left; more than one batch
