@@ -2265,10 +2265,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
     double QL = 0.0, QR = 0.0, QdL = 0.0, rhob = 0.0;
     if (ns) {
         const double2* __restrict__ gS2 = reinterpret_cast<const double2*>(gS);
-        double xR[DIM];  // a ghost's face value is its state
-#pragma unroll
-        for (int d = 0; d < DIM; d++) xR[d] = ghost || !recon ? 0.0 : x[1][d];
-        const double cdiff = sdiff && !ghost ? -ph.diff * 0.25 * area : 0.0;
+        const bool slope_r = recon && !ghost, diffuse = sdiff && !ghost;  // a ghost's face value is its state
+        const double cdiff = -ph.diff * 0.25 * area;
         struct Sp {
             double rl, rr, yl, yr;
             double2 a[DIM], c[DIM];  // gradient words in pairs: [0, DIM) limited densityYi, [DIM, 2 DIM) Yi gradient
@@ -2291,7 +2289,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
             const Sp v = nx;
             if (sp + 1 < ns) load(sp + 1);
             const double gsp = face_seed_of(v.rr, ivR, v.rl, ivL);
-            double wl[2 * DIM], wr[2 * DIM], yl = v.yl, yr = v.yr, dot = 0.0;
+            double wl[2 * DIM], wr[2 * DIM], yl = v.yl, yr = v.yr, dot = 0.0;  // (selected below: gradients may not be finite)
 #pragma unroll
             for (int q = 0; q < DIM; q++) {
                 wl[2 * q] = v.a[q].x;
@@ -2301,14 +2299,16 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
             }
 #pragma unroll
             for (int d = 0; d < DIM; d++) {
-                yl += wl[d] * (recon ? x[0][d] : 0.0);
-                yr += wr[d] * xR[d];
+                yl += wl[d] * x[0][d];
+                yr += wr[d] * x[1][d];
                 dot += nh[d] * (wl[DIM + d] + wr[DIM + d]);
             }
+            yl = recon ? yl : v.yl;
+            yr = slope_r ? yr : v.yr;
             QL += gsp * yl;
             QR += gsp * yr;
             QdL += gsp * (yr - yl);
-            rhob += gsp * cdiff * dot;  // rho_L and rho_R enter the face density alike
+            rhob += diffuse ? gsp * cdiff * dot : 0.0;  // rho_L and rho_R enter the face density alike
             if (sp & 1)
                 W[64 * (NFIX + (sp >> 1))] = make_double2(first, gsp);
             else if (sp + 1 == ns)
