@@ -3038,20 +3038,19 @@ __global__ __launch_bounds__(kBlock) void k_adj_gather(MeshView<double> m, Phys 
     const int64_t N = m.N, NI = m.NI, NG = N - NI;
     const int nc = NE + ph.ns;
     // the contribution its neighbour across slot k wrote for the cell (its mirror slot); padding slots and ghosts read
-    // the cell's own slot 0 and count it zero times, so that the slots' loads are in flight together, and with the next
+    // the cell's own slot 0 and leave it out, so that the slots' loads are in flight together, and with the next
     // component's
     const double* __restrict__ from[KM];
-    double count[KM];
     int32_t nb[KM];
+    bool inner[KM];
     bool any_bnd = false;
 #pragma unroll
     for (int k = 0; k < KM; k++) {
         nb[k] = m.snbr[k * NI + c];
         const int mk = b.mirror[k * NI + c];
-        const bool inner = nb[k] >= 0 && nb[k] < NI;
+        inner[k] = nb[k] >= 0 && nb[k] < NI;
         any_bnd |= nb[k] >= NI;
-        from[k] = b.contrib + (inner ? (int64_t)mk * nc * NI + nb[k] : c);
-        count[k] = inner ? 1.0 : 0.0;
+        from[k] = b.contrib + (inner[k] ? (int64_t)mk * nc * NI + nb[k] : c);
     }
     double own, in[KM];
     auto load = [&](int p) {
@@ -3066,7 +3065,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_gather(MeshView<double> m, Phys 
         for (int k = 0; k < KM; k++) v[k] = in[k];
         if (p + 1 < nc) load(p + 1);
 #pragma unroll
-        for (int k = 0; k < KM; k++) acc += count[k] * v[k];
+        for (int k = 0; k < KM; k++) acc += inner[k] ? v[k] : 0.0;
         if (any_bnd)
 #pragma unroll
             for (int k = 0; k < KM; k++) {
